@@ -7,17 +7,21 @@
 // grid.  Only the non-zero input half of each axis is read and only the
 // needed output half is written:
 //
-//   pass 1  x-FFT (+i)   x[3][NAT] or compact x      -> a1[3][NZ][NY][2NX]
-//   pass 2  y-FFT (+i)   a1                            -> a2[3][NZ][2NY][2NX]
+//   pass 1  x-FFT (+i)   x[3][NAT] or compact x      -> a1[3][2NX][p1: NY][nzp]
+//   pass 2  y-FFT (+i)   a1                            -> a2[3][2NX][p2: 2NY][nzp]
 //   pass 3  z-FFT (+i), 3x3 Green multiply, z-FFT (-i), keep iz < NZ (in place in a2)
 //   pass 4  y-FFT (-i)   a2, keep iy < NY              -> a1
 //   pass 5  x-FFT (-i), keep ix < NX, finish with x, adia, aoff -> y
 //
-// The x axis stays contiguous in every buffer, so passes 2-4 load tiles of
-// consecutive kx columns (coalesced rows) and transform along the strided
-// axis inside LDS.
+// The work arrays keep z contiguous (pitch nzp), so that the heaviest pass,
+// the z transforms around the Green multiply, streams whole columns; passes 1
+// and 5 transpose between x rows and z runs on the way through LDS.  This
+// file holds the LDS-staged kernels for every axis length; lengths with a
+// register shape use the kernels of rows.hpp, matvec_reg.hip and
+// pass3_wave.hpp, which read and write the same arrays.
 #include "state.hpp"
 #include "fft_device.hpp"
+#include "mv_device.hpp"
 #include <vector>
 #include <cmath>
 #include <algorithm>
@@ -36,61 +40,55 @@ static constexpr int PER_NARROW = 8;  // passes 3, 5 (three components in LDS)
 static constexpr int WIDE_THREADS = 1024;
 
 // ---------------------------------------------------------------- pass 1 --
+// rows q = iy NZ + iz, rx of them per workgroup, so that the transposed store
+// writes runs of consecutive z; rows sit in LDS at stride L + 1
 template <int PER>
 __global__ __launch_bounds__(MV_THREADS) void k_pass1_xfwd(
-    const float2* __restrict__ x, float2* __restrict__ a1, const int* __restrict__ rowptr,
-    const int* __restrict__ occ, const float2* __restrict__ twg, FftPlan p, int nx, int nrows,
-    int rx, int nat, int nat0, int compact, int conj_in, BatchArgs ba) {
+    const float2* __restrict__ x, float2* __restrict__ a1, SiteMap map, const float2* __restrict__ twg, FftPlan p,
+    int nx, int ny, int nz, int nzp, int ks, int rx, int nat, int nat0, int compact, int conj_in, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z;
   if (ba.active && !ba.active[rb]) return;
   x += rb * ba.xs;
   a1 += rb * ba.a1s;
-  const int L = p.L;
+  const int L = p.L, LP = rx > 1 ? L + 1 : L;
   float2* tw = sm;
   float2* buf = sm + L;
   const int c = blockIdx.y;
-  const int g0 = blockIdx.x * rx;
+  const int q0 = blockIdx.x * rx, nrows = ny * nz;
   const int T = blockDim.x;
-  const int nr = min(rx, nrows - g0);
+  const int nr = min(rx, nrows - q0);
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  if (!compact) {
-    const float2* xs = x + (size_t)c * nat + (size_t)g0 * nx;
-    for (int idx = threadIdx.x; idx < rx * L; idx += T) {
-      const int r = idx / L, e = idx - r * L;
-      float2 v = make_float2(0.f, 0.f);
-      if (r < nr && e < nx) {
-        v = xs[(size_t)r * nx + e];
-        if (conj_in) v.y = -v.y;
-      }
-      buf[idx] = v;
-    }
-  } else {
-    for (int idx = threadIdx.x; idx < rx * L; idx += T) buf[idx] = make_float2(0.f, 0.f);
-    __syncthreads();
-    const int q0 = rowptr[g0], q1 = rowptr[g0 + nr];
-    const float2* xs = x + (size_t)c * nat0;
-    for (int q = q0 + threadIdx.x; q < q1; q += T) {
-      const int j = occ[q];
-      const int g = j / nx;
-      const int e = j - g * nx;
-      float2 v = xs[q];
+  const float2* xs = x + (size_t)c * (compact ? nat0 : nat);
+  for (int idx = threadIdx.x; idx < rx * L; idx += T) {
+    const int r = idx / L, e = idx - r * L;
+    float2 v = make_float2(0.f, 0.f);
+    if (r < nr && e < nx) {
+      const int q = q0 + r, iy = q / nz, g = iy + ny * (q - iy * nz);
+      const int o = compact ? compact_index(map, g, e, nx) : g * nx + e;
+      if (o >= 0) v = xs[o];
       if (conj_in) v.y = -v.y;
-      buf[(g - g0) * L + e] = v;
     }
+    buf[r * LP + e] = v;
   }
   __syncthreads();
-  fft_run<+1, false, PER>(buf, tw, p, rx, 1, L);
-  float2* out = a1 + ((size_t)c * nrows + g0) * L;
-  for (int idx = threadIdx.x; idx < nr * L; idx += T) out[idx] = buf[idx];
+  fft_run<+1, false, PER>(buf, tw, p, rx, 1, LP);
+  float2* out = a1 + (size_t)c * L * ks;
+  for (int idx = threadIdx.x; idx < nr * L; idx += T) {
+    const int k = idx / nr, r = idx - k * nr;
+    const int q = q0 + r, iy = q / nz, iz = q - iy * nz;
+    out[(size_t)k * ks + (size_t)iy * nzp + iz] = buf[r * LP + k];
+  }
 }
 
 // ------------------------------------------------------------- pass 2, 4 --
-// in [3][nz][nin][gx] -> out [3][nz][nout][gx], FFT along the middle axis.
+// in [3][gx][ins: nin][nzp] -> out [3][gx][outs: nout][nzp], FFT along the middle axis of
+// plane kx, tiles of cy consecutive z.
 template <int DIR, int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass_y(
     const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ twg,
-    FftPlan p, int gx, int nin, int nout, int nz, int cy_log2, size_t ins, size_t outs, BatchArgs ba) {
+    FftPlan p, int gx, int nin, int nout, int nz, int nzp, int ins,
+    int outs, int cy_log2, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z / 3;
   if (ba.active && !ba.active[rb]) return;
@@ -100,99 +98,95 @@ __global__ __launch_bounds__(NT) void k_pass_y(
   const int cy = 1 << cy_log2;
   float2* tw = sm;
   float2* buf = sm + L;
-  const int c = blockIdx.z % 3, iz = blockIdx.y, kx0 = blockIdx.x * cy;
+  const int c = blockIdx.z % 3, kx = blockIdx.y, z0 = blockIdx.x * cy;
   const int T = blockDim.x;
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  const float2* src = in + ((size_t)c * nz + iz) * ins;
+  const float2* src = in + ((size_t)c * gx + kx) * ins;
   for (int idx = threadIdx.x; idx < L * cy; idx += T) {
     const int e = idx >> cy_log2, col = idx & (cy - 1);
-    const int kx = kx0 + col;
+    const int iz = z0 + col;
     float2 v = make_float2(0.f, 0.f);
-    if (e < nin && kx < gx) v = src[(size_t)e * gx + kx];
+    if (e < nin && iz < nz) v = src[(size_t)e * nzp + iz];
     buf[idx] = v;
   }
   __syncthreads();
   fft_run<DIR, true, PER>(buf, tw, p, cy, cy, 1);
-  float2* dst = out + ((size_t)c * nz + iz) * outs;
+  float2* dst = out + ((size_t)c * gx + kx) * outs;
   for (int idx = threadIdx.x; idx < nout * cy; idx += T) {
     const int e = idx >> cy_log2, col = idx & (cy - 1);
-    const int kx = kx0 + col;
-    if (kx < gx) dst[(size_t)e * gx + kx] = buf[idx];
+    const int iz = z0 + col;
+    if (iz < nz) dst[(size_t)e * nzp + iz] = buf[idx];
   }
 }
 
 // ---------------------------------------------------------------- pass 3 --
+// cz contiguous z columns (kx 2NY + ky) per workgroup, each at stride L + 1 in LDS
 template <int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass3_z_green(
     float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg,
-    FftPlan p, int nx, int ny, int nz, int gx, int gy, int cz_log2, size_t plane, BatchArgs ba, GreenGeo gg) {
+    FftPlan p, int nz, int nzp, int p2, int gx, int gy, int cz, BatchArgs ba, GreenGeo gg) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z;
   if (ba.active && !ba.active[rb]) return;
   a2 += rb * ba.a2s;
-  const int L = p.L;  // = 2 nz
-  const int cz = 1 << cz_log2;
+  const int L = p.L, LP = cz > 1 ? L + 1 : L;  // L = 2 nz
   float2* tw = sm;
   float2* b0 = sm + L;
-  float2* b1 = b0 + L * cz;
-  float2* b2 = b1 + L * cz;
-  const int ky = blockIdx.y, kx0 = blockIdx.x * cz;
+  float2* b1 = b0 + LP * cz;
+  float2* b2 = b1 + LP * cz;
+  const int ncol = gx * gy, q0 = blockIdx.x * cz, nc = min(cz, ncol - q0);
   const int T = blockDim.x;
-  const size_t cstride = (size_t)nz * plane;
+  const size_t cstride = (size_t)gx * p2;
+  const auto column = [&](int r) {
+    const int kx = (q0 + r) / gy;
+    return (size_t)kx * p2 + (size_t)(q0 + r - kx * gy) * nzp;
+  };
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
   for (int idx = threadIdx.x; idx < L * cz; idx += T) {
-    const int e = idx >> cz_log2, col = idx & (cz - 1);
-    const int kx = kx0 + col;
+    const int r = idx / L, e = idx - r * L;
     float2 v0 = make_float2(0.f, 0.f), v1 = v0, v2 = v0;
-    if (e < nz && kx < gx) {
-      const size_t o = (size_t)e * plane + (size_t)ky * gx + kx;
+    if (e < nz && r < nc) {
+      const size_t o = column(r) + e;
       v0 = a2[o];
       v1 = a2[o + cstride];
       v2 = a2[o + 2 * cstride];
     }
-    b0[idx] = v0; b1[idx] = v1; b2[idx] = v2;
+    const int li = r * LP + e;
+    b0[li] = v0; b1[li] = v1; b2[li] = v2;
   }
   __syncthreads();
-  fft_run<+1, true, PER>(b0, tw, p, cz, cz, 1);
-  fft_run<+1, true, PER>(b1, tw, p, cz, cz, 1);
-  fft_run<+1, true, PER>(b2, tw, p, cz, cz, 1);
+  fft_run<+1, false, PER>(b0, tw, p, cz, 1, LP);
+  fft_run<+1, false, PER>(b1, tw, p, cz, 1, LP);
+  fft_run<+1, false, PER>(b2, tw, p, cz, 1, LP);
   // symmetric 3x3 multiply; trimmed-octant reconstruction for IPBC=0
   // (cu:109-115), whole grid for IPBC=1
-  const int ox = gg.ox, oy = gg.oy;
-  const int jr = min(ky, gg.my - ky);
-  const float sy = ky <= gg.ty ? 1.f : -1.f;
-  for (int idx = threadIdx.x; idx < L * cz; idx += T) {
-    const int kz = idx >> cz_log2, col = idx & (cz - 1);
-    const int kx = kx0 + col;
-    if (kx >= gx) continue;
-    const int ir = min(kx, gg.mx - kx), kr = min(kz, gg.mz - kz);
-    const float sx = kx <= gg.tx ? 1.f : -1.f;
+  for (int idx = threadIdx.x; idx < L * nc; idx += T) {
+    const int r = idx / L, kz = idx - r * L;
+    const int kx = (q0 + r) / gy, ky = q0 + r - kx * gy;
+    const int ir = min(kx, gg.mx - kx), jr = min(ky, gg.my - ky), kr = min(kz, gg.mz - kz);
+    const float sx = kx <= gg.tx ? 1.f : -1.f, sy = ky <= gg.ty ? 1.f : -1.f;
     const float sz = kz <= gg.tz ? 1.f : -1.f;
-    const Green6 G = green_at(green, (size_t)ir + (size_t)ox * ((size_t)jr + (size_t)oy * kr));
-    const float2 g11 = G.xx;
+    const Green6 G = green_at(green, (size_t)kr + (size_t)gg.oz * ((size_t)jr + (size_t)gg.oy * ir));
     const float2 g12 = cscale(G.xy, sx * sy);
     const float2 g13 = cscale(G.xz, sx * sz);
-    const float2 g22 = G.yy;
     const float2 g23 = cscale(G.yz, sy * sz);
-    const float2 g33 = G.zz;
-    const float2 p0 = b0[idx], p1 = b1[idx], p2 = b2[idx];
-    b0[idx] = cadd(cadd(cmul(g11, p0), cmul(g12, p1)), cmul(g13, p2));
-    b1[idx] = cadd(cadd(cmul(g12, p0), cmul(g22, p1)), cmul(g23, p2));
-    b2[idx] = cadd(cadd(cmul(g13, p0), cmul(g23, p1)), cmul(g33, p2));
+    const int li = r * LP + kz;
+    const float2 p0 = b0[li], p1 = b1[li], p2 = b2[li];
+    b0[li] = cadd(cadd(cmul(G.xx, p0), cmul(g12, p1)), cmul(g13, p2));
+    b1[li] = cadd(cadd(cmul(g12, p0), cmul(G.yy, p1)), cmul(g23, p2));
+    b2[li] = cadd(cadd(cmul(g13, p0), cmul(g23, p1)), cmul(G.zz, p2));
   }
   __syncthreads();
-  fft_run<-1, true, PER>(b0, tw, p, cz, cz, 1);
-  fft_run<-1, true, PER>(b1, tw, p, cz, cz, 1);
-  fft_run<-1, true, PER>(b2, tw, p, cz, cz, 1);
-  for (int idx = threadIdx.x; idx < nz * cz; idx += T) {
-    const int e = idx >> cz_log2, col = idx & (cz - 1);
-    const int kx = kx0 + col;
-    if (kx < gx) {
-      const size_t o = (size_t)e * plane + (size_t)ky * gx + kx;
-      a2[o] = b0[idx];
-      a2[o + cstride] = b1[idx];
-      a2[o + 2 * cstride] = b2[idx];
-    }
+  fft_run<-1, false, PER>(b0, tw, p, cz, 1, LP);
+  fft_run<-1, false, PER>(b1, tw, p, cz, 1, LP);
+  fft_run<-1, false, PER>(b2, tw, p, cz, 1, LP);
+  for (int idx = threadIdx.x; idx < nz * nc; idx += T) {
+    const int r = idx / nz, e = idx - r * nz;
+    const size_t o = column(r) + e;
+    const int li = r * LP + e;
+    a2[o] = b0[li];
+    a2[o + cstride] = b1[li];
+    a2[o + 2 * cstride] = b2[li];
   }
 }
 
@@ -215,9 +209,8 @@ template <int PER>
 __global__ __launch_bounds__(MV_THREADS) void k_pass5_xinv_finish(
     const float2* __restrict__ a1, const float2* __restrict__ twg, FftPlan p,
     const float2* __restrict__ x, float2* __restrict__ y, const float2* __restrict__ adia,
-    const float2* __restrict__ aoff, const int16_t* __restrict__ iocc,
-    const int* __restrict__ rowptr, const int* __restrict__ occ, int nx, int nrows, int rx,
-    int nat, int nat0, int compact, int cj, float inv, BatchArgs ba) {
+    const float2* __restrict__ aoff, const int16_t* __restrict__ iocc, SiteMap map, int nx, int ny, int nz, int nzp,
+    int ks, int rx, int nat, int nat0, int compact, int cj, float inv, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.y;
   if (ba.active && !ba.active[rb]) return;
@@ -226,54 +219,47 @@ __global__ __launch_bounds__(MV_THREADS) void k_pass5_xinv_finish(
   y += rb * ba.xs;
   adia += rb * ba.os;
   aoff += rb * ba.os;
-  const int L = p.L;
+  const int L = p.L, LP = rx > 1 ? L + 1 : L;
   float2* tw = sm;
   float2* b0 = sm + L;
-  float2* b1 = b0 + rx * L;
-  float2* b2 = b1 + rx * L;
-  const int g0 = blockIdx.x * rx;
+  float2* b1 = b0 + rx * LP;
+  float2* b2 = b1 + rx * LP;
+  const int q0 = blockIdx.x * rx, nrows = ny * nz;
   const int T = blockDim.x;
-  const int nr = min(rx, nrows - g0);
+  const int nr = min(rx, nrows - q0);
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  const size_t cs = (size_t)nrows * L;
-  const float2* src = a1 + (size_t)g0 * L;
+  const size_t cs = (size_t)L * ks;
   for (int idx = threadIdx.x; idx < rx * L; idx += T) {
+    const int k = idx / rx, r = idx - k * rx;
     float2 v0 = make_float2(0.f, 0.f), v1 = v0, v2 = v0;
-    if (idx < nr * L) { v0 = src[idx]; v1 = src[idx + cs]; v2 = src[idx + 2 * cs]; }
-    b0[idx] = v0; b1[idx] = v1; b2[idx] = v2;
+    if (r < nr) {
+      const int q = q0 + r, iy = q / nz, iz = q - iy * nz;
+      const float2* src = a1 + (size_t)k * ks + (size_t)iy * nzp + iz;
+      v0 = src[0]; v1 = src[cs]; v2 = src[2 * cs];
+    }
+    const int li = r * LP + k;
+    b0[li] = v0; b1[li] = v1; b2[li] = v2;
   }
   __syncthreads();
-  fft_run<-1, false, PER>(b0, tw, p, rx, 1, L);
-  fft_run<-1, false, PER>(b1, tw, p, rx, 1, L);
-  fft_run<-1, false, PER>(b2, tw, p, rx, 1, L);
-  if (!compact) {
-    for (int idx = threadIdx.x; idx < nr * nx; idx += T) {
-      const int r = idx / nx, ix = idx - r * nx;
-      const size_t j = (size_t)(g0 + r) * nx + ix;
-      float2 r1, r2, r3;
-      if (iocc && iocc[j] == 0) {
-        r1 = r2 = r3 = make_float2(0.f, 0.f);
-      } else {
-        const int li = r * L + ix;
-        finish_site(x[j], x[j + nat], x[j + 2 * (size_t)nat], adia[j], adia[j + nat],
-                    adia[j + 2 * (size_t)nat], aoff[j], aoff[j + nat], aoff[j + 2 * (size_t)nat],
-                    b0[li], b1[li], b2[li], inv, cj != 0, r1, r2, r3);
-      }
-      y[j] = r1; y[j + nat] = r2; y[j + 2 * (size_t)nat] = r3;
+  fft_run<-1, false, PER>(b0, tw, p, rx, 1, LP);
+  fft_run<-1, false, PER>(b1, tw, p, rx, 1, LP);
+  fft_run<-1, false, PER>(b2, tw, p, rx, 1, LP);
+  const size_t sd = compact ? (size_t)nat0 : (size_t)nat;
+  for (int idx = threadIdx.x; idx < nr * nx; idx += T) {
+    const int r = idx / nx, ix = idx - r * nx;
+    const int q = q0 + r, iy = q / nz, g = iy + ny * (q - iy * nz);
+    const int o = compact ? compact_index(map, g, ix, nx) : g * nx + ix;
+    if (o < 0) continue;
+    float2 r1, r2, r3;
+    if (iocc && iocc[o] == 0) {
+      r1 = r2 = r3 = make_float2(0.f, 0.f);
+    } else {
+      const int li = r * LP + ix;
+      const size_t j = (size_t)o;
+      finish_site(x[j], x[j + sd], x[j + 2 * sd], adia[j], adia[j + sd], adia[j + 2 * sd], aoff[j], aoff[j + sd],
+                  aoff[j + 2 * sd], b0[li], b1[li], b2[li], inv, cj != 0, r1, r2, r3);
     }
-  } else {
-    const int q0 = rowptr[g0], q1 = rowptr[g0 + nr];
-    for (int q = q0 + threadIdx.x; q < q1; q += T) {
-      const int j = occ[q];
-      const int g = j / nx;
-      const int ix = j - g * nx;
-      const int li = (g - g0) * L + ix;
-      float2 r1, r2, r3;
-      finish_site(x[q], x[q + nat0], x[q + 2 * (size_t)nat0], adia[q], adia[q + nat0],
-                  adia[q + 2 * (size_t)nat0], aoff[q], aoff[q + nat0], aoff[q + 2 * (size_t)nat0],
-                  b0[li], b1[li], b2[li], inv, cj != 0, r1, r2, r3);
-      y[q] = r1; y[q + nat0] = r2; y[q + 2 * (size_t)nat0] = r3;
-    }
+    y[o] = r1; y[o + sd] = r2; y[o + 2 * sd] = r3;
   }
 }
 
@@ -381,21 +367,25 @@ int matvec_setup(Context& c) {
   }
   if (m.cz < 8) {
     int cw = std::min(16, pow2floor(std::max(1, PER_NARROW * WIDE_THREADS / m.gz)));
-    while (cw > 1 && (size_t)(m.gz + 3 * cw * m.gz) * sizeof(float2) > lds_max) cw /= 2;
+    while (cw > 1 && (size_t)(m.gz + 3 * cw * (m.gz + 1)) * sizeof(float2) > lds_max) cw /= 2;
     if (cw > m.cz) { m.cz = cw; m.tz = WIDE_THREADS; }
   }
   if ((m.ty == WIDE_THREADS || m.tz == WIDE_THREADS) && allow_big_lds(lds_max)) return 206;
   if (upload_twiddles(m.gx, &m.twx) || upload_twiddles(m.gy, &m.twy) || upload_twiddles(m.gz, &m.twz)) return 206;
-  m.p1 = (size_t)c.ny * m.gx;
-  m.p2 = (size_t)m.gy * m.gx;
-  const size_t n1 = (size_t)3 * c.nz * m.p1, n2 = (size_t)3 * c.nz * m.p2;
-  DDH_TRY(hipMalloc((void**)&c.a1, n1 * sizeof(float2)), "malloc FFT work a1", 204);
-  DDH_TRY(hipMalloc((void**)&c.a2, n2 * sizeof(float2)), "malloc FFT work a2", 204);
+  // z runs start on 128-byte lines; targets of a few planes keep a small pitch
+  m.nzp = c.nz > 32 ? (c.nz + 15) & ~15 : (c.nz + 3) & ~3;
+  // an odd number of 256-byte blocks per kx plane: passes 1 and 5 step through
+  // the planes, and a power-of-two step would hit few memory channels
+  const auto odd_blocks = [](int n) { return ((n + 31) / 32 | 1) * 32; };
+  m.p1 = odd_blocks(c.ny * m.nzp);
+  m.p2 = odd_blocks(m.gy * m.nzp);
+  DDH_TRY(hipMalloc((void**)&c.a1, matvec_a1_count(c) * sizeof(float2)), "malloc FFT work a1", 204);
+  DDH_TRY(hipMalloc((void**)&c.a2, matvec_a2_count(c) * sizeof(float2)), "malloc FFT work a2", 204);
   return 0;
 }
 
-size_t matvec_a1_count(const Context& c) { return (size_t)3 * c.nz * c.ny * c.mv.gx; }
-size_t matvec_a2_count(const Context& c) { return (size_t)3 * c.nz * c.mv.p2; }
+size_t matvec_a1_count(const Context& c) { return (size_t)3 * c.mv.gx * c.mv.p1; }
+size_t matvec_a2_count(const Context& c) { return (size_t)3 * c.mv.gx * c.mv.p2; }
 
 void matvec_release(Context& c) {
   for (float2** p : {&c.mv.twx, &c.mv.twy, &c.mv.twz, &c.a1, &c.a2}) {
@@ -411,59 +401,57 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
   const int nrows = c.ny * c.nz;
   const unsigned nb = (unsigned)bt.nrhs;
   float2 *a1 = bt.a1, *a2 = bt.a2;
+  const SiteMap sm{c.rowptr, c.rowlo, c.qmap, c.rows_contiguous};
   if (!c.fft_generic && kind >= 0 && reg_pass(c, which, kind, cj, compact, x, y, adia, aoff, st, bt)) return 0;
   switch (which) {
     case 1: {
       dim3 grid((nrows + m.rx_fwd - 1) / m.rx_fwd, 3, nb);
-      size_t lds = (size_t)(m.gx + m.rx_fwd * m.gx) * sizeof(float2);
-      hipLaunchKernelGGL(k_pass1_xfwd<PER_WIDE>, grid, dim3(MV_THREADS), lds, st, x, a1, c.rowptr, c.occ, m.twx,
-                         m.px, c.nx, nrows, m.rx_fwd, c.nat, c.nat0, compact, cj, bt.k);
+      size_t lds = (size_t)(m.gx + m.rx_fwd * (m.gx + (m.rx_fwd > 1))) * sizeof(float2);
+      hipLaunchKernelGGL(k_pass1_xfwd<PER_WIDE>, grid, dim3(MV_THREADS), lds, st, x, a1, sm, m.twx, m.px, c.nx, c.ny,
+                         c.nz, m.nzp, m.p1, m.rx_fwd, c.nat, c.nat0, compact, cj, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 1 (x FFT)", 21);
       break;
     }
-    case 2: {
-      dim3 grid((m.gx + m.cy - 1) / m.cy, c.nz, 3 * nb);
-      size_t lds = (size_t)(m.gy + m.cy * m.gy) * sizeof(float2);
-      if (m.ty == WIDE_THREADS)
+    case 2:
+    case 4: {
+      const bool fwd = which == 2;
+      dim3 grid((c.nz + m.cy - 1) / m.cy, m.gx, 3 * nb);
+      const size_t lds = (size_t)(m.gy + m.cy * m.gy) * sizeof(float2);
+      const int lg = ilog2(m.cy), ins = fwd ? m.p1 : m.p2, outs = fwd ? m.p2 : m.p1;
+      if (fwd && m.ty == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a1, a2, m.twy,
-                           m.py, m.gx, c.ny, m.gy, c.nz, ilog2(m.cy), m.p1, m.p2, bt.k);
+                           m.py, m.gx, c.ny, m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
+      else if (fwd)
+        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a1, a2, m.twy, m.py, m.gx, c.ny,
+                           m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
+      else if (m.ty == WIDE_THREADS)
+        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2, a1, m.twy,
+                           m.py, m.gx, m.gy, c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
       else
-        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a1, a2, m.twy, m.py, m.gx,
-                           c.ny, m.gy, c.nz, ilog2(m.cy), m.p1, m.p2, bt.k);
-      DDH_LAUNCH_OK("MATVEC pass 2 (y FFT)", 22);
+        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a2, a1, m.twy, m.py, m.gx, m.gy,
+                           c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
+      DDH_LAUNCH_OK("MATVEC y FFT", fwd ? 22 : 24);
       break;
     }
     case 3: {
-      dim3 grid((m.gx + m.cz - 1) / m.cz, m.gy, nb);
-      size_t lds = (size_t)(m.gz + 3 * m.cz * m.gz) * sizeof(float2);
+      dim3 grid((m.gx * m.gy + m.cz - 1) / m.cz, 1, nb);
+      const size_t lds = (size_t)(m.gz + 3 * m.cz * (m.gz + (m.cz > 1))) * sizeof(float2);
       if (m.tz == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass3_z_green<PER_NARROW, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2,
-                           c.green, m.twz, m.pz, c.nx, c.ny, c.nz, m.gx, m.gy, ilog2(m.cz), m.p2, bt.k, green_geo(c));
+                           c.green, m.twz, m.pz, c.nz, m.nzp, m.p2, m.gx, m.gy, m.cz, bt.k, green_geo(c));
       else
         hipLaunchKernelGGL(k_pass3_z_green<PER_NARROW>, grid, dim3(MV_THREADS), lds, st, a2, c.green, m.twz, m.pz,
-                           c.nx, c.ny, c.nz, m.gx, m.gy, ilog2(m.cz), m.p2, bt.k, green_geo(c));
+                           c.nz, m.nzp, m.p2, m.gx, m.gy, m.cz, bt.k, green_geo(c));
       DDH_LAUNCH_OK("MATVEC pass 3 (z FFT + Green)", 23);
-      break;
-    }
-    case 4: {
-      dim3 grid((m.gx + m.cy - 1) / m.cy, c.nz, 3 * nb);
-      size_t lds = (size_t)(m.gy + m.cy * m.gy) * sizeof(float2);
-      if (m.ty == WIDE_THREADS)
-        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2, a1, m.twy,
-                           m.py, m.gx, m.gy, c.ny, c.nz, ilog2(m.cy), m.p2, m.p1, bt.k);
-      else
-        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a2, a1, m.twy, m.py, m.gx,
-                           m.gy, c.ny, c.nz, ilog2(m.cy), m.p2, m.p1, bt.k);
-      DDH_LAUNCH_OK("MATVEC pass 4 (y inverse FFT)", 24);
       break;
     }
     default: {
       dim3 grid((nrows + m.rx_inv - 1) / m.rx_inv, nb);
-      size_t lds = (size_t)(m.gx + 3 * m.rx_inv * m.gx) * sizeof(float2);
+      size_t lds = (size_t)(m.gx + 3 * m.rx_inv * (m.gx + (m.rx_inv > 1))) * sizeof(float2);
       const float inv = 1.f / (float)m.ngrid;
       hipLaunchKernelGGL(k_pass5_xinv_finish<PER_NARROW>, grid, dim3(MV_THREADS), lds, st, a1, m.twx, m.px, x, y,
-                         adia, aoff, compact ? nullptr : c.iocc, c.rowptr, c.occ, c.nx, nrows, m.rx_inv, c.nat,
-                         c.nat0, compact, cj, inv, bt.k);
+                         adia, aoff, compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz, m.nzp, m.p1, m.rx_inv, c.nat, c.nat0,
+                         compact, cj, inv, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 5 (x inverse FFT + finish)", 25);
       break;
     }
@@ -488,11 +476,12 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   return 0;
 }
 
-// Autotuner: for each pass, every register shape of its axis length and the
-// LDS-staged kernel run a few times on the prepared grid (compact vectors,
-// stream events); the fastest is kept in c.mv.kind.  Choices are cached per
-// grid for the life of the process, so re-preparing the same grid (for
-// instance every target orientation of a DDSCAT run) does not re-time.
+// Autotuner: a pass whose axis length has several register shapes runs each a
+// few times on the prepared grid (compact vectors, stream events); the fastest
+// is kept in c.mv.kind.  A pass with one shape takes it, a pass without one the
+// LDS-staged kernel (slower wherever there is a shape).  Choices are cached per
+// grid for the life of the process, so re-preparing the same grid (for instance
+// every target orientation of a DDSCAT run) does not re-time.
 namespace {
 struct TuneKey {
   int nx, ny, nz, ipbc;  // IPBC=1 reads the whole-grid Green in pass 3, not the octant
@@ -533,10 +522,10 @@ int matvec_autotune(Context& c) {
   int rc = 0;
   for (int p = 1; p <= 5 && !rc; ++p) {
     const int ncand = reg_candidates(lens[p], p);
-    if (ncand == 0) continue;
+    if (ncand < 2) continue;
     float best = 1e30f;
     int best_kind = m.kind[p];
-    for (int k = -1; k < ncand && !rc; ++k) {
+    for (int k = 0; k < ncand && !rc; ++k) {
       for (int w = 0; w < 2 && !rc; ++w) rc = launch_pass(c, p, k, 0, 1, c.sx, c.sy, c.adia_c, c.aoff_c, st, bt);
       hipEventRecord(e0, st);
       for (int r = 0; r < 5 && !rc; ++r) rc = launch_pass(c, p, k, 0, 1, c.sx, c.sy, c.adia_c, c.aoff_c, st, bt);

@@ -20,7 +20,9 @@ struct MatvecPlan {
   // tile parameters
   int rx_fwd = 1, rx_inv = 1, cy = 1, cz = 1;
   int ty = 256, tz = 256;  // workgroup size of the LDS-staged y passes and z pass
-  size_t p1 = 0, p2 = 0;  // plane strides (elements) of a1 [3][nz][ny][gx] and a2 [3][nz][plane p2]
+  // z pitch and kx plane strides (elements) of the FFT3D work arrays
+  // a1 [3][gx][p1: ny][nzp] and a2 [3][gx][p2: gy][nzp]
+  int nzp = 0, p1 = 0, p2 = 0;
   // FFT kernel per pass 1..5: index into the register shapes of that pass's
   // axis length, or -1 for the LDS-staged kernel (chosen by the autotuner)
   int kind[6] = {-1, -1, -1, -1, -1, -1};
@@ -69,10 +71,11 @@ struct Context {
   MatvecPlan mv;
   hipStream_t stream = nullptr;
   // Spectral Green tensor, point-interleaved complex64: the trimmed octant
-  // [nz+1][ny+1][nx+1][6] for IPBC=0, the whole grid [2nz][2ny][2nx][6] for IPBC=1
+  // of (nx+1)(ny+1)(nz+1) points for IPBC=0, the whole grid of 2nx 2ny 2nz for IPBC=1
   float2* green = nullptr;
   size_t green_count = 0;
-  // FFT3D work: a1 [3][nz][ny][gx], a2 [3][nz][gy][gx]
+  int green_zfast = 0;  // resident point order: 1 z fastest (FFT3D), 0 x fastest (SLICES)
+  // FFT3D work: a1 [3][gx][p1: ny][nzp], a2 [3][gx][p2: gy][nzp]
   float2 *a1 = nullptr, *a2 = nullptr;
   // occupancy
   int16_t* iocc = nullptr;     // [nat]
@@ -140,7 +143,7 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
                   const MvBatch* bt = nullptr);
 int matvec_setup(Context& c);
 void matvec_release(Context& c);
-// FFT work elements per RHS: a1 [3][nz][ny][gx], a2 [3][nz][gy][gx]
+// FFT work elements per RHS: a1 [3][gx][p1: ny][nzp], a2 [3][gx][p2: gy][nzp]
 size_t matvec_a1_count(const Context& c);
 size_t matvec_a2_count(const Context& c);
 // register-FFT shapes available for pass `which` (1..5) on a padded axis length (0: none)
@@ -183,8 +186,10 @@ double green_pbc_work(const Context& c, const GreenBuild& b);
 
 // The resident spectral Green tensor c.green is stored point-interleaved:
 // the six components (xx, xy, xz, yy, yz, zz) of octant point
-// p = ir + (NX+1)(jr + (NY+1) kr) sit at green[6p .. 6p+5], so a MATVEC reads
-// them as three 16-byte loads from one 48-byte run.  The reference layout
+// (ir, jr, kr) sit at green[6p .. 6p+5], so a MATVEC reads them as three
+// 16-byte loads from one 48-byte run.  The axis that the backend's Green pass
+// transforms along a wave's lanes runs fastest: p = kr + (NZ+1)(jr + (NY+1) ir)
+// for FFT3D, p = ir + (NX+1)(jr + (NY+1) kr) for SLICES.  The reference layout
 // ([6][NZ+1][NY+1][NX+1], CXZC) is converted at the ABI edges.
 struct Green6 {
   float2 xx, xy, xz, yy, yz, zz;
@@ -200,26 +205,27 @@ __device__ __forceinline__ Green6 green_at(const float2* __restrict__ g, size_t 
 // (cu:109-115): index min(k, 2N - k) per axis, the off-diagonal components
 // flip sign with the mirrored axes' parities.  IPBC=1 stores the whole grid.
 // Both use the same instructions:
-//   r = min(k, m - k),  sign = (k <= t) ? +1 : -1,  point = rx + ox (ry + oy rz)
-// octant: m = 2N, t = N, ox = NX+1, oy = NY+1; full grid: m = t = 2^30
-// (no mirror, all signs +1), ox = 2NX, oy = 2NY.
+//   r = min(k, m - k),  sign = (k <= t) ? +1 : -1,
+//   point = rz + oz (ry + oy rx) for FFT3D, rx + ox (ry + oy rz) for SLICES
+// octant: m = 2N, t = N, o = N+1; full grid: m = t = 2^30 (no mirror, all
+// signs +1), o = 2N.
 struct GreenGeo {
-  int ox, oy;
+  int ox, oy, oz;
   int mx, my, mz;
   int tx, ty, tz;
 };
 inline GreenGeo green_geo(const Context& c) {
   constexpr int NOMIRROR = 1 << 30;
-  if (c.ipbc) return GreenGeo{2 * c.nx, 2 * c.ny, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR};
-  return GreenGeo{c.nx + 1, c.ny + 1, 2 * c.nx, 2 * c.ny, 2 * c.nz, c.nx, c.ny, c.nz};
+  if (c.ipbc) return GreenGeo{2 * c.nx, 2 * c.ny, 2 * c.nz, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR, NOMIRROR};
+  return GreenGeo{c.nx + 1, c.ny + 1, c.nz + 1, 2 * c.nx, 2 * c.ny, 2 * c.nz, c.nx, c.ny, c.nz};
 }
 // number of spectral Green points stored: octant or whole padded grid
 inline size_t green_points(int nx, int ny, int nz, int ipbc) {
   return ipbc ? (size_t)(2 * nx) * (2 * ny) * (2 * nz) : (size_t)(nx + 1) * (ny + 1) * (nz + 1);
 }
 
-// component-major [6][npts] <-> point-interleaved [npts][6], device to device
-int green_interleave(Context& c, const float2* comp_major, float2* interleaved, hipStream_t st);
-int green_deinterleave(Context& c, const float2* interleaved, float2* comp_major, hipStream_t st);
+// component-major [6][rz][ry][rx] (x fastest) <-> the backend's resident layout, device to device
+int green_interleave(Context& c, const float2* comp_major, float2* resident, hipStream_t st);
+int green_deinterleave(Context& c, const float2* resident, float2* comp_major, hipStream_t st);
 
 }  // namespace ddhip
