@@ -21,6 +21,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstdio>
+#include <initializer_list>
 #include <vector>
 #include <thread>
 
@@ -45,31 +46,36 @@ struct BatchState {
   int* sel = nullptr;       // [B]
   int* m1 = nullptr;        // [B] device-computed masks (PBCGS2 reliable update)
   int* m2 = nullptr;
-  double* packed = nullptr; // [B][3] status, resid, flags
-  double* hpacked = nullptr;
-  int* hflags = nullptr;    // pinned [B]
+  double* fac = nullptr;    // [3 B] per-RHS factors of the adjoint and EVALQ kernels
   // iteration bookkeeping on the device (kb_step_end): [4][B] ints =
   // iterations, check request, active flags saved at a pause, reliable-update
-  // MATVECs; then the pause flag.  hist: recursive residual of iteration i
-  // at row (i - 1) mod HIST_ROWS.  hctl / hhist: pinned copies.
+  // MATVECs; then the pause flag
   int* ctl = nullptr;
-  double* hist = nullptr;
-  int* hctl = nullptr;
-  double* hhist = nullptr;
+  // Pinned host memory that kernels write (results) and read (flags)
+  // themselves: a status read-back costs one synchronisation and no copy.
+  //   packed [B][3]  status, relative residual, flags of the last iteration
+  //   ictl   [3][B]  iterations, check request, reliable-update MATVECs
+  //   hist   [HIST_ROWS][B]  recursive residual of iteration i at row (i - 1) mod HIST_ROWS
+  //   slots  [B][SLOTS_MAX]  scalars fetched by fetch_slots
+  //   flags  [FLAG_RING][B]  uploads in flight
+  double *hpacked = nullptr, *hhist = nullptr, *hslots = nullptr;
+  int *hictl = nullptr, *hflags = nullptr;
   int capB = 0;
 };
 constexpr int HIST_ROWS = 32;  // > RELIABLE_PERIOD: a chunk never wraps
+constexpr int SLOTS_MAX = 4;   // scalars per RHS in one fetch
+constexpr int FLAG_RING = 8;   // flag uploads between two synchronisations
 BatchState g_bs[MAX_TARGETS + 1];  // one per target slot
 BatchState& bstate(const Context& c) { return g_bs[c.slot]; }
 
 void bs_free(BatchState& S) {
   for (void** p : {(void**)&S.W, (void**)&S.a1, (void**)&S.a2, (void**)&S.scal, (void**)&S.part,
-                   (void**)&S.active, (void**)&S.sel, (void**)&S.m1, (void**)&S.m2, (void**)&S.packed,
-                   (void**)&S.ctl, (void**)&S.hist}) {
+                   (void**)&S.active, (void**)&S.sel, (void**)&S.m1, (void**)&S.m2, (void**)&S.fac,
+                   (void**)&S.ctl}) {
     if (*p) hipFree(*p);
     *p = nullptr;
   }
-  for (void** p : {(void**)&S.hpacked, (void**)&S.hflags, (void**)&S.hctl, (void**)&S.hhist}) {
+  for (void** p : {(void**)&S.hpacked, (void**)&S.hhist, (void**)&S.hslots, (void**)&S.hictl, (void**)&S.hflags}) {
     if (*p) hipHostFree(*p);
     *p = nullptr;
   }
@@ -107,11 +113,11 @@ int bs_ensure(Context& c, BatchState& S, int B, int nvec) {
   }
   if (B > S.capB) {
     for (void** p : {(void**)&S.scal, (void**)&S.part, (void**)&S.active, (void**)&S.sel, (void**)&S.m1,
-                     (void**)&S.m2, (void**)&S.packed, (void**)&S.ctl, (void**)&S.hist}) {
+                     (void**)&S.m2, (void**)&S.fac, (void**)&S.ctl}) {
       if (*p) hipFree(*p);
       *p = nullptr;
     }
-    for (void** p : {(void**)&S.hpacked, (void**)&S.hflags, (void**)&S.hctl, (void**)&S.hhist}) {
+    for (void** p : {(void**)&S.hpacked, (void**)&S.hhist, (void**)&S.hslots, (void**)&S.hictl, (void**)&S.hflags}) {
       if (*p) hipHostFree(*p);
       *p = nullptr;
     }
@@ -123,13 +129,13 @@ int bs_ensure(Context& c, BatchState& S, int B, int nvec) {
     DDH_TRY(hipMalloc((void**)&S.sel, (size_t)B * sizeof(int)), "batched flags", 29);
     DDH_TRY(hipMalloc((void**)&S.m1, (size_t)B * sizeof(int)), "batched flags", 29);
     DDH_TRY(hipMalloc((void**)&S.m2, (size_t)B * sizeof(int)), "batched flags", 29);
-    DDH_TRY(hipMalloc((void**)&S.packed, (size_t)B * 3 * sizeof(double)), "batched status", 29);
-    DDH_TRY(hipHostMalloc((void**)&S.hpacked, (size_t)B * 3 * sizeof(double)), "pinned status", 29);
-    DDH_TRY(hipHostMalloc((void**)&S.hflags, (size_t)B * sizeof(int)), "pinned flags", 29);
+    DDH_TRY(hipMalloc((void**)&S.fac, (size_t)B * 3 * sizeof(double)), "batched factors", 29);
     DDH_TRY(hipMalloc((void**)&S.ctl, ((size_t)4 * B + 1) * sizeof(int)), "batched iteration state", 29);
-    DDH_TRY(hipMalloc((void**)&S.hist, (size_t)HIST_ROWS * B * sizeof(double)), "batched residual history", 29);
-    DDH_TRY(hipHostMalloc((void**)&S.hctl, ((size_t)4 * B + 1) * sizeof(int)), "pinned iteration state", 29);
+    DDH_TRY(hipHostMalloc((void**)&S.hpacked, (size_t)B * 3 * sizeof(double)), "pinned status", 29);
     DDH_TRY(hipHostMalloc((void**)&S.hhist, (size_t)HIST_ROWS * B * sizeof(double)), "pinned residual history", 29);
+    DDH_TRY(hipHostMalloc((void**)&S.hslots, (size_t)B * SLOTS_MAX * sizeof(double)), "pinned scalars", 29);
+    DDH_TRY(hipHostMalloc((void**)&S.hictl, (size_t)3 * B * sizeof(int)), "pinned iteration state", 29);
+    DDH_TRY(hipHostMalloc((void**)&S.hflags, (size_t)FLAG_RING * B * sizeof(int)), "pinned flags", 29);
     S.capB = B;
   }
   S.B = B;
@@ -191,7 +197,7 @@ enum FinOp {
   FIN_P2_BETA1,     // p2::outer, then p2::beta(has_norm = 0) (first half-step)
   FIN_P2_BETA2,     // p2::beta(has_norm = 1)
   FIN_P2_ALPHA,     // p2::alpha
-  FIN_P2_CONVEX,    // p2::convex
+  FIN_P2_CONVEX,    // p2::convex, then the reliable-update masks m1, m2
 };
 
 // One workgroup per RHS, one wave per sum: lane l loads partials l, l + 64,
@@ -200,9 +206,12 @@ enum FinOp {
 template <typename Acc>
 __global__ __launch_bounds__(BT) void kb_finish(const double* __restrict__ part, int nbk, int nsums,
                                                 double* __restrict__ scal, int dst, const int* __restrict__ active,
-                                                int op) {
+                                                int op, int* __restrict__ m1, int* __restrict__ m2) {
   const int r = blockIdx.x;
-  if (active && !active[r]) return;
+  if (active && !active[r]) {
+    if (op == FIN_P2_CONVEX && threadIdx.x == 0) m1[r] = m2[r] = 0;
+    return;
+  }
   double* s = scal + (size_t)r * SCAL_COUNT;
   __shared__ double sums[2 * DOT_MAX];
   constexpr int PER_LANE = BMAX_BLOCKS / 64;
@@ -239,7 +248,14 @@ __global__ __launch_bounds__(BT) void kb_finish(const double* __restrict__ part,
     case FIN_P2_BETA1: p2::outer(s); p2::beta(s, 0); break;
     case FIN_P2_BETA2: p2::beta(s, 1); break;
     case FIN_P2_ALPHA: p2::alpha(s); break;
-    case FIN_P2_CONVEX: p2::convex(s); break;
+    case FIN_P2_CONVEX: {
+      // reliable-update masks from the convex step's flags (cu:474)
+      p2::convex(s);
+      const int f = s[SL_STATUS] == 0.0 ? (int)s[SL_FLAGS] : 0;
+      m1[r] = f & 1;
+      m2[r] = f & 2;
+      break;
+    }
     default: break;
   }
 }
@@ -420,25 +436,46 @@ __global__ __launch_bounds__(BT) void kb_p2_comb(float2* __restrict__ u0, float2
   }
 }
 
-// PBCGS2 reliable-update masks from the convex step's flags (cu:474):
-// m1 = active and rcmp, m2 = active and xpdt
-__global__ void kb_p2_masks(const double* __restrict__ scal, const int* __restrict__ active, int* __restrict__ m1,
-                            int* __restrict__ m2, int B) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= B) return;
-  const double* s = scal + (size_t)r * SCAL_COUNT;
-  const int on = active[r] && s[SL_STATUS] == 0.0;
-  const int f = (int)s[SL_FLAGS];
-  m1[r] = on && (f & 1);
-  m2[r] = on && (f & 2);
+// PBCGS2 reliable update (cu:474) of the RHS in m1 / m2:
+// m1: r0 = bp - A x (in sy);  m2: xp += x, x = 0, bp = r0
+template <typename R>
+__global__ __launch_bounds__(BT) void kb_p2_refresh(float2* __restrict__ r0, float2* __restrict__ bp,
+                                                    float2* __restrict__ xp, float2* __restrict__ x,
+                                                    const float2* __restrict__ sy, const int* __restrict__ m1,
+                                                    const int* __restrict__ m2, size_t n) {
+  const int r = blockIdx.y;
+  const bool f1 = m1[r] != 0, f2_ = m2[r] != 0;
+  if (!f1 && !f2_) return;
+  const size_t off = (size_t)r * n, gstride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gstride) {
+    const size_t k = off + i;
+    float2 v = r0[k];
+    if (f1) {
+      v = f2(cs(cv<R>(bp[k]), cv<R>(sy[k])));
+      r0[k] = v;
+    }
+    if (f2_) {
+      xp[k] = f2(ca(cv<R>(x[k]), cv<R>(xp[k])));
+      x[k] = make_float2(0.f, 0.f);
+      bp[k] = v;
+    }
+  }
 }
 
-// PBCGS2 reliable-update bookkeeping for the RHS in m1 (xpdt from m2)
-__global__ void kb_p2_reliable(double* __restrict__ scal, const int* __restrict__ m1, const int* __restrict__ m2,
-                               int B) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= B || !m1[r]) return;
-  p2::reliable_reals(scal + (size_t)r * SCAL_COUNT, m2[r]);
+// start vectors of a solve (or restart) in one pass: copies of src, then zeros
+struct StartVectors {
+  float2* v[9];
+  int copies, total;
+};
+__global__ __launch_bounds__(BT) void kb_start(const float2* __restrict__ src, StartVectors sv, size_t n,
+                                               const int* __restrict__ active) {
+  const int r = blockIdx.y;
+  if (active && !active[r]) return;
+  const size_t off = (size_t)r * n, gstride = (size_t)gridDim.x * blockDim.x;
+  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gstride) {
+    const float2 a = src[off + i];
+    for (int t = 0; t < sv.total; ++t) sv.v[t][off + i] = t < sv.copies ? a : make_float2(0.f, 0.f);
+  }
 }
 
 // PBCGS2 restart bookkeeping for the RHS in sel: |r| = sqrt(dot slot 0)
@@ -520,27 +557,47 @@ __global__ __launch_bounds__(BT) void kb_adj_grad(const float2* __restrict__ p, 
   }
 }
 
-// packed (status, relative residual, flags) per RHS for the host read-back
-__global__ void kb_pack(const double* __restrict__ scal, double* __restrict__ out, int B) {
+// (status, relative residual, flags) of every RHS into pinned host memory
+__global__ void kb_pack(const double* __restrict__ scal, double* __restrict__ hpacked, int B) {
   const int r = blockIdx.x * blockDim.x + threadIdx.x;
   if (r >= B) return;
-  out[3 * r] = scal[(size_t)r * SCAL_COUNT + SL_STATUS];
-  out[3 * r + 1] = scal[(size_t)r * SCAL_COUNT + SL_RESID];
-  out[3 * r + 2] = scal[(size_t)r * SCAL_COUNT + SL_FLAGS];
+  hpacked[3 * r] = scal[(size_t)r * SCAL_COUNT + SL_STATUS];
+  hpacked[3 * r + 1] = scal[(size_t)r * SCAL_COUNT + SL_RESID];
+  hpacked[3 * r + 2] = scal[(size_t)r * SCAL_COUNT + SL_FLAGS];
+}
+// scalars first .. first + count of every RHS into pinned host memory
+__global__ void kb_slots(const double* __restrict__ scal, int first, int count, double* __restrict__ hslots, int B) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= B) return;
+  for (int k = 0; k < count; ++k) hslots[r * count + k] = scal[(size_t)r * SCAL_COUNT + first + k];
+}
+// flags from pinned host memory; with ctl, also the start of a chunk of
+// iterations: check requests and the pause flag cleared
+__global__ void kb_flags(const int* __restrict__ hflags, int* __restrict__ flags, int* __restrict__ ctl, int B) {
+  const int r = blockIdx.x * blockDim.x + threadIdx.x;
+  if (r >= B) return;
+  flags[r] = hflags[r];
+  if (ctl) {
+    ctl[B + r] = 0;
+    if (r == 0) ctl[4 * B] = 0;
+  }
 }
 
 // End of a batched iteration, on the device, so that several iterations run
-// between host synchronisations: for every RHS that was active, count the
-// iteration (and, P2, a reliable-update MATVEC when flag bit 0 is set), keep
-// its recursive residual in the history, retire it on a breakdown status,
-// and request a host check when the reliable-residual period is reached,
-// the residual is at or below tol, or maxit is reached.  A request pauses
-// the whole batch: the active flags are saved and cleared, so the rest of
-// the launched iterations exit on entry until the host has run the checks.
-// One workgroup.
+// between host synchronisations: for every RHS that was active, finish the
+// reliable update (P2: the RHS in m1, x moved for those in m2), write its
+// status and residual to pinned host memory, count the iteration (and, P2, a
+// reliable-update MATVEC when flag bit 0 is set), keep its recursive residual
+// in the history, retire it on a breakdown status, and request a host check
+// when the reliable-residual period is reached, the residual is at or below
+// tol, or maxit is reached.  A request pauses the whole batch: the active
+// flags are saved and cleared, so the rest of the launched iterations exit on
+// entry until the host has run the checks.  One workgroup.
 template <bool P2>
-__global__ void kb_step_end(const double* __restrict__ packed, int* __restrict__ active, int* __restrict__ ctl,
-                            double* __restrict__ hist, int B, double tol, int maxit, int period) {
+__global__ void kb_step_end(double* __restrict__ scal, int* __restrict__ active, int* __restrict__ ctl,
+                            const int* __restrict__ m1, const int* __restrict__ m2, double* __restrict__ hpacked,
+                            int* __restrict__ hictl, double* __restrict__ hhist, int B, double tol, int maxit,
+                            int period) {
   __shared__ int pause;
   if (threadIdx.x == 0) pause = 0;
   __syncthreads();
@@ -550,16 +607,23 @@ __global__ void kb_step_end(const double* __restrict__ packed, int* __restrict__
   int* nxt = ctl + 3 * B;
   for (int r = threadIdx.x; r < B; r += blockDim.x) {
     if (!active[r]) continue;
-    const double st = packed[3 * r], rs = packed[3 * r + 1];
+    double* s = scal + (size_t)r * SCAL_COUNT;
+    if (P2 && m1[r]) p2::reliable_reals(s, m2[r]);
+    const double st = s[SL_STATUS], rs = s[SL_RESID], fl = s[SL_FLAGS];
+    hpacked[3 * r] = st;
+    hpacked[3 * r + 1] = rs;
+    hpacked[3 * r + 2] = fl;
     const int k = ++it[r];
-    if (P2) nxt[r] += ((int)packed[3 * r + 2]) & 1;
-    hist[(size_t)((k - 1) % HIST_ROWS) * B + r] = rs;
+    hictl[r] = k;
+    if (P2) hictl[2 * B + r] = nxt[r] += ((int)fl) & 1;
+    hhist[(size_t)((k - 1) % HIST_ROWS) * B + r] = rs;
     if (st != 0.0) {
       active[r] = 0;
       continue;
     }
     if (k % period == 0 || rs <= tol || k >= maxit) {
       sel[r] = 1;
+      hictl[B + r] = 1;
       pause = 1;
     }
   }
@@ -713,11 +777,11 @@ struct Ops {
     if (f64) {
       dot_dispatch(d.n, nv, DotsRun<double>{L, *this, mask});
       hipLaunchKernelGGL(kb_finish<double>, dim3(S.B), dim3(BT), 0, st, S.part, nbk_red, 2 * d.n, S.scal, dst,
-                         mask, op);
+                         mask, op, S.m1, S.m2);
     } else {
       dot_dispatch(d.n, nv, DotsRun<float>{L, *this, mask});
       hipLaunchKernelGGL(kb_finish<float>, dim3(S.B), dim3(BT), 0, st, S.part, nbk_red, 2 * d.n, S.scal, dst,
-                         mask, op);
+                         mask, op, S.m1, S.m2);
     }
     DDH_LAUNCH_OK("batched dots", 1);
     return 0;
@@ -741,66 +805,69 @@ struct Ops {
   int fin(int dst, int nsums, const int* mask, int op) {
     if (f64)
       hipLaunchKernelGGL(kb_finish<double>, dim3(S.B), dim3(BT), 0, st, S.part, nbk_vec, nsums, S.scal, dst, mask,
-                         op);
+                         op, S.m1, S.m2);
     else
       hipLaunchKernelGGL(kb_finish<float>, dim3(S.B), dim3(BT), 0, st, S.part, nbk_vec, nsums, S.scal, dst, mask,
-                         op);
+                         op, S.m1, S.m2);
     DDH_LAUNCH_OK("batched finish", 1);
     return 0;
   }
-  int pack() {
-    hipLaunchKernelGGL(kb_pack, dim3((S.B + 63) / 64), dim3(64), 0, st, S.scal, S.packed, S.B);
-    DDH_TRY(hipMemcpyAsync(S.hpacked, S.packed, (size_t)S.B * 3 * sizeof(double), hipMemcpyDeviceToHost, st),
-            "batched status D2H", 1);
-    return 0;
-  }
-  // device iteration bookkeeping after the pack of an iteration
+  dim3 rgrid() const { return dim3((unsigned)((S.B + 63) / 64)); }
+  // device iteration bookkeeping at the end of an iteration
   int step_end(bool p2, double tol, int maxit) {
-    if (p2) hipLaunchKernelGGL(kb_step_end<true>, dim3(1), dim3(256), 0, st, S.packed, S.active, S.ctl, S.hist, S.B,
-                               tol, maxit, RELIABLE_PERIOD);
-    else hipLaunchKernelGGL(kb_step_end<false>, dim3(1), dim3(256), 0, st, S.packed, S.active, S.ctl, S.hist, S.B,
-                            tol, maxit, RELIABLE_PERIOD);
+    if (p2) hipLaunchKernelGGL(kb_step_end<true>, dim3(1), dim3(256), 0, st, S.scal, S.active, S.ctl, S.m1, S.m2,
+                               S.hpacked, S.hictl, S.hhist, S.B, tol, maxit, RELIABLE_PERIOD);
+    else hipLaunchKernelGGL(kb_step_end<false>, dim3(1), dim3(256), 0, st, S.scal, S.active, S.ctl, S.m1, S.m2,
+                            S.hpacked, S.hictl, S.hhist, S.B, tol, maxit, RELIABLE_PERIOD);
     DDH_LAUNCH_OK("batched step end", 1);
     return 0;
   }
-  // check requests and the pause flag cleared before a chunk of iterations
-  int chunk_reset() {
-    DDH_TRY(hipMemsetAsync(S.ctl + S.B, 0, (size_t)S.B * sizeof(int), st), "batched iteration state", 1);
-    DDH_TRY(hipMemsetAsync(S.ctl + 4 * S.B, 0, sizeof(int), st), "batched iteration state", 1);
+  // flags h to the device in stream order.  The pinned staging rows are used
+  // in turn; a row is reused only after a synchronisation.
+  int uploads = 0;
+  int flags(int* dev, const std::vector<int>& h, int* ctl) {
+    if (uploads == FLAG_RING)
+      if (sync()) return 1;
+    int* row = S.hflags + (size_t)uploads++ * S.B;
+    std::copy(h.begin(), h.begin() + S.B, row);
+    hipLaunchKernelGGL(kb_flags, rgrid(), dim3(64), 0, st, row, dev, ctl, S.B);
+    DDH_LAUNCH_OK("batched flags", 1);
     return 0;
   }
-  // iteration state and residual history to the host, then a sync
-  int chunk_fetch() {
-    DDH_TRY(hipMemcpyAsync(S.hctl, S.ctl, ((size_t)4 * S.B + 1) * sizeof(int), hipMemcpyDeviceToHost, st),
-            "batched iteration state D2H", 1);
-    DDH_TRY(hipMemcpyAsync(S.hhist, S.hist, (size_t)HIST_ROWS * S.B * sizeof(double), hipMemcpyDeviceToHost, st),
-            "batched residual history D2H", 1);
-    return sync();
-  }
-  int upload(int* dev, const std::vector<int>& h) {
-    for (int r = 0; r < S.B; ++r) S.hflags[r] = h[r];
-    DDH_TRY(hipMemcpyAsync(dev, S.hflags, (size_t)S.B * sizeof(int), hipMemcpyHostToDevice, st), "flags H2D", 1);
-    // the pinned staging buffer is reused: wait for the copy
-    DDH_TRY(hipStreamSynchronize(st), "flags H2D", 1);
-    return 0;
+  int upload(int* dev, const std::vector<int>& h) { return flags(dev, h, nullptr); }
+  // start of a chunk of iterations of the RHS in act (a pause cleared the
+  // device flags); the stream is idle, so the pinned requests can be cleared here
+  int chunk_start(const std::vector<int>& act) {
+    std::fill(S.hictl + S.B, S.hictl + 2 * (size_t)S.B, 0);
+    return flags(S.active, act, S.ctl);
   }
   int sync() {
     DDH_TRY(hipStreamSynchronize(st), "batched sync", 1);
+    uploads = 0;
     return 0;
   }
   // fetch (status, resid) of every RHS
   int fetch() {
-    if (pack()) return 1;
+    hipLaunchKernelGGL(kb_pack, rgrid(), dim3(64), 0, st, S.scal, S.hpacked, S.B);
+    DDH_LAUNCH_OK("batched status", 1);
     return sync();
   }
-  // full scalar slot k of RHS r (after a sync): read via a small copy
+  // scalar slots first .. first + count of every RHS
   int fetch_slots(int first, int count, std::vector<double>& out) {
-    out.assign((size_t)S.B * count, 0.0);
-    for (int r = 0; r < S.B; ++r)
-      DDH_TRY(hipMemcpyAsync(out.data() + (size_t)r * count, S.scal + (size_t)r * SCAL_COUNT + first,
-                             (size_t)count * sizeof(double), hipMemcpyDeviceToHost, st),
-              "batched scalars D2H", 1);
-    return sync();
+    hipLaunchKernelGGL(kb_slots, rgrid(), dim3(64), 0, st, S.scal, first, count, S.hslots, S.B);
+    DDH_LAUNCH_OK("batched scalars", 1);
+    if (sync()) return 1;
+    out.assign(S.hslots, S.hslots + (size_t)S.B * count);
+    return 0;
+  }
+  // src into the first `copies` vectors of vs, zeros into the others
+  int start(const float2* src, std::initializer_list<float2*> vs, int copies, const int* mask) {
+    StartVectors sv{};
+    for (float2* v : vs) sv.v[sv.total++] = v;
+    sv.copies = copies;
+    hipLaunchKernelGGL(kb_start, vgrid(), dim3(BT), 0, st, src, sv, S.n, mask);
+    DDH_LAUNCH_OK("batched start vectors", 1);
+    return 0;
   }
 };
 
@@ -881,15 +948,10 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
   if (o.upload(S.active, act)) return 51;
   const int* A = S.active;
   const int* Sm = S.sel;
-  LinComb z;  // no terms: exact zeros, whatever the target held
   // |b|
   { DotSet ds; ds.add(b, b, DOT_N2); if (o.dots(ds, SL_D, A, FIN_BNORM)) return 52; }
   auto restart_from = [&](const float2* rs, const int* m) -> int {
-    LinComb cp; cp.lit(rs, 1.0);
-    if (o.lin(r, cp, m) || o.lin(vt, cp, m) || o.lin(wt, cp, m)) return 53;
-    for (float2* v : {p, ap, q, d, sv, atw})
-      if (o.lin(v, z, m)) return 53;
-    return 0;
+    return o.start(rs, {r, vt, wt, p, ap, q, d, sv, atw}, 3, m) ? 53 : 0;
   };
   auto init_scalars = [&](const int* m) -> int {
     if (int rc = o.mv(wt, atw, m)) return rc;
@@ -908,7 +970,8 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
   if (int rc = restart_from(sy, A)) return rc;
   if (int rc = init_scalars(A)) return rc;
   if (int rc = residual(A)) return rc;
-  if (o.fetch()) return 55;
+  std::vector<double> bn;
+  if (o.fetch() || o.fetch_slots(SLOT_BNORM, 1, bn)) return 55;
   for (int k = 0; k < B; ++k) {
     nc[k] = 2;
     resid[k] = S.hpacked[3 * k + 1];
@@ -916,7 +979,6 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
     if (status) { rcode[k] = status == 52 ? 52 : 55; act[k] = 0; }
     else if (!(resid[k] > tol)) act[k] = 0;  // converged at the initial guess (true residual)
   }
-  if (o.upload(S.active, act)) return 55;
   Graph gr;
   // true residual / gap for the RHS in `sel`; returns per-RHS outcomes
   std::vector<double> slots;
@@ -928,9 +990,7 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
     if (int rc = o.mv(xs, sy, Sm)) return rc;
     DotSet ds; ds.add(b, sy, DOT_D2).add(b, sy, DOT_G2, r);
     if (o.dots(ds, SL_D, Sm, FIN_NONE)) return 59;
-    if (o.sync() || o.fetch_slots(SL_D, 4, slots)) return 59;
-    std::vector<double> bn;
-    if (o.fetch_slots(SLOT_BNORM, 1, bn)) return 59;
+    if (o.fetch_slots(SL_D, 4, slots)) return 59;
     for (int k = 0; k < B; ++k) {
       conv[k] = rst[k] = 0;
       if (!sel[k]) continue;
@@ -967,32 +1027,32 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
                          S.part, o.nbk_vec);
     if (o.fin(SLOT_R2, 2, A, FIN_RESID)) return 59;
     DDH_LAUNCH_OK("QMRCCG batch step", 56);
-    if (o.pack()) return 56;
     return o.step_end(false, tol, maxit);
   };
   // iterations run in chunks: kb_step_end counts them on the device and
   // pauses the batch when a RHS needs the host (check, convergence, maxit)
   DDH_TRY(hipMemsetAsync(S.ctl, 0, ((size_t)4 * B + 1) * sizeof(int), o.st), nm, 51);
+  std::fill(S.hictl, S.hictl + 3 * (size_t)B, 0);
   int kchunk = 0;
   while (any_set(act)) {
     int itc = 0;
     for (int k = 0; k < B; ++k)
       if (act[k]) { itc = it[k]; break; }
     kchunk = next_chunk(itc, maxit, kchunk, 1e9);
-    if (o.chunk_reset()) return 59;
+    if (o.chunk_start(act)) return 59;
     for (int i = 0; i < kchunk; ++i)
       if (int rc = run_step(o, gr, use_graph && itc >= GRAPH_FROM_ITER, body)) return rc;
-    if (o.chunk_fetch()) return 59;
+    if (o.sync()) return 59;
     std::fill(sel.begin(), sel.end(), 0);
     double pred = 1e9;
     for (int k = 0; k < B; ++k) {
       if (!act[k]) continue;
-      const int n_it = S.hctl[k] - it[k];
+      const int n_it = S.hictl[k] - it[k];
       nc[k] += 2 * n_it;
       const int status = (int)S.hpacked[3 * k];
       for (int j = 0; j < (status ? n_it - 1 : n_it); ++j)
         c.log.iter(k, S.hhist[(size_t)((it[k] + j) % HIST_ROWS) * B + k]);
-      it[k] = S.hctl[k];
+      it[k] = S.hictl[k];
       if (status) {
         rcode[k] = 58;
         act[k] = 0;
@@ -1000,7 +1060,7 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
       }
       const double r0 = resid[k];
       resid[k] = S.hpacked[3 * k + 1];
-      sel[k] = S.hctl[B + k];
+      sel[k] = S.hictl[B + k];
       pred = std::min(pred, iters_to_tol(r0, resid[k], n_it, tol));
     }
     kchunk = next_chunk(0, RELIABLE_PERIOD, kchunk, pred);
@@ -1038,8 +1098,6 @@ int bsolve_qmrccg(Context& c, BatchState& S, const float2* b, float2* x, const f
         }
       }
     }
-    // a pause cleared the device flags
-    if (o.upload(S.active, act)) return 59;
   }
   DDH_TRY(hipMemcpyAsync(x, xs, vb, hipMemcpyDeviceToDevice, o.st), nm, 61);
   if (o.sync()) return 61;
@@ -1077,7 +1135,6 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
   if (o.upload(S.active, act)) return 92;
   const int* A = S.active;
   const int* Sm = S.sel;
-  LinComb z;  // no terms: exact zeros, whatever the target held
   // r0 = b - A xp for nonzero initial guesses, b otherwise (ZBCG2 NONZERO_X)
   { DotSet ds; ds.add(xp, xp, DOT_N2); if (o.dots(ds, SL_D, A, FIN_NONE)) return 92; }
   if (o.fetch_slots(SL_D, 1, slots)) return 92;
@@ -1090,9 +1147,7 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
     if (o.lin(r0, l, Sm)) return 92;
     for (int k = 0; k < B; ++k) nc[k] += sel[k];
   }
-  { LinComb cp; cp.lit(r0, 1.0); if (o.lin(rr, cp, A) || o.lin(bp, cp, A)) return 92; }
-  for (float2* v : {r1, r2, u0, u1, u2, xv})
-    if (o.lin(v, z, A)) return 92;
+  if (o.start(r0, {rr, bp, r1, r2, u0, u1, u2, xv}, 2, A)) return 92;
   { DotSet ds; ds.add(r0, r0, DOT_N2); if (o.dots(ds, SL_D, A, FIN_P2_INIT)) return 92; }
   if (o.fetch_slots(p2::RNRM0, 1, slots)) return 92;
   for (int k = 0; k < B; ++k) {
@@ -1100,8 +1155,6 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
     resid[k] = rnrm0[k] > 0.0 ? 1.0 : 0.0;
     if (!(resid[k] > tol)) act[k] = 0;
   }
-  if (o.upload(S.active, act)) return 92;
-  const dim3 sg((B + 63) / 64), sb(64);
   auto body = [&]() -> int {
     // first half-step (j = 0)
     { DotSet ds; ds.add(rr, r0, DOT_C); if (o.dots(ds, SL_D, A, FIN_P2_BETA1)) return 94; }
@@ -1129,21 +1182,17 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
     if (o.f64) hipLaunchKernelGGL(kb_p2_comb<double>, o.vgrid(), dim3(BT), 0, o.st, u0, xv, r0, u1, u2, r1, r2, S.scal, S.n, A);
     else hipLaunchKernelGGL(kb_p2_comb<float>, o.vgrid(), dim3(BT), 0, o.st, u0, xv, r0, u1, u2, r1, r2, S.scal, S.n, A);
     // reliable update of r (and x into xp) where the convex step asked for it
-    hipLaunchKernelGGL(kb_p2_masks, sg, sb, 0, o.st, S.scal, A, S.m1, S.m2, B);
     if (int rc = o.mv(xv, sy, S.m1)) return rc;
-    { LinComb l; l.lit(bp, 1.0).lit(sy, -1.0); if (o.lin(r0, l, S.m1)) return 104; }
-    { LinComb l; l.lit(xv, 1.0).lit(xp, 1.0); if (o.lin(xp, l, S.m2)) return 104; }
-    if (o.lin(xv, z, S.m2)) return 104;
-    { LinComb cp; cp.lit(r0, 1.0); if (o.lin(bp, cp, S.m2)) return 104; }
-    hipLaunchKernelGGL(kb_p2_reliable, sg, sb, 0, o.st, S.scal, S.m1, S.m2, B);
+    if (o.f64) hipLaunchKernelGGL(kb_p2_refresh<double>, o.vgrid(), dim3(BT), 0, o.st, r0, bp, xp, xv, sy, S.m1, S.m2, S.n);
+    else hipLaunchKernelGGL(kb_p2_refresh<float>, o.vgrid(), dim3(BT), 0, o.st, r0, bp, xp, xv, sy, S.m1, S.m2, S.n);
     DDH_LAUNCH_OK("PBCGS2 batch step", 103);
-    if (o.pack()) return 103;
     return o.step_end(true, tol, maxit);
   };
   Graph gr;
   std::vector<double> bn;
   // iterations in chunks between host checks, as in the batched QMRCCG
   DDH_TRY(hipMemsetAsync(S.ctl, 0, ((size_t)4 * B + 1) * sizeof(int), o.st), nm, 92);
+  std::fill(S.hictl, S.hictl + 3 * (size_t)B, 0);
   std::vector<int> nxt(B, 0);
   int kchunk = 0;
   while (any_set(act)) {
@@ -1151,22 +1200,22 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
     for (int k = 0; k < B; ++k)
       if (act[k]) { itc = it[k]; break; }
     kchunk = next_chunk(itc, maxit, kchunk, 1e9);
-    if (o.chunk_reset()) return 103;
+    if (o.chunk_start(act)) return 103;
     for (int i = 0; i < kchunk; ++i)
       if (int rc = run_step(o, gr, use_graph && itc >= GRAPH_FROM_ITER, body)) return rc;
-    if (o.chunk_fetch()) return 103;
+    if (o.sync()) return 103;
     std::fill(sel.begin(), sel.end(), 0);
     double pred = 1e9;
     for (int k = 0; k < B; ++k) {
       if (!act[k]) continue;
-      const int n_it = S.hctl[k] - it[k];
-      const int nx_now = S.hctl[3 * B + k];
+      const int n_it = S.hictl[k] - it[k];
+      const int nx_now = S.hictl[2 * B + k];
       nc[k] += 4 * n_it + (nx_now - nxt[k]);
       nxt[k] = nx_now;
       const int status = (int)S.hpacked[3 * k];
       for (int j = 0; j < (status ? n_it - 1 : n_it); ++j)
         c.log.iter(k, S.hhist[(size_t)((it[k] + j) % HIST_ROWS) * B + k]);
-      it[k] = S.hctl[k];
+      it[k] = S.hictl[k];
       if (status) {
         rcode[k] = status;
         act[k] = 0;
@@ -1174,14 +1223,11 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
       }
       const double r0 = resid[k];
       resid[k] = S.hpacked[3 * k + 1];
-      sel[k] = S.hctl[B + k];
+      sel[k] = S.hictl[B + k];
       pred = std::min(pred, iters_to_tol(r0, resid[k], n_it, tol));
     }
     kchunk = next_chunk(0, RELIABLE_PERIOD, kchunk, pred);
-    if (!any_set(sel)) {
-      if (o.upload(S.active, act)) return 104;
-      continue;
-    }
+    if (!any_set(sel)) continue;
     // true residual |bp - A x| and gap |bp - A x - r0| (cu:543-556)
     if (o.upload(S.sel, sel)) return 104;
     if (int rc = o.mv(xv, sy, Sm)) return rc;
@@ -1209,16 +1255,10 @@ int bsolve_pbcgs2(Context& c, BatchState& S, const float2* b, float2* x, const f
       if (o.upload(S.sel, sel)) return 104;
       LinComb lr; lr.lit(bp, 1.0).lit(sy, -1.0);
       LinComb lx; lx.lit(xv, 1.0).lit(xp, 1.0);
-      LinComb cp; cp.lit(r0, 1.0);
-      if (o.lin(r0, lr, Sm) || o.lin(xp, lx, Sm) || o.lin(xv, z, Sm) || o.lin(bp, cp, Sm) || o.lin(rr, cp, Sm))
-        return 104;
-      for (float2* v : {r1, r2, u0, u1, u2})
-        if (o.lin(v, z, Sm)) return 104;
-      hipLaunchKernelGGL(kb_p2_restart, sg, sb, 0, o.st, S.scal, Sm, B);
+      if (o.lin(r0, lr, Sm) || o.lin(xp, lx, Sm) || o.start(r0, {bp, rr, xv, r1, r2, u0, u1, u2}, 2, Sm)) return 104;
+      hipLaunchKernelGGL(kb_p2_restart, o.rgrid(), dim3(64), 0, o.st, S.scal, Sm, B);
       DDH_LAUNCH_OK("PBCGS2 batch restart", 104);
     }
-    // a pause cleared the device flags
-    if (o.upload(S.active, act)) return 104;
   }
   // ZBCG2 returns X + XP with one final true residual (cu:1258-1264)
   std::fill(act.begin(), act.end(), 1);
@@ -1304,8 +1344,7 @@ extern "C" DDSCAT_HIP_API int ddscat_hip_evalq_batch(int nrhs, const void* e, co
     rabs[r] = (float)(akk[r] * ak2 / 1.5);
   }
   hipStream_t st = c.stream;
-  // the per-RHS k^3 terms travel in the partials buffer's head (overwritten by the dots below)
-  float* drabs = (float*)S.part;
+  float* drabs = (float*)S.fac;
   DDH_TRY(hipMemcpyAsync(drabs, rabs.data(), nrhs * sizeof(float), hipMemcpyHostToDevice, st), "evalq_batch", 303);
   float2* q = S.W;
   const size_t os = op_per_rhs ? S.n : 0;
@@ -1363,7 +1402,7 @@ extern "C" DDSCAT_HIP_API int ddscat_hip_cabs_adjoint(int method, int nrhs, cons
     fac[nrhs + r] = (float)(k * ak2 / 1.5);
   }
   hipStream_t st = c.stream;
-  float* dfac = (float*)S.packed;  // 2 nrhs floats fit the 3 nrhs doubles of the status buffer
+  float* dfac = (float*)S.fac;  // 2 nrhs floats
   DDH_TRY(hipMemcpyAsync(dfac, fac.data(), fac.size() * sizeof(float), hipMemcpyHostToDevice, st), "cabs_adjoint", 3);
   const size_t os = op_per_rhs ? S.n : 0;
   const unsigned nb = (unsigned)std::min<size_t>(1024, (c.nat0 + BT - 1) / BT);
@@ -1376,8 +1415,6 @@ extern "C" DDSCAT_HIP_API int ddscat_hip_cabs_adjoint(int method, int nrhs, cons
   const int src = fn(c, S, rhs, mu, (const float2*)adia, (const float2*)aoff, os, maxit, (double)tol, itno, tole,
                      nc.data(), true);
   if (src) return src;
-  // the solve used the status buffer: upload the factors again
-  DDH_TRY(hipMemcpyAsync(dfac, fac.data(), nrhs * sizeof(float), hipMemcpyHostToDevice, st), "cabs_adjoint", 3);
   hipLaunchKernelGGL(kb_adj_grad, dim3(nb, nrhs), dim3(BT), 0, st, (const float2*)p, (const float2*)mu, dfac,
                      (float2*)g_adia, (float2*)g_aoff, c.nat0);
   DDH_LAUNCH_OK("adjoint gradient", 3);
