@@ -6,14 +6,17 @@
 //
 // SCAT: S(k_s) = sum_j P_j exp(-i k_s . r_j), r_j = ((i+1) + x0) dx per axis.
 // The lattice makes the phase separable, exp(-i k.r) = Ex(ix) Ey(iy) Ez(iz),
-// so per direction and lattice row (iy,iz) the kernel forms
-// T = sum_ix Ex(ix) P(ix,iy,iz) over the row's occupied sites (a contiguous
-// compact range) and adds Ey Ez T: three complex FP64 multiply-adds per site
-// and direction, no transcendental per site.  Per-axis phase tables are built
-// in FP64 on the device; row-chunk partials are reduced in a fixed order.
+// and the sites of a row lie symmetrically about its middle, so the row sum
+// is Ex(middle) times real cosines and sines of the sums and differences of
+// mirrored sites: a real matrix product (directions x sites) (sites x rows)
+// that runs on the FP64 matrix cores, at half the multiply-adds of the
+// complex sum (k_farfield_tiles).  Ey Ez weights and the sum over rows follow
+// in registers.  Per-axis phase tables are built in FP64 on the device;
+// row-chunk partials are reduced in a fixed order.
 // Angular quadrature (directions, weights) is restated from cu:849-875 on
 // the host.
 #include "solvers.hpp"
+#include "mv_device.hpp"
 #include "../../include/ddscat_matvec_hip.h"
 #include <vector>
 #include <cmath>
@@ -142,41 +145,203 @@ __global__ void k_phase_tables(const float* __restrict__ kd, int ndir, int nx, i
   tab[(size_t)i * ndir + d] = make_double2(co, -s);
 }
 
-constexpr int FF_DIRS = 64;    // directions per workgroup (one per lane)
-constexpr int FF_ROWS = 32;    // lattice rows per workgroup
+// The tables of k_farfield_tiles, direction fastest: entry i < J = ceil(nx/2)
+// holds (cos, sin) of k_x h_i, h_i = ((nx-1)/2 - i) dx the distance of sites i
+// and nx-1-i from the row's middle; then ny entries Ey and nz entries Ez, the
+// latter times the phase of the row's middle.
+__global__ void k_phase_tables_mid(const float* __restrict__ kd, int ndir, int nx, int ny, int nz, double dx1,
+                                   double dx2, double dx3, double x01, double x02, double x03,
+                                   double2* __restrict__ tab) {
+  const int J = (nx + 1) / 2, L = J + ny + nz;
+  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (id >= (size_t)ndir * L) return;
+  const int i = (int)(id / ndir), d = (int)(id - (size_t)i * ndir);
+  double s, co;
+  if (i < J) {
+    sincos(kd[3 * d] * (0.5 * (double)(nx - 1 - 2 * i) * dx1), &s, &co);
+    tab[id] = make_double2(co, s);
+  } else if (i < J + ny) {
+    sincos(kd[3 * d + 1] * (((double)(i - J + 1) + x02) * dx2), &s, &co);
+    tab[id] = make_double2(co, -s);
+  } else {
+    sincos(kd[3 * d + 2] * (((double)(i - J - ny + 1) + x03) * dx3), &s, &co);
+    double sm, cm;
+    sincos(kd[3 * d] * ((0.5 * (double)(nx + 1) + x01) * dx1), &sm, &cm);
+    tab[id] = zmul(make_double2(co, -s), make_double2(cm, -sm));
+  }
+}
 
-// partial[chunk][d][3] = sum over the chunk's rows of Ey Ez sum_row Ex P
-__global__ __launch_bounds__(FF_DIRS) void k_farfield_rows(
-    const float2* __restrict__ p, const int* __restrict__ occ, const int* __restrict__ rowptr,
-    const double2* __restrict__ tab, int ndir, int nx, int ny, int nz, int nat0, double2* __restrict__ part) {
-  const int chunk = blockIdx.x;
-  const int d = blockIdx.y * FF_DIRS + threadIdx.x;
-  const int nrows = ny * nz;
-  const int g0 = chunk * FF_ROWS, g1 = min(nrows, g0 + FF_ROWS);
-  double2 s0 = make_double2(0, 0), s1 = s0, s2 = s0;
-  if (d < ndir) {
-    const double2* t = tab + d;
-    const size_t sd = (size_t)ndir;
-    for (int g = g0; g < g1; ++g) {
-      const int q0 = rowptr[g], q1 = rowptr[g + 1];
-      if (q0 == q1) continue;
-      double2 r0 = make_double2(0, 0), r1 = r0, r2 = r0;
-      const int base = g * nx;
-      for (int q = q0; q < q1; ++q) {
-        const double2 e = t[(size_t)(occ[q] - base) * sd];
-        const float2 a = p[q], b = p[q + nat0], cc = p[q + 2 * nat0];
-        r0.x += e.x * a.x - e.y * a.y; r0.y += e.x * a.y + e.y * a.x;
-        r1.x += e.x * b.x - e.y * b.y; r1.y += e.x * b.y + e.y * b.x;
-        r2.x += e.x * cc.x - e.y * cc.y; r2.y += e.x * cc.y + e.y * cc.x;
+constexpr int FF_DIRS = 64;    // directions per workgroup of the position-weighted sums (one per lane)
+constexpr int FF_ROWS = 32;    // lattice rows per workgroup
+constexpr int FF_GROUP = 8;    // lattice rows per matrix product: 8 rows x (re, im) = 16 columns per component
+constexpr int FF_WAVES = 8;    // waves per workgroup: 16 directions each, and one row of a group to stage each
+constexpr int FF_PAIRS = 64;   // site pairs per LDS stage, one per lane
+static_assert(FF_GROUP == FF_WAVES && FF_PAIRS == 64, "a wave stages one row, a lane one pair");
+
+template <int CTL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+
+// partial[pol][chunk][d][3] = sum over the chunk's rows of Ey Ez sum_row Ex P.
+// FF_GROUP rows at a time: with S and D the sum and difference of the sites
+// at +h and -h from a row's middle,
+//   sum_row Ex P = Ex(mid) sum_h [ cos(k h) S - i sin(k h) D ],
+// i.e. columns (Sr, Si) against cosines plus (Di, -Dr) against sines.  The
+// workgroup forms the columns of 64 site pairs in LDS once for all its
+// directions, and every wave multiplies them with the table entries of its 16
+// (mfma f64 16x16x4: A lane (direction l%16, pair l/16), B lane (pair l/16,
+// column l%16), D[t] lane (direction 4t + l/16, column l%16)); three
+// components give three independent accumulators.  Outer pairs that no row of
+// the group occupies are skipped.  The next stage's sites are read while the
+// current one is multiplied, and s[][] keeps one part per lane (real parts in
+// columns < FF_GROUP), which holds the kernel at 4 waves per SIMD.
+// Bound by FP64 matrix issue: a 128^3 sphere (1.10 M sites), two
+// polarizations, 724 directions in 625 us, matrix cores busy 60 % of its
+// cycles (sites read in front of their use and both parts per lane: 750 us;
+// 132 registers, so 3 waves per SIMD: 905 us; one lane per direction and a
+// complex multiply-add per site on the vector units: 3180 us).
+__global__ __launch_bounds__(64 * FF_WAVES, 4) void k_farfield_tiles(
+    const float2* __restrict__ pin, const int* __restrict__ occ, SiteMap sm, const double2* __restrict__ tab, int ndir,
+    int nx, int ny, int nz, int nat0, double2* __restrict__ part) {
+  typedef double v4d __attribute__((ext_vector_type(4)));
+  constexpr int PITCH = 3 * 16 + 1;  // entries per pair; odd, so that the stage's writes spread over the banks
+  constexpr int GROUPS = FF_ROWS / FF_GROUP;
+  __shared__ double2 cols[FF_PAIRS * PITCH];
+  const int chunk = blockIdx.x, nchunks = gridDim.x, pol = blockIdx.z;
+  const int lane = threadIdx.x & 63, lc = lane & 15, lk = lane >> 4;
+  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+  const int d0 = (blockIdx.y + w * gridDim.y) * 16;  // tiles dealt out so that a short last round is shared
+  const int nrows = ny * nz, J = (nx + 1) / 2;
+  const size_t sd = (size_t)ndir;
+  const float2* p = pin + (size_t)pol * 3 * nat0;
+  const double2* ta = tab + min(d0 + lc, ndir - 1);
+
+  // lane r < FF_ROWS: row r of the chunk, its compact range and its outermost occupied pair
+  int rq0 = 0, rcnt = 0, rlo = 0, rout = J;
+  const int gl = min(chunk * FF_ROWS + lane, nrows - 1), riz = gl / ny, riy = gl - riz * ny;
+  {
+    const int g = chunk * FF_ROWS + lane;
+    if (lane < FF_ROWS && g < nrows) {
+      rq0 = sm.rowptr[g];
+      rcnt = sm.rowptr[g + 1] - rq0;
+      rlo = sm.rowlo[g];
+      if (rcnt > 0) {
+        const int last = sm.contiguous ? rlo + rcnt - 1 : occ[rq0 + rcnt - 1] - g * nx;
+        rout = min(rlo, nx - 1 - last);
       }
-      const int iy = g % ny, iz = g / ny;
-      const double2 eyz = zmul(t[(size_t)(nx + iy) * sd], t[(size_t)(nx + ny + iz) * sd]);
-      s0 = zadd(s0, zmul(eyz, r0));
-      s1 = zadd(s1, zmul(eyz, r1));
-      s2 = zadd(s2, zmul(eyz, r2));
     }
-    double2* o = part + ((size_t)chunk * ndir + d) * 3;
-    o[0] = s0; o[1] = s1; o[2] = s2;
+    rout = min(rout, __shfl_xor(rout, 1));
+    rout = min(rout, __shfl_xor(rout, 2));
+    rout = min(rout, __shfl_xor(rout, 4));
+  }
+  // first stage of group k: whole steps of 4 pairs end at the row's middle; pairs before 0 are empty columns
+  auto start = [&](int k) {
+    const int out = __builtin_amdgcn_readlane(rout, k * FF_GROUP);
+    return J - ((J - out + 3) & ~3);
+  };
+  auto skip_empty = [&](int& k, int& i0) {
+    for (; k < GROUPS; ++k)
+      if ((i0 = start(k)) < J) return;
+  };
+  float2 m[3], q[3];  // this lane's pair of the wave's row: sites i and nx - 1 - i
+  auto fetch = [&](int k, int i0) {
+    const int i = i0 + lane, r = k * FF_GROUP + w;
+    int qm = -1, qp = -1;
+    const int q0 = __builtin_amdgcn_readlane(rq0, r), cnt = __builtin_amdgcn_readlane(rcnt, r),
+              lo = __builtin_amdgcn_readlane(rlo, r);
+    if (i >= 0 && i < J) {
+      if (sm.contiguous) {
+        const unsigned dm = (unsigned)(i - lo), dp = (unsigned)(nx - 1 - i - lo);
+        qm = dm < (unsigned)cnt ? q0 + (int)dm : -1;
+        qp = dp < (unsigned)cnt ? q0 + (int)dp : -1;
+      } else if (chunk * FF_ROWS + r < nrows) {
+        const int* row = sm.qmap + (size_t)(chunk * FF_ROWS + r) * nx;
+        qm = row[i];
+        qp = row[nx - 1 - i];
+      }
+      if (2 * i + 1 == nx) qp = -1;  // the middle site stands alone
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      m[c] = qm >= 0 ? p[qm + (size_t)c * nat0] : make_float2(0.f, 0.f);
+      q[c] = qp >= 0 ? p[qp + (size_t)c * nat0] : make_float2(0.f, 0.f);
+    }
+  };
+
+  double s[3][4];  // columns < FF_GROUP: real parts, the others: imaginary parts
+#pragma unroll
+  for (int c = 0; c < 3; ++c)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) s[c][t] = 0.0;
+  v4d acc[3];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) acc[c] = v4d{0.0, 0.0, 0.0, 0.0};
+  int k = 0, i0 = 0;
+  skip_empty(k, i0);
+  if (k < GROUPS) fetch(k, i0);
+  while (k < GROUPS) {
+    __syncthreads();  // the previous stage is read
+    {
+      double2* o = cols + lane * PITCH + w;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        o[c * 16] = make_double2((double)q[c].x + m[c].x, (double)q[c].y - m[c].y);
+        o[c * 16 + FF_GROUP] = make_double2((double)q[c].y + m[c].y, (double)m[c].x - q[c].x);
+      }
+    }
+    __syncthreads();
+    const int kc = k, ic = i0;
+    i0 += FF_PAIRS;
+    if (i0 >= J) skip_empty(++k, i0);
+    double2 next = d0 < ndir ? ta[(size_t)max(ic + lk, 0) * sd] : make_double2(0, 0);
+    if (k < GROUPS) fetch(k, i0);
+    if (d0 >= ndir) continue;
+    const int steps = min(J - ic, FF_PAIRS) / 4;
+    const double2* b = cols + lk * PITCH + lc;
+    const double2* tn = ta + (ptrdiff_t)(ic + lk) * (ptrdiff_t)sd;
+    for (int st = 0; st < steps; ++st) {
+      const double2 a = next;
+      tn += 4 * sd;
+      if (st + 1 < steps) next = *tn;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b[16 * c].x, acc[c], 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 3; ++c) acc[c] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b[16 * c].y, acc[c], 0, 0, 0);
+      b += 4 * PITCH;
+    }
+    if (k == kc) continue;  // the group goes on
+    const int r = kc * FF_GROUP + (lc & (FF_GROUP - 1));
+    const double2 *ty = tab + (size_t)(J + __shfl(riy, r)) * sd, *tz = tab + (size_t)(J + ny + __shfl(riz, r)) * sd;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const int d = min(d0 + 4 * t + lk, ndir - 1);
+      const double2 e = zmul(ty[d], tz[d]);
+      const double ei = lc < FF_GROUP ? -e.y : e.y;  // times the other part
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        s[c][t] += e.x * acc[c][t];
+        s[c][t] += ei * dpp_move<0x128>(acc[c][t]);  // row_ror:8
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) acc[c] = v4d{0.0, 0.0, 0.0, 0.0};
+  }
+  if (d0 >= ndir) return;
+#pragma unroll
+  for (int t = 0; t < 4; ++t) {
+    const int d = d0 + 4 * t + lk;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      double v = s[c][t];  // over the 8 columns of this lane's part
+      v += dpp_move<0x141>(v);  // row_half_mirror
+      v += dpp_move<0xb1>(v);   // quad_perm [1,0,3,2]
+      v += dpp_move<0x4e>(v);   // quad_perm [2,3,0,1]
+      if ((lc & (FF_GROUP - 1)) == 0 && d < ndir)
+        reinterpret_cast<double*>(part)[((((size_t)pol * nchunks + chunk) * ndir + d) * 3 + c) * 2 + lc / FF_GROUP] = v;
+    }
   }
 }
 
@@ -234,14 +399,30 @@ __global__ __launch_bounds__(FF_DIRS) void k_farfield_rows_pos(
   for (int i = 0; i < 12; ++i) o[i] = acc[i];
 }
 
-// S[d][width] = sum over chunks of partial[chunk][d][width], fixed order
-__global__ void k_farfield_reduce(const double2* __restrict__ part, int nchunks, int ndir, int width,
-                                  double2* __restrict__ S) {
-  const size_t id = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= (size_t)ndir * width) return;
+// S[pol][id] = sum over chunks of partial[pol][chunk][id], id < ids, fixed
+// order: 16 slices of the chunks per workgroup of 32 sums, each slice summed
+// in order, then the slices.  (One thread per sum waited for every load of a
+// chain of nchunks: 130 us for 512 chunks of 724 directions.)
+constexpr int FF_RED_IDS = 32, FF_RED_SLICES = 16;
+__global__ __launch_bounds__(FF_RED_IDS * FF_RED_SLICES) void k_farfield_reduce(const double2* __restrict__ part,
+                                                                                int nchunks, int ids, size_t spitch,
+                                                                                double2* __restrict__ S) {
+  __shared__ double2 sl[FF_RED_SLICES][FF_RED_IDS];
+  const int il = threadIdx.x % FF_RED_IDS, slice = threadIdx.x / FF_RED_IDS;
+  const int id = blockIdx.x * FF_RED_IDS + il;
+  const double2* src = part + (size_t)blockIdx.y * nchunks * ids;
+  const int per = (nchunks + FF_RED_SLICES - 1) / FF_RED_SLICES, c0 = slice * per, c1 = min(nchunks, c0 + per);
   double2 acc = make_double2(0, 0);
-  for (int ch = 0; ch < nchunks; ++ch) acc = zadd(acc, part[(size_t)ch * ndir * width + id]);
-  S[id] = acc;
+  if (id < ids)
+#pragma unroll 8
+    for (int ch = c0; ch < c1; ++ch) acc = zadd(acc, src[(size_t)ch * ids + id]);
+  sl[slice][il] = acc;
+  __syncthreads();
+  if (slice == 0 && id < ids) {
+#pragma unroll
+    for (int k = 1; k < FF_RED_SLICES; ++k) acc = zadd(acc, sl[k][il]);
+    S[blockIdx.y * spitch + id] = acc;
+  }
 }
 
 // Incident-beam torque terms, per workgroup: out[blk][0..2] = sum Im(P^* . E) r,
@@ -292,34 +473,31 @@ __global__ __launch_bounds__(TQ_THREADS) void k_torque_local(const float2* __res
   }
 }
 
-// S[d][3] for all directions (host result) of the compact polarization p.
+// S[pol][d][3] for all directions (host result) of npol consecutive compact
+// polarizations p[npol][3][nat0].
 // Device workspace (directions, phase tables, row-chunk partials, sums):
 // allocated per call, or carved out of `region` (the allocation-free SCAT
 // entry), where the direction slab shrinks to fit.  Returns 1 on failure, 2
 // when the region cannot hold even one direction's workspace.
 static int farfield_sums(Context& c, const float2* p, const std::vector<float>& kdirs, const float dx[3],
                          const float x0[3], std::vector<std::complex<double>>& S, const FarfieldRegion* region,
-                         bool pos = false) {
+                         bool pos = false, int npol = 1) {
   const int ndir = (int)(kdirs.size() / 3);
   const int width = pos ? 12 : 3;  // complex sums per direction: S, or S and the position-weighted R
-  S.assign((size_t)ndir * width, 0.0);
+  const size_t nsum = (size_t)ndir * width;
+  S.assign(npol * nsum, 0.0);
   if (ndir == 0) return 0;
   hipStream_t st = c.stream;
   const int L = c.nx + c.ny + c.nz;
   const int nrows = c.ny * c.nz;
   const int nchunks = (nrows + FF_ROWS - 1) / FF_ROWS;
-  float* dk = nullptr;
-  double2 *tab = nullptr, *part = nullptr, *dS = nullptr;
-  int rc = 0;
-  int slab = 0;
-  auto cleanup = [&]() {
-    if (region) return;
-    hipFree(dk); hipFree(tab); hipFree(part); hipFree(dS);
-  };
+  const SiteMap sm{c.rowptr, c.rowlo, c.qmap, c.rows_contiguous};
+  auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  const size_t fixed = up(kdirs.size() * sizeof(float)) + up(npol * nsum * sizeof(double2));
+  const size_t per_dir = (size_t)L * sizeof(double2) + (size_t)npol * nchunks * width * sizeof(double2);
+  unsigned char *own = nullptr, *base = nullptr;
+  int rc = 0, slab = 0;
   if (region) {
-    auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
-    const size_t fixed = up(kdirs.size() * sizeof(float)) + up((size_t)ndir * width * sizeof(double2));
-    const size_t per_dir = (size_t)L * sizeof(double2) + (size_t)nchunks * width * sizeof(double2);
     if (region->bytes < fixed + 512 + per_dir) {
       char msg[200];
       std::snprintf(msg, sizeof(msg), "far-field workspace of %d directions on %d lattice rows needs more than the "
@@ -328,24 +506,22 @@ static int farfield_sums(Context& c, const float2* p, const std::vector<float>& 
       return 2;
     }
     slab = (int)std::min<size_t>((size_t)ndir, (region->bytes - fixed - 512) / per_dir);
-    unsigned char* b = region->base;
-    dk = (float*)b; b += up(kdirs.size() * sizeof(float));
-    dS = (double2*)b; b += up((size_t)ndir * width * sizeof(double2));
-    tab = (double2*)b; b += up((size_t)slab * L * sizeof(double2));
-    part = (double2*)b;
+    base = region->base;
   } else {
     // bound the partial buffer: process directions in slabs
     slab = std::max(FF_DIRS, std::min(ndir, (int)std::max<size_t>(FF_DIRS, (size_t)(256u << 20) /
-                                                                    ((size_t)nchunks * width * sizeof(double2)))));
-    if (hipMalloc((void**)&dk, kdirs.size() * sizeof(float)) != hipSuccess ||
-        hipMalloc((void**)&tab, (size_t)slab * L * sizeof(double2)) != hipSuccess ||
-        hipMalloc((void**)&part, (size_t)nchunks * slab * width * sizeof(double2)) != hipSuccess ||
-        hipMalloc((void**)&dS, (size_t)ndir * width * sizeof(double2)) != hipSuccess) {
+                                                                    ((size_t)npol * nchunks * width * sizeof(double2)))));
+    if (hipMalloc((void**)&own, fixed + 512 + slab * per_dir) != hipSuccess) {
       set_error("GPU SCAT", "far-field workspace allocation failed");
-      cleanup();
       return 1;
     }
+    base = own;
   }
+  float* dk = (float*)base;
+  double2* dS = (double2*)(base + up(kdirs.size() * sizeof(float)));
+  double2* tab = (double2*)(base + fixed);
+  double2* part = (double2*)(base + fixed + up((size_t)slab * L * sizeof(double2)));
+  auto cleanup = [&]() { if (own) hipFree(own); };
   if (hipMemcpyAsync(dk, kdirs.data(), kdirs.size() * sizeof(float), hipMemcpyHostToDevice, st) != hipSuccess) {
     set_error("GPU SCAT", "directions H2D failed");
     cleanup();
@@ -353,22 +529,28 @@ static int farfield_sums(Context& c, const float2* p, const std::vector<float>& 
   }
   for (int d0 = 0; d0 < ndir && !rc; d0 += slab) {
     const int nd = std::min(slab, ndir - d0);
-    const size_t nt = (size_t)nd * L;
-    hipLaunchKernelGGL(k_phase_tables, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, dk + 3 * d0, nd, c.nx,
-                       c.ny, c.nz, (double)dx[0], (double)dx[1], (double)dx[2], (double)x0[0], (double)x0[1],
-                       (double)x0[2], tab);
-    if (pos)
+    if (pos) {
+      const size_t nt = (size_t)nd * L;
+      hipLaunchKernelGGL(k_phase_tables, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, dk + 3 * d0, nd, c.nx,
+                         c.ny, c.nz, (double)dx[0], (double)dx[1], (double)dx[2], (double)x0[0], (double)x0[1],
+                         (double)x0[2], tab);
       hipLaunchKernelGGL(k_farfield_rows_pos, dim3(nchunks, (nd + FF_DIRS - 1) / FF_DIRS), dim3(FF_DIRS), 0, st, p,
                          c.occ, c.rowptr, tab, nd, c.nx, c.ny, c.nz, c.nat0, (double)dx[0], (double)dx[1],
                          (double)dx[2], (double)x0[0], (double)x0[1], (double)x0[2], part);
-    else
-      hipLaunchKernelGGL(k_farfield_rows, dim3(nchunks, (nd + FF_DIRS - 1) / FF_DIRS), dim3(FF_DIRS), 0, st, p,
-                         c.occ, c.rowptr, tab, nd, c.nx, c.ny, c.nz, c.nat0, part);
-    hipLaunchKernelGGL(k_farfield_reduce, dim3((unsigned)((nd * width + 255) / 256)), dim3(256), 0, st, part,
-                       nchunks, nd, width, dS + (size_t)width * d0);
+    } else {
+      const size_t nt = (size_t)nd * ((c.nx + 1) / 2 + c.ny + c.nz);
+      hipLaunchKernelGGL(k_phase_tables_mid, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0, st, dk + 3 * d0, nd,
+                         c.nx, c.ny, c.nz, (double)dx[0], (double)dx[1], (double)dx[2], (double)x0[0], (double)x0[1],
+                         (double)x0[2], tab);
+      hipLaunchKernelGGL(k_farfield_tiles, dim3(nchunks, (nd + 16 * FF_WAVES - 1) / (16 * FF_WAVES), npol),
+                         dim3(64 * FF_WAVES), 0, st, p, c.occ, sm, tab, nd, c.nx, c.ny, c.nz, c.nat0, part);
+    }
+    hipLaunchKernelGGL(k_farfield_reduce, dim3((unsigned)((nd * width + FF_RED_IDS - 1) / FF_RED_IDS), npol),
+                       dim3(FF_RED_IDS * FF_RED_SLICES), 0, st, part, nchunks, nd * width, nsum,
+                       dS + (size_t)width * d0);
     if (hipGetLastError() != hipSuccess) { set_error("GPU SCAT", "far-field kernel launch failed"); rc = 1; }
   }
-  if (!rc && (hipMemcpyAsync(S.data(), dS, (size_t)ndir * width * sizeof(double2), hipMemcpyDeviceToHost, st) != hipSuccess ||
+  if (!rc && (hipMemcpyAsync(S.data(), dS, npol * nsum * sizeof(double2), hipMemcpyDeviceToHost, st) != hipSuccess ||
               hipStreamSynchronize(st) != hipSuccess)) {
     set_error("GPU SCAT", "far-field sums D2H failed");
     rc = 1;
@@ -596,9 +778,8 @@ int scat_matrix(Context& c, int npair, const float2* p, int ndir, const float* a
     }
     const size_t o = (size_t)q * ndir * 3;
     std::vector<float> kd(aks + o, aks + o + 3 * (size_t)ndir);
-    std::vector<std::complex<double>> S[2];
-    for (int j = 0; j < 2; ++j)
-      if (farfield_sums(c, p + (2 * (size_t)q + j) * n, kd, dx, x0, S[j], nullptr)) return 341;
+    std::vector<std::complex<double>> S;  // [2][ndir][3]
+    if (farfield_sums(c, p + 2 * (size_t)q * n, kd, dx, x0, S, nullptr, false, 2)) return 341;
     for (int d = 0; d < ndir; ++d) {
       const float* a = em1 + o + 3 * d;
       const float* b = em2 + o + 3 * d;
@@ -606,8 +787,8 @@ int scat_matrix(Context& c, int npair, const float2* p, int ndir, const float* a
       for (int j = 0; j < 2; ++j) {
         std::complex<double> s1 = 0.0, s2 = 0.0;
         for (int kk = 0; kk < 3; ++kk) {
-          s1 += (double)a[kk] * S[j][3 * d + kk];
-          s2 += (double)b[kk] * S[j][3 * d + kk];
+          s1 += (double)a[kk] * S[3 * ((size_t)j * ndir + d) + kk];
+          s2 += (double)b[kk] * S[3 * ((size_t)j * ndir + d) + kk];
         }
         f[2 * j] = term * s1;
         f[2 * j + 1] = term * s2;
