@@ -133,7 +133,7 @@ int finish_prepare(Context& c, const int16_t* iocc, int code_alloc, int code_occ
   c.rows_contiguous = contiguous ? 1 : 0;
   DDH_TRY(hipMalloc((void**)&c.rowlo, (size_t)nrows * sizeof(int)), "malloc row map", code_alloc);
   DDH_TRY(hipMemcpy(c.rowlo, rowlo.data(), (size_t)nrows * sizeof(int), hipMemcpyHostToDevice), "row map H2D", code_alloc);
-  if (!contiguous || c.backend == BACKEND_SLICES) {
+  if (!contiguous) {
     std::vector<int> qmap((size_t)c.nat, -1);
     for (size_t q = 0; q < occ.size() && q < (size_t)c.nat0; ++q) qmap[(size_t)occ[q]] = (int)q;
     DDH_TRY(hipMalloc((void**)&c.qmap, (size_t)c.nat * sizeof(int)), "malloc site map", code_alloc);
@@ -149,7 +149,7 @@ int finish_prepare(Context& c, const int16_t* iocc, int code_alloc, int code_occ
   DDH_TRY(hipMemcpy(c.rowptr, rowptr.data(), ((size_t)nrows + 1) * sizeof(int), hipMemcpyHostToDevice), "row map H2D", code_occ);
   DDH_TRY(hipMemset(c.adia, 0, n * sizeof(float2)), "clear adia", code_alloc);
   DDH_TRY(hipMemset(c.aoff, 0, n * sizeof(float2)), "clear aoff", code_alloc);
-  if (c.backend == BACKEND_FFT3D && matvec_autotune(c)) return code_alloc;
+  if (matvec_autotune(c)) return code_alloc;
   return 0;
 }
 

@@ -181,23 +181,16 @@ struct Reg2 {
 // kernels whose tiles are narrower than a 128-byte line (C < 16).  Blocks go
 // round-robin over the 8 XCDs by linear id, and each XCD has its own L2, so
 // the W = 16/C tiles sharing one line are given to blocks 8 ids apart (same
-// XCD, back to back); with `mirror` the group also holds the kx mirror tiles
-// NT-1-b, which read the same Green octant entries.  Falls back to the plain
-// order (mirror: b and NT-1-b h = ceil(NT/2) apart) when NT is not a multiple
-// of 8 times the group size or C >= 16.
+// XCD, back to back).  The plain order when NT is not a multiple of 8 times W
+// or C >= 16.
 template <int C>
-__device__ __forceinline__ int xcd_tile(int bx, int NT, bool mirror) {
+__device__ __forceinline__ int xcd_tile(int bx, int NT) {
   constexpr int W = C >= 16 ? 1 : 16 / C;
-  const int g = mirror ? 2 * W : W;
-  if (W > 1 && NT % (8 * g) == 0) {
+  if (W > 1 && NT % (8 * W) == 0) {
     const int m = bx >> 3, r = bx & 7;
-    const int q = r + 8 * (m / g), slot = m % g;
-    if (!mirror) return W * q + slot;
-    return slot < W ? W * q + slot : NT - 1 - (W * q + (slot - W));
+    return W * (r + 8 * (m / W)) + m % W;
   }
-  if (!mirror) return bx;
-  const int h = (NT + 1) / 2;
-  return bx < h ? bx : NT - 1 - (bx - h);
+  return bx;
 }
 
 // The padded axes have length L = R1 R2 = 2N with data (forward input) and
@@ -211,39 +204,20 @@ template <int R2>
 __device__ __forceinline__ bool lower_half(int n2, int n, int N) {
   return (2 * n2 + 1 < R2) || (2 * n2 + 1 == R2 && n < N);
 }
-// lane-pair layout: element i of lane-parity h holds n = t + Q (h + 2 i), t < Q
-template <int Q>
-__device__ __forceinline__ bool lower_half_pair(int i, int n, int N) {
-  return (2 * i + 1 < Q / 2) || (2 * i < Q / 2 && n < N);
-}
-
 template <int R1, int R2>
 __device__ __forceinline__ bool reg2_owns(int t, int i) {
   return Reg2<R1, R2>::G * R1 == R2 || t + R1 * i < R2;
 }
 
-// LDS exchange index of element (k2, n1) of sequence s.
-//  LAY 0 (column passes, lanes run over s): (k2 R1 + n1) P + s, P = C + 1.
-//  LAY 1 (row passes, lanes run over n1 when writing and over k2 when
-//  reading): s P + k2 (R1 + 1) + n1 with P >= R2 (R1 + 1): consecutive n1 and
-//  k2 strides of R1 + 1 both hit distinct banks.
-template <int LAY, int R1>
+// LDS exchange index of element (k2, n1) of sequence s: lanes run over s, P = C + 1
+template <int R1>
 __device__ __forceinline__ int lidx(int k2, int n1, int s, int P) {
-  return LAY == 0 ? (k2 * R1 + n1) * P + s : s * P + k2 * (R1 + 1) + n1;
-}
-// per-sequence stride for LAY 1: R2 (R1 + 1) rounded up so that two
-// sequences of one 32-lane half-wave fall on disjoint 4-byte banks (odd multiple of 16)
-template <int R1, int R2>
-__host__ __device__ constexpr int row_stride() {
-  const int base = R2 * (R1 + 1);
-  int s = (base + 15) / 16 * 16;
-  if ((s / 16) % 2 == 0) s += 16;
-  return s;
+  return (k2 * R1 + n1) * P + s;
 }
 
 // forward: v[n2] = x[t + R1 n2] (n2 < R2) in; v[i R1 + k1] = X[(t + R1 i) + R2 k1]
 // out for the groups i the thread owns
-template <int R1, int R2, int DIR, int LAY = 0>
+template <int R1, int R2, int DIR>
 __device__ __forceinline__ void fft2_fwd(float2* v, float2* __restrict__ lds, const float2* __restrict__ twL, int t,
                                          int s, int P) {
   dft_reg<R2, DIR>(v);
@@ -251,7 +225,7 @@ __device__ __forceinline__ void fft2_fwd(float2* v, float2* __restrict__ lds, co
   for (int k2 = 0; k2 < R2; ++k2) {
     float2 w = twL[t * k2];
     if (DIR < 0) w.y = -w.y;
-    lds[lidx<LAY, R1>(k2, t, s, P)] = k2 == 0 ? v[0] : cmul(v[k2], w);
+    lds[lidx<R1>(k2, t, s, P)] = k2 == 0 ? v[0] : cmul(v[k2], w);
   }
   __syncthreads();
 #pragma unroll
@@ -260,7 +234,7 @@ __device__ __forceinline__ void fft2_fwd(float2* v, float2* __restrict__ lds, co
     const int k2 = t + R1 * i;
     float2 u[R1];
 #pragma unroll
-    for (int n1 = 0; n1 < R1; ++n1) u[n1] = lds[lidx<LAY, R1>(k2, n1, s, P)];
+    for (int n1 = 0; n1 < R1; ++n1) u[n1] = lds[lidx<R1>(k2, n1, s, P)];
     dft_reg<R1, DIR>(u);
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) v[i * R1 + k1] = u[k1];
@@ -269,7 +243,7 @@ __device__ __forceinline__ void fft2_fwd(float2* v, float2* __restrict__ lds, co
 
 // inverse of the forward distribution: v[i R1 + k1] = Y[(t + R1 i) + R2 k1] in
 // (owned groups), v[n2] = y[t + R1 n2] out (direction DIR, normally -1)
-template <int R1, int R2, int DIR, int LAY = 0>
+template <int R1, int R2, int DIR>
 __device__ __forceinline__ void fft2_inv(float2* v, float2* __restrict__ lds, const float2* __restrict__ twL, int t,
                                          int s, int P) {
 #pragma unroll
@@ -284,12 +258,12 @@ __device__ __forceinline__ void fft2_inv(float2* v, float2* __restrict__ lds, co
     for (int n1 = 0; n1 < R1; ++n1) {
       float2 w = twL[n1 * k2];
       if (DIR < 0) w.y = -w.y;
-      lds[lidx<LAY, R1>(k2, n1, s, P)] = n1 == 0 ? u[0] : cmul(u[n1], w);
+      lds[lidx<R1>(k2, n1, s, P)] = n1 == 0 ? u[0] : cmul(u[n1], w);
     }
   }
   __syncthreads();
 #pragma unroll
-  for (int k2 = 0; k2 < R2; ++k2) v[k2] = lds[lidx<LAY, R1>(k2, t, s, P)];
+  for (int k2 = 0; k2 < R2; ++k2) v[k2] = lds[lidx<R1>(k2, t, s, P)];
   dft_reg<R2, DIR>(v);
 }
 
@@ -297,7 +271,7 @@ __device__ __forceinline__ void fft2_inv(float2* v, float2* __restrict__ lds, co
 // LDS in turn, so the exchange buffer holds L*P floats instead of L*P
 // float2.  Half the LDS per workgroup doubles the workgroups a CU can hold
 // for kernels whose occupancy LDS limits (pass 1); two more barriers.
-template <int R1, int R2, int DIR, int LAY = 0>
+template <int R1, int R2, int DIR>
 __device__ __forceinline__ void fft2_fwd_s(float2* v, float* __restrict__ lds, const float2* __restrict__ twL, int t,
                                            int s, int P) {
   constexpr int G = Reg2<R1, R2>::G;
@@ -310,24 +284,24 @@ __device__ __forceinline__ void fft2_fwd_s(float2* v, float* __restrict__ lds, c
   }
   float re[G * R1];
 #pragma unroll
-  for (int k2 = 0; k2 < R2; ++k2) lds[lidx<LAY, R1>(k2, t, s, P)] = v[k2].x;
+  for (int k2 = 0; k2 < R2; ++k2) lds[lidx<R1>(k2, t, s, P)] = v[k2].x;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < G; ++i) {
     if (!reg2_owns<R1, R2>(t, i)) continue;
 #pragma unroll
-    for (int n1 = 0; n1 < R1; ++n1) re[i * R1 + n1] = lds[lidx<LAY, R1>(t + R1 * i, n1, s, P)];
+    for (int n1 = 0; n1 < R1; ++n1) re[i * R1 + n1] = lds[lidx<R1>(t + R1 * i, n1, s, P)];
   }
   __syncthreads();
 #pragma unroll
-  for (int k2 = 0; k2 < R2; ++k2) lds[lidx<LAY, R1>(k2, t, s, P)] = v[k2].y;
+  for (int k2 = 0; k2 < R2; ++k2) lds[lidx<R1>(k2, t, s, P)] = v[k2].y;
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < G; ++i) {
     if (!reg2_owns<R1, R2>(t, i)) continue;
     float2 u[R1];
 #pragma unroll
-    for (int n1 = 0; n1 < R1; ++n1) u[n1] = make_float2(re[i * R1 + n1], lds[lidx<LAY, R1>(t + R1 * i, n1, s, P)]);
+    for (int n1 = 0; n1 < R1; ++n1) u[n1] = make_float2(re[i * R1 + n1], lds[lidx<R1>(t + R1 * i, n1, s, P)]);
     dft_reg<R1, DIR>(u);
 #pragma unroll
     for (int k1 = 0; k1 < R1; ++k1) v[i * R1 + k1] = u[k1];
@@ -335,7 +309,7 @@ __device__ __forceinline__ void fft2_fwd_s(float2* v, float* __restrict__ lds, c
 }
 
 // Split-exchange form of fft2_inv (real and imaginary parts cross LDS in turn).
-template <int R1, int R2, int DIR, int LAY = 0>
+template <int R1, int R2, int DIR>
 __device__ __forceinline__ void fft2_inv_s(float2* v, float* __restrict__ lds, const float2* __restrict__ twL, int t,
                                            int s, int P) {
   constexpr int G = Reg2<R1, R2>::G;
@@ -358,22 +332,22 @@ __device__ __forceinline__ void fft2_inv_s(float2* v, float* __restrict__ lds, c
   for (int i = 0; i < G; ++i) {
     if (!reg2_owns<R1, R2>(t, i)) continue;
 #pragma unroll
-    for (int n1 = 0; n1 < R1; ++n1) lds[lidx<LAY, R1>(t + R1 * i, n1, s, P)] = v[i * R1 + n1].x;
+    for (int n1 = 0; n1 < R1; ++n1) lds[lidx<R1>(t + R1 * i, n1, s, P)] = v[i * R1 + n1].x;
   }
   __syncthreads();
   float re[R2];
 #pragma unroll
-  for (int k2 = 0; k2 < R2; ++k2) re[k2] = lds[lidx<LAY, R1>(k2, t, s, P)];
+  for (int k2 = 0; k2 < R2; ++k2) re[k2] = lds[lidx<R1>(k2, t, s, P)];
   __syncthreads();
 #pragma unroll
   for (int i = 0; i < G; ++i) {
     if (!reg2_owns<R1, R2>(t, i)) continue;
 #pragma unroll
-    for (int n1 = 0; n1 < R1; ++n1) lds[lidx<LAY, R1>(t + R1 * i, n1, s, P)] = v[i * R1 + n1].y;
+    for (int n1 = 0; n1 < R1; ++n1) lds[lidx<R1>(t + R1 * i, n1, s, P)] = v[i * R1 + n1].y;
   }
   __syncthreads();
 #pragma unroll
-  for (int k2 = 0; k2 < R2; ++k2) v[k2] = make_float2(re[k2], lds[lidx<LAY, R1>(k2, t, s, P)]);
+  for (int k2 = 0; k2 < R2; ++k2) v[k2] = make_float2(re[k2], lds[lidx<R1>(k2, t, s, P)]);
   dft_reg<R2, DIR>(v);
 }
 
@@ -391,273 +365,6 @@ __device__ __forceinline__ float2 dft_m_out(const float2* z, int m) {
 #pragma unroll
   for (int q = 1; q < M; ++q) r = cadd(r, cmul(root_m<M, DIR>((q * m) % M), z[q]));
   return r;
-}
-
-// ---- lane-pair split DFTs: a Q-point DFT (Q even) held by two adjacent
-// lanes (h = lane & 1), Q/2 values each; one radix-2 step crosses the pair
-// through a lane shuffle.
-// DIT form: a[j] = x[h + 2j] in, a[j] = X[(Q/2) h + j] out.
-template <int Q, int DIR>
-__device__ __forceinline__ void dit_pair(float2* a, int h) {
-  constexpr int H = Q / 2;
-  dft_reg<H, DIR>(a);
-  const float sg = h ? -1.f : 1.f;
-#pragma unroll
-  for (int m = 0; m < H; ++m) {
-    const float2 tw = twc<Q, DIR>(a[m], m);
-    const float2 z = h ? tw : a[m];  // lane 0: Y0[m], lane 1: w^m Y1[m]
-    const float2 b = make_float2(__shfl_xor(z.x, 1), __shfl_xor(z.y, 1));
-    a[m] = make_float2(b.x + sg * z.x, b.y + sg * z.y);  // Y0 + w Y1 | Y0 - w Y1
-  }
-}
-// DIF form: a[j] = x[(Q/2) h + j] in, a[j] = X[h + 2j] out.
-template <int Q, int DIR>
-__device__ __forceinline__ void dif_pair(float2* a, int h) {
-  constexpr int H = Q / 2;
-#pragma unroll
-  for (int j = 0; j < H; ++j) {
-    const float2 b = make_float2(__shfl_xor(a[j].x, 1), __shfl_xor(a[j].y, 1));
-    const float2 sum = make_float2(a[j].x + b.x, a[j].y + b.y);         // lane 0: x[j] + x[j+H]
-    const float2 dif = twc<Q, DIR>(make_float2(b.x - a[j].x, b.y - a[j].y), j);  // lane 1: (x[j] - x[j+H]) w^j
-    a[j] = h ? dif : sum;
-  }
-  dft_reg<H, DIR>(a);
-}
-
-// LDS index for the lane-pair transform of L = Q^2 points over C columns:
-// element (k2, n1) of column s; the two halves of k2 sit side by side in a
-// padded row of P2 slots so that a lane pair (h = 0, 1) hits disjoint banks.
-template <int Q>
-__device__ __forceinline__ int pidx(int k2, int n1, int s, int C, int P2) {
-  constexpr int H = Q / 2;
-  return ((k2 % H) * Q + n1) * P2 + (k2 / H) * C + s;
-}
-__host__ __device__ constexpr int pair_stride(int C) {
-  int p = (2 * C + 15) / 16 * 16;
-  if ((p / 16) % 2 == 0) p += 16;
-  return p;
-}
-
-// forward two-level transform with lane pairs (virtual thread t of Q per
-// column, lane half h): v[j] = x[t + Q (h + 2j)] in,
-// v[j] = X[t + Q ((Q/2) h + j)] out
-template <int Q, int DIR>
-__device__ __forceinline__ void fft2p_fwd(float2* v, float2* __restrict__ lds, const float2* __restrict__ twL, int t,
-                                          int h, int s, int C, int P2) {
-  constexpr int H = Q / 2;
-  dit_pair<Q, DIR>(v, h);
-#pragma unroll
-  for (int j = 0; j < H; ++j) {
-    const int k2 = H * h + j;
-    float2 w = twL[t * k2];
-    if (DIR < 0) w.y = -w.y;
-    lds[pidx<Q>(k2, t, s, C, P2)] = cmul(v[j], w);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < H; ++j) v[j] = lds[pidx<Q>(t, h + 2 * j, s, C, P2)];
-  dit_pair<Q, DIR>(v, h);
-}
-
-// inverse of fft2p_fwd's distribution: v[j] = Y[t + Q ((Q/2) h + j)] in,
-// v[j] = y[t + Q (h + 2j)] out
-template <int Q, int DIR>
-__device__ __forceinline__ void fft2p_inv(float2* v, float2* __restrict__ lds, const float2* __restrict__ twL, int t,
-                                          int h, int s, int C, int P2) {
-  constexpr int H = Q / 2;
-  dif_pair<Q, DIR>(v, h);
-#pragma unroll
-  for (int j = 0; j < H; ++j) {
-    const int n1 = h + 2 * j;
-    float2 w = twL[n1 * t];
-    if (DIR < 0) w.y = -w.y;
-    lds[pidx<Q>(t, n1, s, C, P2)] = cmul(v[j], w);
-  }
-  __syncthreads();
-#pragma unroll
-  for (int j = 0; j < H; ++j) v[j] = lds[pidx<Q>(H * h + j, t, s, C, P2)];
-  dif_pair<Q, DIR>(v, h);
-}
-
-// ---- register Stockham stages
-// A length L = R0 R1 R2 R3 transform (R3 = 1: three stages) held by T = L / V
-// threads per sequence, V values per thread.  Forward stage s of radix R and
-// span P = R0 ... R_{s-1}: butterfly i = j + T b (b < V / R) of thread j
-// gathers u_r = d[i + r L / R] (r < R), multiplies u_r by w_{PR}^{r (i mod P)},
-// does the R-point DFT and scatters y_r to (i - i mod P) R + i mod P + r P.
-// After the last stage d is the transform in natural order (self-sorting
-// Stockham).  Stage 0 gathers from registers the caller loaded, the stages
-// between exchange through LDS, and the last stage's outputs stay in
-// registers: thread j ends with X[i + r L / R_last] at v[b R_last + r].  The
-// inverse runs the transposed stages in reverse order (gather from the
-// scatter positions, conjugate DFT, conjugate twiddle, scatter to the gather
-// positions) and leaves y where stage 0 gathered from.  Half the registers
-// of the two-level form for the same length, one more LDS exchange.
-constexpr int sk_rad(int s, int r0, int r1, int r2, int r3) { return s == 0 ? r0 : s == 1 ? r1 : s == 2 ? r2 : r3; }
-template <int V_, int R0, int R1, int R2, int R3 = 1>
-struct SkPlan {
-  static constexpr int V = V_, L = R0 * R1 * R2 * R3, T = L / V, S = R3 > 1 ? 4 : 3;
-  static constexpr int rad(int s) { return sk_rad(s, R0, R1, R2, R3); }
-  static constexpr int span(int s) { return s == 0 ? 1 : span(s - 1) * rad(s - 1); }
-  // LDS swizzle shift: stage 0 scatters with stride R0
-  static constexpr int SH = R0 == 8 ? 3 : 2;
-  static_assert(V % R0 == 0 && V % R1 == 0 && V % R2 == 0 && V % R3 == 0, "every radix divides V");
-  static_assert(R0 % 2 == 0, "even first radix: the zero half of a padded input is a compile-time set");
-  static_assert(L % 32 == 0, "the LDS swizzle permutes within 32-point blocks");
-};
-// LDS slot of point idx of sequence col: C sequences interleaved, the point
-// index XOR-swizzled within 32-point blocks so that the stride-R0 scatter of
-// stage 0 and the unit-stride gathers of a wave both hit distinct banks.
-template <int C, int SH>
-__device__ __forceinline__ int sk_lds(int idx, int col) {
-  constexpr int M = C >= 32 ? 0 : 32 / C - 1;
-  return C * (idx ^ ((idx >> SH) & M)) + col;
-}
-template <class PL, int s>
-__device__ __forceinline__ int sk_scatter(int i, int r) {
-  constexpr int R = PL::rad(s), P = PL::span(s);
-  const int k = i % P;
-  return (i - k) * R + k + r * P;
-}
-template <class PL, int s>
-__device__ __forceinline__ int sk_gather(int i, int r) {
-  return i + r * (PL::L / PL::rad(s));
-}
-// stage-s twiddles and DFTs of thread j's butterflies (forward order: twiddle, DFT)
-template <class PL, int s, int DIR>
-__device__ __forceinline__ void sk_fwd_bfly(float2* v, const float2* __restrict__ twL, int j) {
-  constexpr int R = PL::rad(s), P = PL::span(s), NB = PL::V / R, TS = PL::L / (P * R);
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    if constexpr (P > 1) {
-      const int k = (j + PL::T * b) % P;
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        float2 w = twL[r * k * TS];
-        if (DIR < 0) w.y = -w.y;
-        v[b * R + r] = cmul(v[b * R + r], w);
-      }
-    }
-    dft_reg<R, DIR>(v + b * R);
-  }
-}
-// transposed stage s (DFT, then twiddle; DIR is the inverse's sign)
-template <class PL, int s, int DIR>
-__device__ __forceinline__ void sk_inv_bfly(float2* v, const float2* __restrict__ twL, int j) {
-  constexpr int R = PL::rad(s), P = PL::span(s), NB = PL::V / R, TS = PL::L / (P * R);
-#pragma unroll
-  for (int b = 0; b < NB; ++b) {
-    dft_reg<R, DIR>(v + b * R);
-    if constexpr (P > 1) {
-      const int k = (j + PL::T * b) % P;
-#pragma unroll
-      for (int r = 1; r < R; ++r) {
-        float2 w = twL[r * k * TS];
-        if (DIR < 0) w.y = -w.y;
-        v[b * R + r] = cmul(v[b * R + r], w);
-      }
-    }
-  }
-}
-// LDS exchange buffer of an exchange (K sequences of L points per column,
-// K L C slots): with NBUF = 2 consecutive exchanges alternate between two
-// buffers, so a write needs no barrier of its own (every thread passed the
-// previous exchange's barrier after its reads of the buffer it now
-// overwrites).
-// RC: the stage functions recompute the exchange addresses from fresh
-// copies of the thread indices at every exchange instead of letting the
-// compiler keep them live across transforms (fewer registers, more VALU).
-template <class PL, int C, int NBUF, int K, bool RC = false>
-struct SkLds {
-  float2* xb;
-  int e = 0;
-  __device__ __forceinline__ float2* next() {
-    if (NBUF == 1) {
-      __syncthreads();
-      return xb;
-    }
-    float2* b = xb + (e & 1) * (K * PL::L * C);
-    ++e;
-    return b;
-  }
-};
-// K sequences advance stage by stage together (v[q V .. q V + V) is
-// sequence q), so one barrier serves all K and a stage's twiddles are
-// read once for the K.
-// forward stages s .. S-1 (stage s-1's butterflies done, its outputs in v)
-template <class PL, int s, int C, int NBUF, int K, int DIR, bool RC>
-__device__ __forceinline__ void sk_fwd_from(float2* v, SkLds<PL, C, NBUF, K, RC>& lx, const float2* __restrict__ twL,
-                                            int j, int col) {
-  if constexpr (s < PL::S) {
-    constexpr int V = PL::V, LC = PL::L * C;
-    constexpr int Rp = PL::rad(s - 1), NBp = V / Rp, R = PL::rad(s), NB = V / R;
-    float2* xb = lx.next();
-    // fresh copies of the thread indices: the exchange addresses are then
-    // recomputed here instead of kept live from an earlier transform
-    if constexpr (RC) asm volatile("" : "+v"(j), "+v"(col));
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-#pragma unroll
-      for (int b = 0; b < NBp; ++b)
-#pragma unroll
-        for (int r = 0; r < Rp; ++r)
-          xb[q * LC + sk_lds<C, PL::SH>(sk_scatter<PL, s - 1>(j + PL::T * b, r), col)] = v[q * V + b * Rp + r];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          v[q * V + b * R + r] = xb[q * LC + sk_lds<C, PL::SH>(sk_gather<PL, s>(j + PL::T * b, r), col)];
-#pragma unroll
-    for (int q = 0; q < K; ++q) sk_fwd_bfly<PL, s, DIR>(v + q * V, twL, j);
-    sk_fwd_from<PL, s + 1, C, NBUF, K, DIR>(v, lx, twL, j, col);
-  }
-}
-// whole forward transform of K sequences: stage-0 gathers in, last stage's outputs out
-template <class PL, int C, int NBUF, int K, int DIR, bool RC>
-__device__ __forceinline__ void sk_forward(float2* v, SkLds<PL, C, NBUF, K, RC>& lx, const float2* __restrict__ twL, int j,
-                                           int col) {
-#pragma unroll
-  for (int q = 0; q < K; ++q) sk_fwd_bfly<PL, 0, DIR>(v + q * PL::V, twL, j);
-  sk_fwd_from<PL, 1, C, NBUF, K, DIR>(v, lx, twL, j, col);
-}
-// transposed stages s .. 0 (v holds stage s's scatter positions)
-template <class PL, int s, int C, int NBUF, int K, int DIR, bool RC>
-__device__ __forceinline__ void sk_inv_from(float2* v, SkLds<PL, C, NBUF, K, RC>& lx, const float2* __restrict__ twL,
-                                            int j, int col) {
-  constexpr int V = PL::V, LC = PL::L * C;
-#pragma unroll
-  for (int q = 0; q < K; ++q) sk_inv_bfly<PL, s, DIR>(v + q * V, twL, j);
-  if constexpr (s > 0) {
-    constexpr int R = PL::rad(s), NB = V / R, Rn = PL::rad(s - 1), NBn = V / Rn;
-    float2* xb = lx.next();
-    if constexpr (RC) asm volatile("" : "+v"(j), "+v"(col));
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-#pragma unroll
-      for (int b = 0; b < NB; ++b)
-#pragma unroll
-        for (int r = 0; r < R; ++r)
-          xb[q * LC + sk_lds<C, PL::SH>(sk_gather<PL, s>(j + PL::T * b, r), col)] = v[q * V + b * R + r];
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < K; ++q)
-#pragma unroll
-      for (int b = 0; b < NBn; ++b)
-#pragma unroll
-        for (int r = 0; r < Rn; ++r)
-          v[q * V + b * Rn + r] = xb[q * LC + sk_lds<C, PL::SH>(sk_scatter<PL, s - 1>(j + PL::T * b, r), col)];
-    sk_inv_from<PL, s - 1, C, NBUF, K, DIR>(v, lx, twL, j, col);
-  }
-}
-// whole inverse transform of K sequences: the forward's output distribution
-// in, stage-0 gather positions out
-template <class PL, int C, int NBUF, int K, int DIR, bool RC>
-__device__ __forceinline__ void sk_inverse(float2* v, SkLds<PL, C, NBUF, K, RC>& lx, const float2* __restrict__ twL, int j,
-                                           int col) {
-  sk_inv_from<PL, PL::S - 1, C, NBUF, K, DIR>(v, lx, twL, j, col);
 }
 
 }  // namespace ddhip

@@ -82,12 +82,12 @@ __global__ __launch_bounds__(MV_THREADS) void k_pass1_xfwd(
 }
 
 // ------------------------------------------------------------- pass 2, 4 --
-// in [3][gx][ins: nin][nzp] -> out [3][gx][outs: nout][nzp], FFT along the middle axis of
-// plane kx, tiles of cy consecutive z.
+// a1 [3][gx][p1: ny][nzp] <-> a2 [3][2H][p2: gy][nzp], FFT along the middle axis of
+// a plane, tiles of cy consecutive z.
 template <int DIR, int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass_y(
     const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ twg,
-    FftPlan p, int gx, int nin, int nout, int nz, int nzp, int ins,
+    FftPlan p, KxSlab sl, int nin, int nout, int nz, int nzp, int ins,
     int outs, int cy_log2, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z / 3;
@@ -98,10 +98,11 @@ __global__ __launch_bounds__(NT) void k_pass_y(
   const int cy = 1 << cy_log2;
   float2* tw = sm;
   float2* buf = sm + L;
-  const int c = blockIdx.z % 3, kx = blockIdx.y, z0 = blockIdx.x * cy;
+  const int c = blockIdx.z % 3, slot = blockIdx.y, z0 = blockIdx.x * cy;
   const int T = blockDim.x;
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  const float2* src = in + ((size_t)c * gx + kx) * ins;
+  const size_t pl1 = (size_t)c * sl.gx + sl.kx(slot), pl2 = (size_t)c * (2 * sl.H) + slot;
+  const float2* src = in + (DIR > 0 ? pl1 : pl2) * ins;
   for (int idx = threadIdx.x; idx < L * cy; idx += T) {
     const int e = idx >> cy_log2, col = idx & (cy - 1);
     const int iz = z0 + col;
@@ -111,7 +112,7 @@ __global__ __launch_bounds__(NT) void k_pass_y(
   }
   __syncthreads();
   fft_run<DIR, true, PER>(buf, tw, p, cy, cy, 1);
-  float2* dst = out + ((size_t)c * gx + kx) * outs;
+  float2* dst = out + (DIR > 0 ? pl2 : pl1) * outs;
   for (int idx = threadIdx.x; idx < nout * cy; idx += T) {
     const int e = idx >> cy_log2, col = idx & (cy - 1);
     const int iz = z0 + col;
@@ -120,11 +121,11 @@ __global__ __launch_bounds__(NT) void k_pass_y(
 }
 
 // ---------------------------------------------------------------- pass 3 --
-// cz contiguous z columns (kx 2NY + ky) per workgroup, each at stride L + 1 in LDS
+// cz contiguous z columns (slot 2NY + ky) per workgroup, each at stride L + 1 in LDS
 template <int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass3_z_green(
     float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg,
-    FftPlan p, int nz, int nzp, int p2, int gx, int gy, int cz, BatchArgs ba, GreenGeo gg) {
+    FftPlan p, int nz, int nzp, int p2, KxSlab sl, int gy, int cz, BatchArgs ba, GreenGeo gg) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z;
   if (ba.active && !ba.active[rb]) return;
@@ -134,12 +135,12 @@ __global__ __launch_bounds__(NT) void k_pass3_z_green(
   float2* b0 = sm + L;
   float2* b1 = b0 + LP * cz;
   float2* b2 = b1 + LP * cz;
-  const int ncol = gx * gy, q0 = blockIdx.x * cz, nc = min(cz, ncol - q0);
+  const int ncol = 2 * sl.H * gy, q0 = blockIdx.x * cz, nc = min(cz, ncol - q0);
   const int T = blockDim.x;
-  const size_t cstride = (size_t)gx * p2;
+  const size_t cstride = (size_t)(2 * sl.H) * p2;
   const auto column = [&](int r) {
-    const int kx = (q0 + r) / gy;
-    return (size_t)kx * p2 + (size_t)(q0 + r - kx * gy) * nzp;
+    const int slot = (q0 + r) / gy;
+    return (size_t)slot * p2 + (size_t)(q0 + r - slot * gy) * nzp;
   };
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
   for (int idx = threadIdx.x; idx < L * cz; idx += T) {
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(NT) void k_pass3_z_green(
   // (cu:109-115), whole grid for IPBC=1
   for (int idx = threadIdx.x; idx < L * nc; idx += T) {
     const int r = idx / L, kz = idx - r * L;
-    const int kx = (q0 + r) / gy, ky = q0 + r - kx * gy;
+    const int slot = (q0 + r) / gy, kx = sl.kx(slot), ky = q0 + r - slot * gy;
     const int ir = min(kx, gg.mx - kx), jr = min(ky, gg.my - ky), kr = min(kz, gg.mz - kz);
     const float sx = kx <= gg.tx ? 1.f : -1.f, sy = ky <= gg.ty ? 1.f : -1.f;
     const float sz = kz <= gg.tz ? 1.f : -1.f;
@@ -335,19 +336,19 @@ static int allow_big_lds(size_t bytes) {
   return 0;
 }
 
-int matvec_setup(Context& c) {
+int matvec_plan(Context& c, const char* name) {
   MatvecPlan& m = c.mv;
   m = MatvecPlan{};
   m.nx = c.nx; m.ny = c.ny; m.nz = c.nz; m.nat = c.nat; m.nat0 = c.nat0;
   m.gx = 2 * c.nx; m.gy = 2 * c.ny; m.gz = 2 * c.nz;
   m.ngrid = (size_t)m.gx * m.gy * m.gz;
   if (!fft_make_plan(m.gx, m.px) || !fft_make_plan(m.gy, m.py) || !fft_make_plan(m.gz, m.pz)) {
-    set_error("MATVEC plan", "2*NX, 2*NY, 2*NZ must factor into 2, 3, 5 and 7");
+    set_error(name, "2*NX, 2*NY, 2*NZ must factor into 2, 3, 5 and 7");
     return 206;
   }
   const int wide = PER_WIDE * MV_THREADS, narrow = PER_NARROW * MV_THREADS;
   if (m.gx > wide || m.gy > wide || m.gz > narrow / 1 || m.gx > narrow) {
-    set_error("MATVEC plan", "padded grid axis exceeds the LDS FFT limit (2N <= 2048)");
+    set_error(name, "padded grid axis exceeds the LDS FFT limit (2N <= 2048)");
     return 206;
   }
   const int nrows = c.ny * c.nz;
@@ -379,6 +380,11 @@ int matvec_setup(Context& c) {
   const auto odd_blocks = [](int n) { return ((n + 31) / 32 | 1) * 32; };
   m.p1 = odd_blocks(c.ny * m.nzp);
   m.p2 = odd_blocks(m.gy * m.nzp);
+  return 0;
+}
+
+int matvec_setup(Context& c) {
+  if (int rc = matvec_plan(c, "MATVEC plan")) return rc;
   DDH_TRY(hipMalloc((void**)&c.a1, matvec_a1_count(c) * sizeof(float2)), "malloc FFT work a1", 204);
   DDH_TRY(hipMalloc((void**)&c.a2, matvec_a2_count(c) * sizeof(float2)), "malloc FFT work a2", 204);
   return 0;
@@ -415,33 +421,33 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
     case 2:
     case 4: {
       const bool fwd = which == 2;
-      dim3 grid((c.nz + m.cy - 1) / m.cy, m.gx, 3 * nb);
+      dim3 grid((c.nz + m.cy - 1) / m.cy, 2 * bt.slab.H, 3 * nb);
       const size_t lds = (size_t)(m.gy + m.cy * m.gy) * sizeof(float2);
       const int lg = ilog2(m.cy), ins = fwd ? m.p1 : m.p2, outs = fwd ? m.p2 : m.p1;
       if (fwd && m.ty == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a1, a2, m.twy,
-                           m.py, m.gx, c.ny, m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
+                           m.py, bt.slab, c.ny, m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
       else if (fwd)
-        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a1, a2, m.twy, m.py, m.gx, c.ny,
+        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a1, a2, m.twy, m.py, bt.slab, c.ny,
                            m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
       else if (m.ty == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2, a1, m.twy,
-                           m.py, m.gx, m.gy, c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
+                           m.py, bt.slab, m.gy, c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
       else
-        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a2, a1, m.twy, m.py, m.gx, m.gy,
+        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a2, a1, m.twy, m.py, bt.slab, m.gy,
                            c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
       DDH_LAUNCH_OK("MATVEC y FFT", fwd ? 22 : 24);
       break;
     }
     case 3: {
-      dim3 grid((m.gx * m.gy + m.cz - 1) / m.cz, 1, nb);
+      dim3 grid((2 * bt.slab.H * m.gy + m.cz - 1) / m.cz, 1, nb);
       const size_t lds = (size_t)(m.gz + 3 * m.cz * (m.gz + (m.cz > 1))) * sizeof(float2);
       if (m.tz == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass3_z_green<PER_NARROW, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2,
-                           c.green, m.twz, m.pz, c.nz, m.nzp, m.p2, m.gx, m.gy, m.cz, bt.k, green_geo(c));
+                           c.green, m.twz, m.pz, c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, bt.k, green_geo(c));
       else
         hipLaunchKernelGGL(k_pass3_z_green<PER_NARROW>, grid, dim3(MV_THREADS), lds, st, a2, c.green, m.twz, m.pz,
-                           c.nz, m.nzp, m.p2, m.gx, m.gy, m.cz, bt.k, green_geo(c));
+                           c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, bt.k, green_geo(c));
       DDH_LAUNCH_OK("MATVEC pass 3 (z FFT + Green)", 23);
       break;
     }
@@ -466,6 +472,7 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   MvBatch bt = btp ? *btp : MvBatch{};
   if (!bt.a1) bt.a1 = c.a1;
   if (!bt.a2) bt.a2 = c.a2;
+  bt.slab = KxSlab{0, c.nx, c.mv.gx};
   for (int p = 1; p <= 5; ++p) {
     if (ev) hipEventRecord(ev[p - 1], st);
     if (int rc = launch_pass(c, p, c.mv.kind[p], cj, compact, x, y, adia, aoff, st, bt)) return rc;
@@ -474,6 +481,17 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   if (ev) hipEventRecord(ev[5], st);
   c.matvec_count += (unsigned)bt.nrhs;
   return 0;
+}
+
+int matvec_slab(Context& c, hipStream_t st, const MvBatch& bt) {
+  for (int p = 2; p <= 4; ++p)
+    if (int rc = launch_pass(c, p, c.mv.kind[p], 0, 0, nullptr, nullptr, nullptr, nullptr, st, bt)) return rc;
+  return 0;
+}
+
+int matvec_end_pass(Context& c, int which, int cwhat, const float2* x, float2* y, const float2* adia,
+                    const float2* aoff, int layout, hipStream_t st, const MvBatch& bt) {
+  return launch_pass(c, which, c.mv.kind[which], cwhat == 'C' ? 1 : 0, layout ? 1 : 0, x, y, adia, aoff, st, bt);
 }
 
 // Autotuner: a pass whose axis length has several register shapes runs each a
@@ -519,6 +537,8 @@ int matvec_autotune(Context& c) {
   MvBatch bt;
   bt.a1 = c.a1;
   bt.a2 = c.a2;
+  bt.slab = KxSlab{0, c.nx, m.gx};
+  if (c.backend == BACKEND_SLICES) slices_slab(c, 0, bt);
   int rc = 0;
   for (int p = 1; p <= 5 && !rc; ++p) {
     const int ncand = reg_candidates(lens[p], p);

@@ -31,46 +31,48 @@ constexpr int P3_WAVES = 4;  // waves per workgroup (1 to 8 measured within 4 %)
 // for the others.
 //  aligned: blocks of `per` consecutive ky of one kx, in groups of four
 //           mirrors (+-kx, block b and nkb - 1 - b);
-//  flat:    blocks of `per` consecutive columns kx 2NY + ky of the half
-//           kx < NX, in groups of two (+-kx); taken where 2NY leaves more
+//  flat:    blocks of `per` consecutive columns slot 2NY + ky of the half
+//           slot < H, in groups of two (+-kx); taken where 2NY leaves more
 //           than an eighth of an aligned block's lanes idle.
 struct P3Cols {
+  KxSlab sl;  // the planes of a2
   int per;    // columns per workgroup
   int flat;
   int nkb;    // aligned: ky blocks per kx; flat: blocks per half
   int groups; // groups of mirrors
   int nrhs;
 };
-inline P3Cols p3_cols(int gx, int gy, int per, int nrhs) {
+inline P3Cols p3_cols(const KxSlab& sl, int gy, int per, int nrhs) {
   P3Cols q;
+  q.sl = sl;
   q.per = per;
   q.nrhs = nrhs;
   const int nkb = (gy + per - 1) / per;
   q.flat = (long long)8 * nkb * per > (long long)9 * gy;
   if (q.flat) {
-    q.nkb = (int)(((long long)(gx / 2) * gy + per - 1) / per);
+    q.nkb = (int)(((long long)sl.H * gy + per - 1) / per);
     q.groups = q.nkb;
   } else {
     q.nkb = nkb;
-    q.groups = (gx / 2) * ((nkb + 1) / 2);
+    q.groups = sl.H * ((nkb + 1) / 2);
   }
   return q;
 }
 inline unsigned p3_blocks(const P3Cols& q) { return (unsigned)((q.groups + 7) / 8 * 8 * (q.flat ? 2 : 4) * q.nrhs); }
-// right-hand side of this workgroup and (kx, ky) of its column `col`; ky < 0 past the end
-__device__ __forceinline__ void p3_column(const P3Cols& q, int col, int gx, int gy, int& rb, int& kx, int& ky) {
+// right-hand side of this workgroup and (plane slot, ky) of its column `col`; ky < 0 past the end
+__device__ __forceinline__ void p3_column(const P3Cols& q, int col, int gy, int& rb, int& ps, int& ky) {
   const int x8 = (int)blockIdx.x & 7, sq = (int)blockIdx.x >> 3, nm = q.flat ? 2 : 4;
   const int sp = sq / q.nrhs;
   rb = sq - sp * q.nrhs;
   const int g = sp / nm, slot = sp - g * nm, grp = g * 8 + x8;
   ky = -1;
-  kx = 0;
+  ps = 0;
   if (grp >= q.groups) return;
   int half;
   if (q.flat) {
     const int hc = grp * q.per + col;
     half = hc / gy;
-    if (half >= gx / 2) return;
+    if (half >= q.sl.H) return;
     ky = hc - half * gy;
   } else {
     const int hb = (q.nkb + 1) / 2;
@@ -81,7 +83,7 @@ __device__ __forceinline__ void p3_column(const P3Cols& q, int col, int gx, int 
     if (ky >= gy) { ky = -1; return; }
   }
   const int mx = q.flat ? slot : slot >> 1;
-  kx = mx ? (half == 0 ? gx / 2 : gx - half) : half;
+  ps = half + mx * q.sl.H;
 }
 
 // Green points are loaded in groups of two (12 registers each; groups of one
@@ -98,7 +100,7 @@ constexpr int p3_waves_per_simd() {
 }
 template <class PL, bool MIRROR>
 __global__ __launch_bounds__(64 * P3_WAVES) __attribute__((amdgpu_waves_per_eu(p3_waves_per_simd<PL>()))) void kw_pass3(
-    float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg, int nz, int nzp, int p2, int gx, int gy,
+    float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg, int nz, int nzp, int p2, int gy,
     BatchArgs ba, GreenGeo gg, P3Cols q) {
   constexpr int L = PL::L, T = PL::T, V = PL::V, SEQ = PL::SEQ, R0 = PL::rad(0), SL = PL::S - 1, RL = PL::rad(SL);
   static_assert(R0 % 2 == 0, "the zero half of a padded column is a compile-time set");
@@ -108,15 +110,16 @@ __global__ __launch_bounds__(64 * P3_WAVES) __attribute__((amdgpu_waves_per_eu(p
   __syncthreads();
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, seq = lane / T, j = lane - seq * T;
   if (T * SEQ < 64 && seq >= SEQ) return;
-  int rb, kx, ky;
-  p3_column(q, w * SEQ + seq, gx, gy, rb, kx, ky);
+  int rb, ps, ky;
+  p3_column(q, w * SEQ + seq, gy, rb, ps, ky);
   if (ky < 0 || (ba.active && !ba.active[rb])) return;
+  const int kx = q.sl.kx(ps);
   float2* const xb = xbuf + (w * SEQ + seq) * PL::SLOTS;
   // workgroup-uniform base per component, 32-bit byte offsets per lane (the
   // launcher checks that a component and the Green array span < 4 GiB)
   char* const cb = reinterpret_cast<char*>(a2 + rb * ba.a2s);
-  const size_t csb = (size_t)gx * p2 * sizeof(float2);
-  const unsigned o0 = ((unsigned)kx * (unsigned)p2 + (unsigned)ky * (unsigned)nzp) * 8u;
+  const size_t csb = (size_t)(2 * q.sl.H) * p2 * sizeof(float2);
+  const unsigned o0 = ((unsigned)ps * (unsigned)p2 + (unsigned)ky * (unsigned)nzp) * 8u;
   // stage-0 inputs: v[c][b R0 + r] = x_c[j + T b + r L / R0], zero for r >= R0 / 2
   float2 v[3][V];
 #pragma unroll
@@ -193,9 +196,9 @@ __global__ __launch_bounds__(64 * P3_WAVES) __attribute__((amdgpu_waves_per_eu(p
 template <class PL>
 static void launch_kw_pass3(Context& c, const MvBatch& bt, hipStream_t st) {
   const MatvecPlan& m = c.mv;
-  const P3Cols q = p3_cols(m.gx, m.gy, P3_WAVES * PL::SEQ, bt.nrhs);
+  const P3Cols q = p3_cols(bt.slab, m.gy, P3_WAVES * PL::SEQ, bt.nrhs);
   const auto kernel = c.ipbc ? &kw_pass3<PL, false> : &kw_pass3<PL, true>;
-  hipLaunchKernelGGL(kernel, dim3(p3_blocks(q)), dim3(64 * P3_WAVES), 0, st, bt.a2, c.green, m.twz, c.nz, m.nzp, m.p2, m.gx, m.gy,
+  hipLaunchKernelGGL(kernel, dim3(p3_blocks(q)), dim3(64 * P3_WAVES), 0, st, bt.a2, c.green, m.twz, c.nz, m.nzp, m.p2, m.gy,
                      bt.k, green_geo(c), q);
 }
 struct P3Shape {

@@ -74,7 +74,6 @@ struct Context {
   // of (nx+1)(ny+1)(nz+1) points for IPBC=0, the whole grid of 2nx 2ny 2nz for IPBC=1
   float2* green = nullptr;
   size_t green_count = 0;
-  int green_zfast = 0;  // resident point order: 1 z fastest (FFT3D), 0 x fastest (SLICES)
   // FFT3D work: a1 [3][gx][p1: ny][nzp], a2 [3][gx][p2: gy][nzp]
   float2 *a1 = nullptr, *a2 = nullptr;
   // occupancy
@@ -120,16 +119,22 @@ void release_solver_workspace(Context& c);
 struct BatchArgs {
   size_t xs = 0, os = 0, a1s = 0, a2s = 0;
   const int* active = nullptr;
-  // SLICES z-forward input read straight from the MATVEC's x: element j of
-  // component c is gsrc[c gcs + gmap[j]] (compact; 0 where gmap[j] < 0) or
-  // gsrc[c gcs + j] (gmap == nullptr), conjugated when gconj
-  const float2* gsrc = nullptr;
-  const int* gmap = nullptr;
-  size_t gcs = 0;
-  int gconj = 0;
+};
+// The kx planes of a2: 2 H slots, slot s < H holding kx = h0 + s and slot H + s
+// its mirror 2NX - kx (the plane of the same Green entries; for kx = 0, which
+// is its own mirror, kx = NX).  H = NX is every plane (FFT3D); SLICES runs
+// passes 2 to 4 over slabs of a few H.
+struct KxSlab {
+  int h0 = 0, H = 0, gx = 0;
+  __host__ __device__ int kx(int slot) const {
+    if (slot < H) return h0 + slot;
+    const int h = h0 + slot - H;
+    return h == 0 ? gx / 2 : gx - h;
+  }
 };
 struct MvBatch {
   int nrhs = 1;
+  KxSlab slab;           // H = 0: every plane
   BatchArgs k;
   float2* a1 = nullptr;  // nullptr: the context's single-RHS buffers
   float2* a2 = nullptr;
@@ -151,22 +156,15 @@ int reg_candidates(int L, int which);
 // register-FFT pass `which` (1..5) with shape `cand` of its axis length; 1 = launched
 int reg_pass(Context& c, int which, int cand, int cj, int compact, const float2* x, float2* y, const float2* adia,
              const float2* aoff, hipStream_t st, const MvBatch& bt);
-// SLICES y-FFT + Green + inverse y-FFT of nb slice planes from kz = k0 with
-// the register kernels when 2NY has a register shape; 1 = launched.  act (all
-// SLICES launchers): the right-hand side's active flag in a batch, or nullptr.
-int slices_y_green_reg(Context& c, float2* sl, int k0, int nb, hipStream_t st, const int* act);
-// SLICES x-FFT (dir +1: zwork rows -> slice) or inverse x-FFT (dir -1:
-// slice -> zwork rows) of nb planes from kz = k0 with the register kernels
-// when 2NX has a register shape; 1 = launched
-int slices_x_reg(Context& c, int dir, float2* zw, float2* sl, int k0, int nb, hipStream_t st, const int* act);
-// SLICES z-FFT (dir +1: [3][NZ][NY][NX] -> zwork) or inverse z-FFT (dir -1:
-// zwork -> [3][NZ][NY][NX]) with the register column kernels when 2NZ has a
-// register shape; 1 = launched.  slices_z_reg_length: whether L has one.
-// gather (dir +1 only): `in` is the MATVEC's x, compact through the site map
-// when `compact`, conjugated when `cj`, read inside the z-FFT's loads.
-int slices_z_reg(Context& c, int dir, const float2* in, float2* out, hipStream_t st, const int* act,
-                 bool gather = false, int compact = 0, int cj = 0);
-int slices_z_reg_length(int L);
+// passes 2 to 4 on the planes bt.slab of a1, through the slab's planes in bt.a2
+int matvec_slab(Context& c, hipStream_t st, const MvBatch& bt);
+// SLICES: bt's slab and a2: the slab of planes from half-plane h0 and its buffer
+void slices_slab(const Context& c, int h0, MvBatch& bt);
+// pass 1 (x -> a1) or 5 (a1 -> y) alone
+int matvec_end_pass(Context& c, int which, int cwhat, const float2* x, float2* y, const float2* adia,
+                    const float2* aoff, int layout, hipStream_t st, const MvBatch& bt);
+// axis lengths, pitches and twiddles of c.mv
+int matvec_plan(Context& c, const char* name);
 // times every FFT kernel candidate of each pass and stores the fastest in c.mv.kind
 int matvec_autotune(Context& c);
 
@@ -187,9 +185,8 @@ double green_pbc_work(const Context& c, const GreenBuild& b);
 // The resident spectral Green tensor c.green is stored point-interleaved:
 // the six components (xx, xy, xz, yy, yz, zz) of octant point
 // (ir, jr, kr) sit at green[6p .. 6p+5], so a MATVEC reads them as three
-// 16-byte loads from one 48-byte run.  The axis that the backend's Green pass
-// transforms along a wave's lanes runs fastest: p = kr + (NZ+1)(jr + (NY+1) ir)
-// for FFT3D, p = ir + (NX+1)(jr + (NY+1) kr) for SLICES.  The reference layout
+// 16-byte loads from one 48-byte run.  The axis that the Green pass transforms
+// runs fastest: p = kr + (NZ+1)(jr + (NY+1) ir).  The reference layout
 // ([6][NZ+1][NY+1][NX+1], CXZC) is converted at the ABI edges.
 struct Green6 {
   float2 xx, xy, xz, yy, yz, zz;
@@ -206,7 +203,7 @@ __device__ __forceinline__ Green6 green_at(const float2* __restrict__ g, size_t 
 // flip sign with the mirrored axes' parities.  IPBC=1 stores the whole grid.
 // Both use the same instructions:
 //   r = min(k, m - k),  sign = (k <= t) ? +1 : -1,
-//   point = rz + oz (ry + oy rx) for FFT3D, rx + ox (ry + oy rz) for SLICES
+//   point = rz + oz (ry + oy rx)
 // octant: m = 2N, t = N, o = N+1; full grid: m = t = 2^30 (no mirror, all
 // signs +1), o = 2N.
 struct GreenGeo {
@@ -224,7 +221,7 @@ inline size_t green_points(int nx, int ny, int nz, int ipbc) {
   return ipbc ? (size_t)(2 * nx) * (2 * ny) * (2 * nz) : (size_t)(nx + 1) * (ny + 1) * (nz + 1);
 }
 
-// component-major [6][rz][ry][rx] (x fastest) <-> the backend's resident layout, device to device
+// component-major [6][rz][ry][rx] (x fastest) <-> the resident layout, device to device
 int green_interleave(Context& c, const float2* comp_major, float2* resident, hipStream_t st);
 int green_deinterleave(Context& c, const float2* resident, float2* comp_major, hipStream_t st);
 
