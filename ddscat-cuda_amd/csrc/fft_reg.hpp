@@ -146,6 +146,8 @@ __device__ __forceinline__ void dft_reg(float2* a) {
     dft3<DIR>(a);
   } else if constexpr (R == 5) {
     dft5<DIR>(a);
+  } else if constexpr (R == 7) {
+    dft7<DIR>(a);
   } else if constexpr (R == 16) {
     dft_comp<4, 4, DIR>(a);
   } else if constexpr (R == 32) {

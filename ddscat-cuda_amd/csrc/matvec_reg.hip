@@ -222,10 +222,11 @@ struct YShape {
   void (*fn)(Context&, int, const MvBatch&, hipStream_t);
 };
 #define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>}
-// One shape per padded length 2N, N = 2^a 3^b 5^c from 12 to 256 and a few
+// One shape per padded length 2N, N = 2^a 3^b 5^c 7^d from 12 to 256 and a few
 // above (two-level, R1 threads per column, at most 25 values each, C columns
 // per workgroup; 512 and 768 points by decimation, 20 and 30 % faster there).
-// Lengths with a factor 7 and those above 768 use the LDS-staged kernels.
+// Lengths of other sizes use the LDS-staged kernels (the y passes of a 70^3
+// grid: 34 us each against 14 to 16 here, 196^3: 470 against 213 to 235).
 static const YShape kYShapes[] = {
     Y_SHAPE(6, 4, 32), Y_SHAPE(6, 5, 32), Y_SHAPE(4, 8, 64), Y_SHAPE(6, 6, 32), Y_SHAPE(8, 5, 32), Y_SHAPE(8, 6, 32),
     Y_SHAPE(10, 5, 32), Y_SHAPE(9, 6, 32), Y_SHAPE(10, 6, 32), Y_SHAPE(8, 8, 32), Y_SHAPE(12, 6, 16),
@@ -237,6 +238,12 @@ static const YShape kYShapes[] = {
     Y_SHAPE(20, 20, 16), Y_SHAPE(24, 18, 16), Y_SHAPE(25, 18, 16), Y_SHAPE(24, 20, 16), Y_SHAPE(27, 18, 16),
     Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
     Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>},
+    // a factor 7
+    Y_SHAPE(7, 4, 32), Y_SHAPE(7, 6, 32), Y_SHAPE(8, 7, 32), Y_SHAPE(10, 7, 32), Y_SHAPE(12, 7, 16),
+    Y_SHAPE(14, 7, 16), Y_SHAPE(14, 8, 16), Y_SHAPE(14, 9, 16), Y_SHAPE(14, 10, 16), Y_SHAPE(14, 12, 16),
+    Y_SHAPE(14, 14, 32), Y_SHAPE(15, 14, 16), Y_SHAPE(16, 14, 16), Y_SHAPE(18, 14, 16), Y_SHAPE(20, 14, 16),
+    Y_SHAPE(21, 14, 16), Y_SHAPE(21, 16, 16), Y_SHAPE(25, 14, 16), Y_SHAPE(27, 14, 16), Y_SHAPE(28, 14, 16),
+    Y_SHAPE(30, 14, 16), Y_SHAPE(28, 16, 16), Y_SHAPE(35, 14, 8), Y_SHAPE(28, 18, 8),
 };
 
 // candidate `cand` of the table entries that `match`

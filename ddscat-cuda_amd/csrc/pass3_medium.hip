@@ -12,6 +12,10 @@ static const P3Shape kShapes[] = {
     P3_PLAN(18, 6, 3, 9), P3_PLAN(15, 12, 15), P3_PLAN(16, 16, 12), P3_PLAN(10, 20, 10), P3_PLAN(18, 18, 12),
     P3_PLAN(16, 16, 15), P3_PLAN(25, 10, 5, 5), P3_PLAN(16, 16, 16), P3_PLAN(30, 10, 3, 9), P3_PLAN(18, 18, 16),
     P3_PLAN(20, 20, 15), P3_PLAN(20, 20, 16), P3_PLAN(18, 18, 18),
+    // a factor 7: here three stages of 7 to 14 values beat two of 18 to 21
+    // (252^3 grid points: 152 against 181 us, 280^3: 226, 257, 294^3: 258, 301)
+    P3_PLAN(14, 14, 12), P3_PLAN(14, 14, 14), P3_PLAN(15, 14, 15), P3_PLAN(16, 14, 16), P3_PLAN(21, 6, 6, 7),
+    P3_PLAN(56, 8, 5, 7), P3_PLAN(49, 6, 7, 7),
 };
 const P3Shape* p3_shapes_medium(int& n) {
   n = (int)(sizeof(kShapes) / sizeof(kShapes[0]));

@@ -14,6 +14,9 @@ static const P3Shape kShapes[] = {
     P3_PLAN(5, 10, 5), P3_PLAN(9, 6, 9), P3_PLAN(10, 10, 6), P3_PLAN(8, 8, 8), P3_PLAN(9, 8, 9), P3_PLAN(10, 8, 10),
     P3_PLAN(10, 10, 9), P3_PLAN(12, 12, 8), P3_PLAN(10, 10, 10), P3_PLAN(12, 12, 9), P3_PLAN(12, 12, 10),
     P3_PLAN(8, 16, 8), P3_PLAN(12, 12, 12), P3_PLAN(30, 6, 5, 5), P3_PLAN(16, 16, 10),
+    // a factor 7
+    P3_PLAN(7, 4, 7), P3_PLAN(7, 6, 7), P3_PLAN(8, 8, 7), P3_PLAN(10, 10, 7), P3_PLAN(12, 12, 7), P3_PLAN(14, 14, 7),
+    P3_PLAN(14, 14, 8), P3_PLAN(14, 14, 9), P3_PLAN(14, 14, 10),
 };
 const P3Shape* p3_shapes_short(int& n) {
   n = (int)(sizeof(kShapes) / sizeof(kShapes[0]));

@@ -12,6 +12,9 @@ static const RowShape kShapes[] = {
     X_BOTH(20, 20), X_BOTH(24, 18), X_BOTH(25, 18), X_BOTH(24, 20), X_BOTH(27, 18), X_FWD(25, 20, 16),
     X_FWD(32, 16, 16), X_BOTH(27, 20), X_BOTH(24, 24), X_BOTH(25, 24), X_BOTH(32, 20), X_BOTH(27, 24), X_BOTH(30, 24),
     X_BOTH(30, 25), X_BOTH(32, 24),
+    // a factor 7
+    X_BOTH(20, 14), X_BOTH(21, 14), X_BOTH(24, 14), X_BOTH(25, 14), X_BOTH(27, 14), X_BOTH(28, 14), X_BOTH(28, 15),
+    X_BOTH(32, 14), X_BOTH(35, 14), X_BOTH(28, 18),
     // 512 points: 32 rows, 256 bytes of a1 per kx (256^3: 506 us against 551 with 16 rows)
     X_INV(32, 16, 32, 2, true, false), X_INV(32, 16, 16, 2, true, false), X_INV(32, 24, 16, 4, true, false),
     X_INV(25, 20, 16, 2, false, false),

@@ -13,6 +13,10 @@ static const RowShape kShapes[] = {
     X_BOTH(12, 9, 16),  X_BOTH(12, 10, 16), X_BOTH(16, 8, 16),  X_BOTH(12, 12, 16), X_BOTH(15, 10, 16),
     X_BOTH(16, 10, 16), X_BOTH(18, 9, 16),  X_BOTH(15, 12, 16), X_BOTH(16, 12, 16), X_FWD(20, 10, 16),
     X_FWD(18, 12, 16),  X_BOTH(16, 15, 16), X_FWD(25, 10, 16),  X_BOTH(16, 16, 16),
+    // a factor 7
+    X_BOTH(7, 4, 32), X_BOTH(7, 6, 32), X_BOTH(8, 7, 32), X_BOTH(10, 7, 32), X_BOTH(12, 7, 16), X_BOTH(14, 7, 16),
+    X_BOTH(16, 7, 16), X_BOTH(14, 9, 16), X_BOTH(14, 10, 16), X_BOTH(14, 12, 16), X_BOTH(14, 14, 16),
+    X_BOTH(15, 14, 16), X_BOTH(16, 14, 16), X_BOTH(18, 14, 16),
     // one component at a time (200 points: 72 -> 65 us, 216: 77 -> 73 us on 128 x 128 rows)
     X_INV(20, 10, 16, 5, false, false), X_INV(18, 12, 16, 3, false, false), X_INV(25, 10, 16, 5, false, false),
 };
