@@ -374,16 +374,19 @@ int matvec_plan(Context& c, const char* name) {
   if ((m.ty == WIDE_THREADS || m.tz == WIDE_THREADS) && allow_big_lds(lds_max)) return 206;
   if (upload_twiddles(m.gx, &m.twx) || upload_twiddles(m.gy, &m.twy) || upload_twiddles(m.gz, &m.twz)) return 206;
   // z runs start on 128-byte lines, or on half lines where a whole one would
-  // pad by more than a tenth (8 right-hand sides of 48 x 50 x 50: 161 us at a
-  // pitch of 64, 147 at 56, 146 at 52; NZ = 108, which 112 pads by 4 %: 350 us,
-  // 361 unpadded); targets of a few planes keep a small pitch
+  // pad by more than a twentieth (16 right-hand sides of 48 x 50 x 50: 357 us at
+  // a pitch of 64, 332 at 56; of 72 x 80 x 120: 1,827 at 128, 1,724 at 120;
+  // NZ = 108, which 112 pads by 4 %: 350 us, 361 unpadded); targets of a few
+  // planes keep a small pitch
   const int line = (c.nz + 15) & ~15;
-  m.nzp = c.nz <= 32 ? (c.nz + 3) & ~3 : 10 * (line - c.nz) > c.nz ? (c.nz + 7) & ~7 : line;
-  // an odd number of 256-byte blocks per kx plane: passes 1 and 5 step through
-  // the planes, and a power-of-two step would hit few memory channels
-  const auto odd_blocks = [](int n) { return ((n + 31) / 32 | 1) * 32; };
-  m.p1 = odd_blocks(c.ny * m.nzp);
-  m.p2 = odd_blocks(m.gy * m.nzp);
+  m.nzp = c.nz <= 32 ? (c.nz + 3) & ~3 : 20 * (line - c.nz) > c.nz ? (c.nz + 7) & ~7 : line;
+  // an odd number of 128-byte lines per kx plane: passes 1 and 5 step through
+  // the planes, and an even step hits fewer memory channels (pass 4 at 256^3
+  // 505 us with the power of two it has unpadded, 456 so; an odd number of
+  // 256-byte blocks 0 to 4 % slower on MATVECs of 16 right-hand sides)
+  const auto odd_lines = [](int n) { return ((n + 15) / 16 | 1) * 16; };
+  m.p1 = odd_lines(c.ny * m.nzp);
+  m.p2 = odd_lines(m.gy * m.nzp);
   return 0;
 }
 
