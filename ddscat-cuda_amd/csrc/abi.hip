@@ -194,6 +194,7 @@ extern "C" DDSCAT_HIP_API int ddscat_hip_set_pass_kernel(int pass, int kind) {
   const int lens[6] = {0, c.mv.gx, c.mv.gy, c.mv.gz, c.mv.gy, c.mv.gx};
   if (kind < -1 || kind >= reg_candidates(lens[pass], pass)) { set_error("set_pass_kernel", "no such kernel"); return 11; }
   c.mv.kind[pass] = kind;
+  if (pass >= 2 && pass <= 4) c.mv.plane = 0;
   c.mv.tuned = 0;
   return 0;
 }

@@ -482,6 +482,11 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   bt.slab = KxSlab{0, c.nx, c.mv.gx};
   for (int p = 1; p <= 5; ++p) {
     if (ev) hipEventRecord(ev[p - 1], st);
+    if (c.mv.plane && p >= 2 && p <= 4) {
+      if (p != 3) continue;
+      if (int rc = plane_yz_launch(c, st, bt)) return rc;
+      continue;
+    }
     if (int rc = launch_pass(c, p, c.mv.kind[p], cj, compact, x, y, adia, aoff, st, bt)) return rc;
   }
   DDH_LAUNCH_OK("MATVEC register passes", 20);
@@ -525,6 +530,7 @@ int matvec_autotune(Context& c) {
   const int lens[6] = {0, m.gx, m.gy, m.gz, m.gy, m.gx};
   for (int p = 1; p <= 5; ++p) m.kind[p] = reg_candidates(lens[p], p) > 0 ? 0 : -1;
   m.tuned = 0;
+  if (int rc = plane_yz_setup(c)) return rc;
   if (!c.autotune || c.fft_generic || !c.sx || !c.sy || !c.adia_c || !c.aoff_c) return 0;
   const TuneKey key{c.nx, c.ny, c.nz, c.ipbc};
   auto it = tune_cache().find(key);

@@ -90,6 +90,43 @@ __device__ __forceinline__ void p3_column(const P3Cols& q, int col, int gy, int&
 // and four points 133 and 129 us against 122 at 128^3).  MIRROR: octant stored (IPBC=0), else the whole
 // grid (one kernel with both forms of the multiply keeps a second copy of the
 // column live across the branch: 256 instead of 161 registers at 16 x 16)
+// z-FFT, Green multiply and inverse z-FFT of a column held as stage-0 inputs
+// in v; xb: the column's exchange slots; g0: byte offset of its Green entries
+template <class PL, bool MIRROR>
+__device__ __forceinline__ void p3_transform(float2 (&v)[3][PL::V], float2* xb, const float2* tw, int j,
+                                             const char* gb, unsigned g0) {
+  constexpr int L = PL::L, SL = PL::S - 1, RL = PL::rad(SL);
+#pragma unroll
+  for (int c = 0; c < 3; ++c) w_forward<PL, +1>(v[c], xb, tw, j);
+#pragma unroll
+  for (int b = 0; b < PL::nb(SL); ++b)
+#pragma unroll
+    for (int r = 0; r < RL; ++r) {
+      const int e = b * RL + r, k = w_bfly<PL, SL>(j, b) + r * (L / RL);
+      // a point lies in the mirrored half k > L / 2 when 2 r >= RL, but for
+      // k = L / 2 itself and, with an odd RL, the middle group's first half
+      const bool up = MIRROR && 2 * r + 1 >= RL;
+      const bool mixed = MIRROR && (2 * r == RL || 2 * r + 1 == RL);
+      const bool hi = up && (!mixed || k > L / 2);
+      const Green6 G = green_at_b(gb, g0 + (unsigned)(hi ? L - k : k) * 48u);
+      float2 g13 = G.xz, g23 = G.yz;
+      if (mixed) {
+        const float sz = hi ? -1.f : 1.f;
+        g13 = cscale(g13, sz);
+        g23 = cscale(g23, sz);
+      } else if (up) {
+        g13 = make_float2(-g13.x, -g13.y);
+        g23 = make_float2(-g23.x, -g23.y);
+      }
+      const float2 p0 = v[0][e], p1 = v[1][e], p2 = v[2][e];
+      v[0][e] = cdot3(G.xx, p0, G.xy, p1, g13, p2);
+      v[1][e] = cdot3(G.xy, p0, G.yy, p1, g23, p2);
+      v[2][e] = cdot3(g13, p0, g23, p1, G.zz, p2);
+      if (e & 1) __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+  for (int c = 0; c < 3; ++c) w_inverse<PL, -1>(v[c], xb, tw, j);
+}
 // The waves per SIMD that 6 V registers of column data leave room for are
 // asked of the compiler: left alone it ends a few registers above a step now
 // and then (18 x 16 points at 170 instead of 168, 2 waves instead of 3: 385 us
@@ -102,7 +139,7 @@ template <class PL, bool MIRROR>
 __global__ __launch_bounds__(64 * P3_WAVES) __attribute__((amdgpu_waves_per_eu(p3_waves_per_simd<PL>()))) void kw_pass3(
     float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg, int nz, int nzp, int p2, int gy,
     BatchArgs ba, GreenGeo gg, P3Cols q) {
-  constexpr int L = PL::L, T = PL::T, V = PL::V, SEQ = PL::SEQ, R0 = PL::rad(0), SL = PL::S - 1, RL = PL::rad(SL);
+  constexpr int L = PL::L, T = PL::T, V = PL::V, SEQ = PL::SEQ, R0 = PL::rad(0);
   static_assert(R0 % 2 == 0, "the zero half of a padded column is a compile-time set");
   __shared__ float2 tw[L];
   __shared__ float2 xbuf[P3_WAVES * SEQ * PL::SLOTS];
@@ -143,38 +180,8 @@ __global__ __launch_bounds__(64 * P3_WAVES) __attribute__((amdgpu_waves_per_eu(p
       v[0][e] = cscale(v[0][e], sx);
       v[1][e] = cscale(v[1][e], sy);
     }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) w_forward<PL, +1>(v[c], xb, tw, j);
-  const char* const gb = reinterpret_cast<const char*>(green);
   const unsigned g0 = ((unsigned)ir * (unsigned)gg.oy + (unsigned)jr) * (unsigned)gg.oz * 48u;
-#pragma unroll
-  for (int b = 0; b < PL::nb(SL); ++b)
-#pragma unroll
-    for (int r = 0; r < RL; ++r) {
-      const int e = b * RL + r, k = w_bfly<PL, SL>(j, b) + r * (L / RL);
-      // a point lies in the mirrored half k > L / 2 when 2 r >= RL, but for
-      // k = L / 2 itself and, with an odd RL, the middle group's first half
-      const bool up = MIRROR && 2 * r + 1 >= RL;
-      const bool mixed = MIRROR && (2 * r == RL || 2 * r + 1 == RL);
-      const bool hi = up && (!mixed || k > L / 2);
-      const Green6 G = green_at_b(gb, g0 + (unsigned)(hi ? L - k : k) * 48u);
-      float2 g13 = G.xz, g23 = G.yz;
-      if (mixed) {
-        const float sz = hi ? -1.f : 1.f;
-        g13 = cscale(g13, sz);
-        g23 = cscale(g23, sz);
-      } else if (up) {
-        g13 = make_float2(-g13.x, -g13.y);
-        g23 = make_float2(-g23.x, -g23.y);
-      }
-      const float2 p0 = v[0][e], p1 = v[1][e], p2 = v[2][e];
-      v[0][e] = cdot3(G.xx, p0, G.xy, p1, g13, p2);
-      v[1][e] = cdot3(G.xy, p0, G.yy, p1, g23, p2);
-      v[2][e] = cdot3(g13, p0, g23, p1, G.zz, p2);
-      if (e & 1) __builtin_amdgcn_sched_barrier(0);
-    }
-#pragma unroll
-  for (int c = 0; c < 3; ++c) w_inverse<PL, -1>(v[c], xb, tw, j);
+  p3_transform<PL, MIRROR>(v, xb, tw, j, reinterpret_cast<const char*>(green), g0);
 #pragma unroll
   for (int b = 0; b < PL::nb(0); ++b) {
     const unsigned ob = o0 + 8u * (unsigned)w_bfly<PL, 0>(j, b);

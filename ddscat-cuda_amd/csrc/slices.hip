@@ -82,7 +82,9 @@ int slices_matvec(Context& c, int cwhat, const float2* x, float2* y, const float
   bt.a1 = c.a1;
   bt.k.active = act;
   if (int rc = matvec_end_pass(c, 1, cwhat, x, y, adia, aoff, layout, st, bt)) return rc;
-  if (s.nslab == 1) {
+  if (c.mv.plane) {
+    if (int rc = plane_yz_launch(c, st, bt)) return rc;
+  } else if (s.nslab == 1) {
     slices_slab(c, 0, bt);
     if (int rc = matvec_slab(c, st, bt)) return rc;
   } else {

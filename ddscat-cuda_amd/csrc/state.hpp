@@ -26,6 +26,7 @@ struct MatvecPlan {
   // FFT kernel per pass 1..5: index into the register shapes of that pass's
   // axis length, or -1 for the LDS-staged kernel (chosen by the autotuner)
   int kind[6] = {-1, -1, -1, -1, -1, -1};
+  int plane = 0;  // passes 2 to 4 by the plane kernel (plane_yz.hpp)
   int tuned = 0;
 };
 
@@ -160,6 +161,10 @@ int reg_pass(Context& c, int which, int cand, int cj, int compact, const float2*
 int matvec_slab(Context& c, hipStream_t st, const MvBatch& bt);
 // SLICES: bt's slab and a2: the slab of planes from half-plane h0 and its buffer
 void slices_slab(const Context& c, int h0, MvBatch& bt);
+// the plane kernel in place of passes 2 to 4, in place on every plane of bt.a1:
+// whether the prepared grid takes it (c.mv.plane), and its launch
+int plane_yz_setup(Context& c);
+int plane_yz_launch(Context& c, hipStream_t st, const MvBatch& bt);
 // pass 1 (x -> a1) or 5 (a1 -> y) alone
 int matvec_end_pass(Context& c, int which, int cwhat, const float2* x, float2* y, const float2* adia,
                     const float2* aoff, int layout, hipStream_t st, const MvBatch& bt);
