@@ -5,6 +5,7 @@
 // (ddscat_cuda_unified/cuda/ddscat_matvec_cuda.cu:66-79, 1005-1026).
 #include "state.hpp"
 #include "solver_common.hpp"
+#include <algorithm>
 #include <vector>
 #include <cstring>
 #include <mutex>
@@ -68,7 +69,7 @@ void release_context(Context& c) {
   slices_release(c);
   batch_release(c);
   dfree(c.green);
-  dfree(c.iocc); dfree(c.occ); dfree(c.rowptr); dfree(c.rowlo); dfree(c.qmap);
+  dfree(c.iocc); dfree(c.occ); dfree(c.rowptr); dfree(c.rowlo); dfree(c.qmap); dfree(c.ysup);
   dfree(c.adia); dfree(c.aoff); dfree(c.adia_c); dfree(c.aoff_c);
   dfree(c.xfull); dfree(c.yfull);
   dfree(c.sx); dfree(c.sy); dfree(c.sb);
@@ -86,6 +87,36 @@ void release_context(Context& c) {
   c.precision = prec;
   c.fft_generic = gen;
   c.autotune = tune;
+}
+
+// The occupied iy range of each run of 1 << zsh lattice planes iz, the planes
+// that share a half or whole 128-byte line of a1.  Worth a table where it
+// leaves out a thirty-second of the rows (an ellipsoid: a fifth) of an a1 that
+// does not fit the 256 MiB in front of HBM, and where the y passes are those
+// of 512 and 768 points (MATVECs of ellipsoids: 256^3 2,660 -> 2,570 us, SLICES
+// 2,665 -> 2,590, 384^3 9,435 -> 9,120).  The shorter two-level kernels had
+// less to gain: 160^3 720 without and 730 with, 200^3 1,461 and 1,448.
+constexpr size_t SUPPORT_MIN_A1 = (size_t)256 << 20;
+static int upload_support(Context& c, const std::vector<int>& rowptr, int code) {
+  c.mv.zsh = c.mv.nzp % 16 == 0 ? 4 : 3;
+  if (c.mv.nzp % 8 || (c.mv.gy != 512 && c.mv.gy != 768) || matvec_a1_count(c) * sizeof(float2) < SUPPORT_MIN_A1) return 0;
+  const int zt = 1 << c.mv.zsh, runs = c.mv.nzp / zt;
+  std::vector<int2> sup((size_t)runs);
+  long long rows = 0;
+  for (int r = 0; r < runs; ++r) {
+    int lo = c.ny, hi = 0;
+    for (int iz = r * zt; iz < std::min(c.nz, (r + 1) * zt); ++iz)
+      for (int iy = 0; iy < c.ny; ++iy) {
+        const size_t g = iy + (size_t)c.ny * iz;
+        if (rowptr[g + 1] > rowptr[g]) { lo = std::min(lo, iy); hi = std::max(hi, iy + 1); }
+      }
+    sup[r] = hi > lo ? make_int2(lo, hi) : make_int2(0, 0);
+    rows += sup[r].y - sup[r].x;
+  }
+  if (32 * rows > 31LL * runs * c.ny) return 0;
+  DDH_TRY(hipMalloc((void**)&c.ysup, sup.size() * sizeof(int2)), "malloc row support", code);
+  DDH_TRY(hipMemcpy(c.ysup, sup.data(), sup.size() * sizeof(int2), hipMemcpyHostToDevice), "row support H2D", code);
+  return 0;
 }
 
 // Common tail of prepare_green / prepare: dimensions already set, Green
@@ -133,6 +164,7 @@ int finish_prepare(Context& c, const int16_t* iocc, int code_alloc, int code_occ
   c.rows_contiguous = contiguous ? 1 : 0;
   DDH_TRY(hipMalloc((void**)&c.rowlo, (size_t)nrows * sizeof(int)), "malloc row map", code_alloc);
   DDH_TRY(hipMemcpy(c.rowlo, rowlo.data(), (size_t)nrows * sizeof(int), hipMemcpyHostToDevice), "row map H2D", code_alloc);
+  if (int r = upload_support(c, rowptr, code_alloc)) return r;
   if (!contiguous) {
     std::vector<int> qmap((size_t)c.nat, -1);
     for (size_t q = 0; q < occ.size() && q < (size_t)c.nat0; ++q) qmap[(size_t)occ[q]] = (int)q;

@@ -472,6 +472,13 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
   return 0;
 }
 
+void matvec_support(const Context& c, int layout, BatchArgs& k) {
+  const MatvecPlan& m = c.mv;
+  const bool reg = !c.fft_generic && !m.plane && m.kind[1] >= 0 && m.kind[2] >= 0 && m.kind[4] >= 0 && m.kind[5] >= 0;
+  k.ysup = layout && reg ? c.ysup : nullptr;
+  k.zsh = m.zsh;
+}
+
 int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float2* adia,
                   const float2* aoff, int layout, hipStream_t st, hipEvent_t* ev, const MvBatch* btp) {
   const int cj = (cwhat == 'C') ? 1 : 0;
@@ -479,6 +486,7 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   MvBatch bt = btp ? *btp : MvBatch{};
   if (!bt.a1) bt.a1 = c.a1;
   if (!bt.a2) bt.a2 = c.a2;
+  matvec_support(c, layout, bt.k);
   bt.slab = KxSlab{0, c.nx, c.mv.gx};
   for (int p = 1; p <= 5; ++p) {
     if (ev) hipEventRecord(ev[p - 1], st);

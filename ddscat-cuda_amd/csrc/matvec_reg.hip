@@ -95,7 +95,8 @@ __global__ __launch_bounds__(R1 * C) void kr_passy(const float2* __restrict__ in
 // 768-point column tile of C = 8 needs about 36 KB of LDS instead of the
 // 61 KB of the two-level 32 x 24 shape.  DIR = +1: nin (<= L/2, pruned)
 // inputs -> L spectral outputs; DIR = -1: L spectral inputs -> nout (<= L/2).
-template <int M, int C, int DIR>
+// SUP: only the inputs or outputs in the row support.
+template <int M, int C, int DIR, bool SUP>
 __global__ __launch_bounds__(M * 16 * C) void kr_passym(const float2* __restrict__ in, float2* __restrict__ out,
                                                     const float2* __restrict__ twg, Cols q, int nin, int nout,
                                                     BatchArgs ba) {
@@ -118,6 +119,7 @@ __global__ __launch_bounds__(M * 16 * C) void kr_passym(const float2* __restrict
   const bool live = q0 + s < q.total;
   int o, col;
   column_of(q, q0, live ? s : 0, o, col);
+  const int2 sup = SUP ? ba.ysup[col >> ba.zsh] : make_int2(0, DIR > 0 ? nin : nout);
   const int gx = q.pitch;
   const size_t o1 = c * q.c1 + q.sl.kx(o) * q.p1 + col, o2 = c * q.c2 + o * q.p2 + col;
   const float2* src = in + (DIR > 0 ? o1 : o2);
@@ -159,7 +161,7 @@ __global__ __launch_bounds__(M * 16 * C) void kr_passym(const float2* __restrict
 #pragma unroll
     for (int n2 = 0; n2 < R; ++n2) {
       const int n = M * (t + R * n2) + m;
-      v[n2] = live && n2 < R / 2 && n < nin ? src[(size_t)n * gx] : make_float2(0.f, 0.f);
+      v[n2] = live && n2 < R / 2 && (!SUP || n >= sup.x) && n < sup.y ? src[(size_t)n * gx] : make_float2(0.f, 0.f);
     }
     __syncthreads();
     fft2_fwd_s<R, R, +1>(v, xf, twS, t, sv, PS);  // v[i] = Y_m[t + 16 i]
@@ -180,7 +182,7 @@ __global__ __launch_bounds__(M * 16 * C) void kr_passym(const float2* __restrict
 #pragma unroll
       for (int n2 = 0; n2 < R / 2; ++n2) {
         const int n = M * (t + R * n2) + m;
-        if (n < nout) dst[(size_t)n * gx] = v[n2];
+        if ((!SUP || n >= sup.x) && n < sup.y) dst[(size_t)n * gx] = v[n2];
       }
     }
   }
@@ -212,10 +214,13 @@ static void launch_y_m(Context& c, int dir, const MvBatch& bt, hipStream_t st) {
   const MatvecPlan& m = c.mv;
   const Cols q = y_cols(c, bt.slab);
   const dim3 grid((q.total + C - 1) / C, 1, 3 * (unsigned)bt.nrhs), block(M * 16 * C);
-  if (dir > 0)
-    hipLaunchKernelGGL((kr_passym<M, C, +1>), grid, block, 0, st, bt.a1, bt.a2, m.twy, q, c.ny, m.gy, bt.k);
-  else
-    hipLaunchKernelGGL((kr_passym<M, C, -1>), grid, block, 0, st, bt.a2, bt.a1, m.twy, q, m.gy, c.ny, bt.k);
+  if (dir > 0) {
+    const auto kernel = bt.k.ysup ? &kr_passym<M, C, +1, true> : &kr_passym<M, C, +1, false>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, bt.a1, bt.a2, m.twy, q, c.ny, m.gy, bt.k);
+  } else {
+    const auto kernel = bt.k.ysup ? &kr_passym<M, C, -1, true> : &kr_passym<M, C, -1, false>;
+    hipLaunchKernelGGL(kernel, grid, block, 0, st, bt.a2, bt.a1, m.twy, q, m.gy, c.ny, bt.k);
+  }
 }
 struct YShape {
   int L;

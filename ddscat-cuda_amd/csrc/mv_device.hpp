@@ -17,6 +17,22 @@ struct SiteMap {
   int contiguous;
 };
 
+// whether any of rows q0 .. q0 + C - 1 (q = iy nzp + iz) is in the support; uniform
+template <int C>
+__device__ __forceinline__ bool rows_in_support(const BatchArgs& ba, int q0, int ny, int nzp) {
+  if (!ba.ysup) return true;
+  const int zt = 1 << ba.zsh;
+  int iy = q0 / nzp, iz = q0 - iy * nzp;
+  bool any = false;
+  for (int n = 0; n < C && iy < ny; n += zt) {
+    const int2 r = ba.ysup[iz >> ba.zsh];
+    any |= iy >= r.x && iy < r.y;
+    iz += zt;
+    if (iz >= nzp) { iz -= nzp; ++iy; }
+  }
+  return any;
+}
+
 // compact index of site (row g, ix), or -1 when void
 __device__ __forceinline__ int compact_index(const SiteMap& m, int g, int ix, int nx) {
   if (m.contiguous) {

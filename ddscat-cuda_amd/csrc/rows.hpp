@@ -42,6 +42,7 @@ __global__ __launch_bounds__(R1 * C) void kx_fwd(const float2* __restrict__ x, f
   x += rb * ba.xs;
   a1 += rb * ba.a1s;
   const int c = blockIdx.y, q0 = blockIdx.x * C;
+  if (!rows_in_support<C>(ba, q0, ny, nzp)) return;
   for (int i = threadIdx.x; i < L; i += RT) twL[i] = twg[i];
   // load side: lanes over x
   const int t = threadIdx.x % R1, s = threadIdx.x / R1;
@@ -151,6 +152,7 @@ __global__ __launch_bounds__(R1 * C) void kx_inv(const float2* __restrict__ a1, 
   adia += rb * ba.os;
   aoff += rb * ba.os;
   const int q0 = blockIdx.x * C;
+  if (!rows_in_support<C>(ba, q0, ny, nzp)) return;
   for (int i = threadIdx.x; i < L; i += RT) twL[i] = twg[i];
   const int s2 = threadIdx.x % C, t2 = threadIdx.x / C;  // load side: lanes over the rows
   const int t = threadIdx.x % R1, s = threadIdx.x / R1;  // finish side: lanes over x

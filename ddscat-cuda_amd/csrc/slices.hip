@@ -81,6 +81,7 @@ int slices_matvec(Context& c, int cwhat, const float2* x, float2* y, const float
   MvBatch bt;
   bt.a1 = c.a1;
   bt.k.active = act;
+  matvec_support(c, layout, bt.k);
   if (int rc = matvec_end_pass(c, 1, cwhat, x, y, adia, aoff, layout, st, bt)) return rc;
   if (c.mv.plane) {
     if (int rc = plane_yz_launch(c, st, bt)) return rc;

@@ -26,6 +26,7 @@ struct MatvecPlan {
   // FFT kernel per pass 1..5: index into the register shapes of that pass's
   // axis length, or -1 for the LDS-staged kernel (chosen by the autotuner)
   int kind[6] = {-1, -1, -1, -1, -1, -1};
+  int zsh = 0;    // log2 of the z run length of the row support (c.ysup)
   int plane = 0;  // passes 2 to 4 by the plane kernel (plane_yz.hpp)
   int tuned = 0;
 };
@@ -83,6 +84,7 @@ struct Context {
   int* rowptr = nullptr;       // [ny*nz+1] compact range of each (iy,iz) row
   int* rowlo = nullptr;        // [ny*nz] first occupied ix of each row
   int* qmap = nullptr;         // [nat] full site -> compact index (-1 void); built when rows are not intervals
+  int2* ysup = nullptr;        // occupied iy range of each z run (BatchArgs::ysup); nullptr where it is nearly all
   int rows_contiguous = 0;     // every row's occupied sites form one interval
   int fft_generic = 0;         // 1: force the LDS-staged generic FFT kernels
   int autotune = 1;            // 1: time the FFT kernel candidates per pass at prepare
@@ -120,6 +122,12 @@ void release_solver_workspace(Context& c);
 struct BatchArgs {
   size_t xs = 0, os = 0, a1s = 0, a2s = 0;
   const int* active = nullptr;
+  // Support of a compact vector: occupied iy range [x, y) of each 1 << zsh
+  // consecutive iz; nullptr: all rows.  Pass 1 leaves the rows of a1 outside
+  // it unwritten and pass 2 takes them as zero; pass 4 leaves them unwritten
+  // and pass 5, which has no site there, does not read them.
+  const int2* ysup = nullptr;
+  int zsh = 0;
 };
 // The kx planes of a2: 2 H slots, slot s < H holding kx = h0 + s and slot H + s
 // its mirror 2NX - kx (the plane of the same Green entries; for kx = 0, which
@@ -148,6 +156,8 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
                   const float2* aoff, int layout, hipStream_t st, hipEvent_t* ev = nullptr,
                   const MvBatch* bt = nullptr);
 int matvec_setup(Context& c);
+// sets the row support in k for a call of this layout, where the kernels of the plan honour it
+void matvec_support(const Context& c, int layout, BatchArgs& k);
 void matvec_release(Context& c);
 // FFT work elements per RHS: a1 [3][gx][p1: ny][nzp], a2 [3][gx][p2: gy][nzp]
 size_t matvec_a1_count(const Context& c);
