@@ -30,13 +30,14 @@ __device__ __forceinline__ void column_of(const Cols& q, int q0, int s, int& o, 
   }
 }
 // nin inputs -> nout outputs per column.
-template <int R1, int R2, int C, int DIR>
+template <int R1, int R2, int C, bool SPL, int DIR>
 __global__ __launch_bounds__(R1 * C) void kr_passy(const float2* __restrict__ in, float2* __restrict__ out,
                                                const float2* __restrict__ twg, Cols q, int nin, int nout,
                                                BatchArgs ba) {
   constexpr int L = R1 * R2, RT = R1 * C, P = C + 1, G = Reg2<R1, R2>::G, VN = Reg2<R1, R2>::VN;
   __shared__ float2 twL[L];
-  __shared__ float2 buf[L * P];
+  __shared__ float2 buf[SPL ? (L * P + 1) / 2 : L * P];
+  float* const bufs = reinterpret_cast<float*>(buf);
   const int rb = blockIdx.z / 3;
   if (ba.active && !ba.active[rb]) return;
   in += rb * (DIR > 0 ? ba.a1s : ba.a2s);
@@ -59,7 +60,10 @@ __global__ __launch_bounds__(R1 * C) void kr_passy(const float2* __restrict__ in
       v[n2] = live && lower_half<R2>(n2, n, nin) ? src[(size_t)n * gx] : make_float2(0.f, 0.f);
     }
     __syncthreads();
-    fft2_fwd<R1, R2, +1>(v, buf, twL, t, s, P);
+    if constexpr (SPL)
+      fft2_fwd_s<R1, R2, +1>(v, bufs, twL, t, s, P);
+    else
+      fft2_fwd<R1, R2, +1>(v, buf, twL, t, s, P);
     if (live) {
 #pragma unroll
       for (int i = 0; i < G; ++i)
@@ -75,7 +79,10 @@ __global__ __launch_bounds__(R1 * C) void kr_passy(const float2* __restrict__ in
         v[i * R1 + k1] = (live && reg2_owns<R1, R2>(t, i)) ? src[(size_t)((t + R1 * i) + R2 * k1) * gx]
                                                            : make_float2(0.f, 0.f);
     __syncthreads();
-    fft2_inv<R1, R2, -1>(v, buf, twL, t, s, P);
+    if constexpr (SPL)
+      fft2_inv_s<R1, R2, -1>(v, bufs, twL, t, s, P);
+    else
+      fft2_inv<R1, R2, -1>(v, buf, twL, t, s, P);
     if (live) {
 #pragma unroll
       for (int n2 = 0; n2 < R2; ++n2) {
@@ -199,15 +206,15 @@ static Cols y_cols(const Context& c, const KxSlab& sl) {
   const size_t p1 = m.p1, p2 = m.p2;
   return Cols{m.nzp, m.nzp * 2 * sl.H, m.nzp, p1, p2, p1 * m.gx, p2 * 2 * sl.H, sl};
 }
-template <int R1, int R2, int C>
+template <int R1, int R2, int C, bool SPL = false>
 static void launch_y(Context& c, int dir, const MvBatch& bt, hipStream_t st) {
   const MatvecPlan& m = c.mv;
   const Cols q = y_cols(c, bt.slab);
   const dim3 grid((q.total + C - 1) / C, 1, 3 * (unsigned)bt.nrhs), block(R1 * C);
   if (dir > 0)
-    hipLaunchKernelGGL((kr_passy<R1, R2, C, +1>), grid, block, 0, st, bt.a1, bt.a2, m.twy, q, c.ny, m.gy, bt.k);
+    hipLaunchKernelGGL((kr_passy<R1, R2, C, SPL, +1>), grid, block, 0, st, bt.a1, bt.a2, m.twy, q, c.ny, m.gy, bt.k);
   else
-    hipLaunchKernelGGL((kr_passy<R1, R2, C, -1>), grid, block, 0, st, bt.a2, bt.a1, m.twy, q, m.gy, c.ny, bt.k);
+    hipLaunchKernelGGL((kr_passy<R1, R2, C, SPL, -1>), grid, block, 0, st, bt.a2, bt.a1, m.twy, q, m.gy, c.ny, bt.k);
 }
 template <int M, int C>
 static void launch_y_m(Context& c, int dir, const MvBatch& bt, hipStream_t st) {
@@ -227,9 +234,15 @@ struct YShape {
   void (*fn)(Context&, int, const MvBatch&, hipStream_t);
 };
 #define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>}
+#define Y_SPLIT(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C, true>}
 // One shape per padded length 2N, N = 2^a 3^b 5^c 7^d from 12 to 256 and a few
 // above (two-level, R1 threads per column, at most 25 values each, C columns
 // per workgroup; 512 and 768 points by decimation, 20 and 30 % faster there).
+// The real and imaginary parts cross in turn (Y_SPLIT), with half the LDS and
+// twice the workgroups on a CU for two further barriers, at the lengths where
+// that gained a percent or more of a MATVEC: 192^3 1,249 -> 1,165 us, 200^3
+// 1,536 -> 1,413, 216^3 1,974 -> 1,809, 240^3 2,582 -> 2,520, 144^3 539 -> 529,
+// 162^3 827 -> 811 (96^3 to 140^3: 0 to 2 % slower, 250^3 2,825 and 2,984).
 // Lengths of other sizes use the LDS-staged kernels (the y passes of a 70^3
 // grid: 34 us each against 14 to 16 here, 196^3: 470 against 213 to 235).
 static const YShape kYShapes[] = {
@@ -238,9 +251,9 @@ static const YShape kYShapes[] = {
     Y_SHAPE(10, 8, 32), Y_SHAPE(10, 9, 32), Y_SHAPE(12, 8, 16), Y_SHAPE(10, 10, 32), Y_SHAPE(12, 9, 16),
     Y_SHAPE(12, 10, 16), Y_SHAPE(8, 16, 32), Y_SHAPE(12, 12, 16), Y_SHAPE(15, 10, 16), Y_SHAPE(16, 10, 16),
     Y_SHAPE(18, 9, 16), Y_SHAPE(15, 12, 16), Y_SHAPE(16, 12, 16), Y_SHAPE(20, 10, 16), Y_SHAPE(18, 12, 16),
-    Y_SHAPE(16, 15, 16), Y_SHAPE(25, 10, 16), Y_SHAPE(16, 16, 32), Y_SHAPE(18, 15, 16), Y_SHAPE(18, 16, 16),
-    Y_SHAPE(20, 15, 16), Y_SHAPE(20, 16, 16), Y_SHAPE(18, 18, 16), Y_SHAPE(20, 18, 16), Y_SHAPE(24, 16, 16),
-    Y_SHAPE(20, 20, 16), Y_SHAPE(24, 18, 16), Y_SHAPE(25, 18, 16), Y_SHAPE(24, 20, 16), Y_SHAPE(27, 18, 16),
+    Y_SHAPE(16, 15, 16), Y_SHAPE(25, 10, 16), Y_SHAPE(16, 16, 32), Y_SHAPE(18, 15, 16), Y_SPLIT(18, 16, 16),
+    Y_SHAPE(20, 15, 16), Y_SHAPE(20, 16, 16), Y_SPLIT(18, 18, 16), Y_SHAPE(20, 18, 16), Y_SPLIT(24, 16, 16),
+    Y_SPLIT(20, 20, 16), Y_SPLIT(24, 18, 16), Y_SPLIT(25, 18, 16), Y_SPLIT(24, 20, 16), Y_SHAPE(27, 18, 16),
     Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
     Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>},
     // a factor 7
@@ -248,7 +261,7 @@ static const YShape kYShapes[] = {
     Y_SHAPE(14, 7, 16), Y_SHAPE(14, 8, 16), Y_SHAPE(14, 9, 16), Y_SHAPE(14, 10, 16), Y_SHAPE(14, 12, 16),
     Y_SHAPE(14, 14, 32), Y_SHAPE(15, 14, 16), Y_SHAPE(16, 14, 16), Y_SHAPE(18, 14, 16), Y_SHAPE(20, 14, 16),
     Y_SHAPE(21, 14, 16), Y_SHAPE(21, 16, 16), Y_SHAPE(25, 14, 16), Y_SHAPE(27, 14, 16), Y_SHAPE(28, 14, 16),
-    Y_SHAPE(30, 14, 16), Y_SHAPE(28, 16, 16), Y_SHAPE(35, 14, 8), Y_SHAPE(28, 18, 8),
+    Y_SPLIT(30, 14, 16), Y_SHAPE(28, 16, 16), Y_SHAPE(35, 14, 8), Y_SHAPE(28, 18, 8),
 };
 
 // candidate `cand` of the table entries that `match`
