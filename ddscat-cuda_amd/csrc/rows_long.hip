@@ -8,8 +8,8 @@
 namespace ddhip {
 #define X_BOTH(R1, R2) X_FWD(R1, R2, 16), X_INV(R1, R2, 16, 2, true, false)
 static const RowShape kShapes[] = {
-    X_BOTH(18, 15), X_BOTH(18, 16), X_BOTH(20, 15), X_BOTH(20, 16), X_BOTH(18, 18), X_BOTH(20, 18), X_BOTH(24, 16),
-    X_BOTH(20, 20), X_BOTH(24, 18), X_BOTH(25, 18), X_BOTH(24, 20), X_BOTH(27, 18), X_FWD(25, 20, 16),
+    X_BOTH(18, 15), X_FWD(18, 16, 16), X_BOTH(20, 15), X_FWD(20, 16, 16), X_BOTH(18, 18), X_BOTH(20, 18),
+    X_BOTH(16, 24), X_BOTH(20, 20), X_BOTH(24, 18), X_BOTH(25, 18), X_BOTH(32, 15), X_BOTH(27, 18), X_FWD(25, 20, 16),
     X_FWD(32, 16, 16), X_BOTH(27, 20), X_BOTH(24, 24), X_BOTH(25, 24), X_BOTH(32, 20), X_BOTH(27, 24), X_BOTH(30, 24),
     X_BOTH(30, 25), X_BOTH(32, 24),
     // a factor 7
@@ -18,6 +18,10 @@ static const RowShape kShapes[] = {
     // 512 points: 32 rows, 256 bytes of a1 per kx (256^3: 506 us against 551 with 16 rows)
     X_INV(32, 16, 32, 2, true, false), X_INV(32, 16, 16, 2, true, false), X_INV(32, 24, 16, 4, true, false),
     X_INV(25, 20, 16, 2, false, false),
+    // 16 lanes along x: the finish reads and writes whole 128-byte lines, and
+    // 16 x 18 took 144^3 from 531 to 500 us against 18 x 16, 16 x 20 160^3 from 720
+    // to 691 against 20 x 16 (pass 1, which only reads x, is the same either way)
+    X_INV(16, 18, 16, 2, true, false), X_INV(16, 20, 16, 2, true, false),
 };
 const RowShape* row_shapes_long(int& n) {
   n = (int)(sizeof(kShapes) / sizeof(kShapes[0]));

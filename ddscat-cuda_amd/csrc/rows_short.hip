@@ -1,7 +1,10 @@
 // x-pass shapes for padded x axes of 24 to 256 points (rows.hpp): two-level
 // register transforms, R1 lanes per row, at most 18 to 25 values per lane.
 // 32 rows per workgroup where R1 is small (workgroups of 128 threads and
-// more), 16 rows (one 128-byte line of a1 per kx) otherwise.
+// more), 16 rows (one 128-byte line of a1 per kx) otherwise.  16 lanes where
+// 16 divides the length, so that the finish of pass 5 touches whole 128-byte
+// lines of the vectors: 8 right-hand sides of 48 x 96 x 96 553 -> 533 us with 16 x 6
+// in place of 12 x 8, 40 x 80 x 80 340 -> 333 (16 x 5, 10 x 8), 72^3 506 -> 500.
 #include "rows.hpp"
 
 namespace ddhip {
@@ -9,8 +12,8 @@ namespace ddhip {
 static const RowShape kShapes[] = {
     X_BOTH(6, 4, 32),   X_BOTH(6, 5, 32),   X_BOTH(4, 8, 32),   X_BOTH(6, 6, 32),   X_BOTH(8, 5, 32),
     X_BOTH(8, 6, 32),   X_BOTH(10, 5, 32),  X_BOTH(9, 6, 32),   X_BOTH(10, 6, 32),  X_BOTH(8, 8, 32),
-    X_BOTH(12, 6, 16),  X_BOTH(10, 8, 16),  X_BOTH(10, 9, 16),  X_BOTH(12, 8, 16),  X_BOTH(10, 10, 16),
-    X_BOTH(12, 9, 16),  X_BOTH(12, 10, 16), X_BOTH(16, 8, 16),  X_BOTH(12, 12, 16), X_BOTH(15, 10, 16),
+    X_BOTH(12, 6, 16),  X_BOTH(16, 5, 16),  X_BOTH(10, 9, 16),  X_BOTH(16, 6, 16),  X_BOTH(10, 10, 16),
+    X_BOTH(12, 9, 16),  X_BOTH(12, 10, 16), X_BOTH(16, 8, 16),  X_BOTH(16, 9, 16),  X_BOTH(15, 10, 16),
     X_BOTH(16, 10, 16), X_BOTH(18, 9, 16),  X_BOTH(15, 12, 16), X_BOTH(16, 12, 16), X_FWD(20, 10, 16),
     X_FWD(18, 12, 16),  X_BOTH(16, 15, 16), X_FWD(25, 10, 16),  X_BOTH(16, 16, 16),
     // a factor 7
