@@ -7,14 +7,15 @@
 // columns of a wave are loaded, transformed and stored independently of every
 // other wave, so memory, LDS and VALU phases of different waves overlap.
 //
-// What bounds it: at 256 points (128^3) VALU issue, about 80 us of the pass's
-// 122 us if it ran alone; at 512 and 768 points LDS exchanges and the VALU in
-// about equal parts.  Measured against the kernels this one replaced, which
-// walked z with the plane stride and synchronised 256- to 768-thread
-// workgroups at every exchange (bytes: a2 in and out and the octant once):
-//   128^3, 256 points: 148 -> 122 us (4.1 TB/s)
-//   256^3, 512 points: 1,830 -> 1,130 us (3.6 TB/s)
-//   384^3, 768 points: 7,700 -> 4,520 us (3.0 TB/s)
+// What bounds it: VALU issue, 60 % of the cycles at 256 points (128^3), 76 % at
+// 512 and 98 % at 768, where the power limit also holds the clock at 1.7 GHz;
+// 95 % of the instructions are FP32 arithmetic.  Measured against the kernels
+// this one replaced, which walked z with the plane stride and synchronised
+// 256- to 768-thread workgroups at every exchange (bytes: a2 in and out and the
+// octant once):
+//   128^3, 256 points: 148 -> 125 us (4.1 TB/s)
+//   256^3, 512 points: 1,830 -> 1,078 us (3.75 TB/s)
+//   384^3, 768 points: 7,700 -> 4,150 us (3.3 TB/s)
 #pragma once
 #include "fft_wave.hpp"
 #include "mv_device.hpp"
