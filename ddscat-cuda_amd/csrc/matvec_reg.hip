@@ -243,14 +243,18 @@ struct YShape {
 // that gained a percent or more of a MATVEC: 192^3 1,249 -> 1,165 us, 200^3
 // 1,536 -> 1,413, 216^3 1,974 -> 1,809, 240^3 2,582 -> 2,520, 144^3 539 -> 529,
 // 162^3 827 -> 811 (96^3 to 140^3: 0 to 2 % slower, 250^3 2,825 and 2,984).
+// 32 columns where z runs are often no whole lines long and 16 columns then
+// straddle two (144, 150 and 180 points: 8 right-hand sides of 64 x 72 x 72 445 ->
+// 436 us, 64 x 75 x 64 377 -> 369, 64 x 90 x 72 535 -> 529; 120, 160 and 192 points
+// within a percent either way).
 // Lengths of other sizes use the LDS-staged kernels (the y passes of a 70^3
 // grid: 34 us each against 14 to 16 here, 196^3: 470 against 213 to 235).
 static const YShape kYShapes[] = {
     Y_SHAPE(6, 4, 32), Y_SHAPE(6, 5, 32), Y_SHAPE(4, 8, 64), Y_SHAPE(6, 6, 32), Y_SHAPE(8, 5, 32), Y_SHAPE(8, 6, 32),
     Y_SHAPE(10, 5, 32), Y_SHAPE(9, 6, 32), Y_SHAPE(10, 6, 32), Y_SHAPE(8, 8, 32), Y_SHAPE(12, 6, 16),
     Y_SHAPE(10, 8, 32), Y_SHAPE(10, 9, 32), Y_SHAPE(12, 8, 16), Y_SHAPE(10, 10, 32), Y_SHAPE(12, 9, 16),
-    Y_SHAPE(12, 10, 16), Y_SHAPE(8, 16, 32), Y_SHAPE(12, 12, 16), Y_SHAPE(15, 10, 16), Y_SHAPE(16, 10, 16),
-    Y_SHAPE(18, 9, 16), Y_SHAPE(15, 12, 16), Y_SHAPE(16, 12, 16), Y_SHAPE(20, 10, 16), Y_SHAPE(18, 12, 16),
+    Y_SHAPE(12, 10, 16), Y_SHAPE(8, 16, 32), Y_SHAPE(12, 12, 32), Y_SHAPE(15, 10, 32), Y_SHAPE(16, 10, 16),
+    Y_SHAPE(18, 9, 16), Y_SHAPE(15, 12, 32), Y_SHAPE(16, 12, 16), Y_SHAPE(20, 10, 16), Y_SHAPE(18, 12, 16),
     Y_SHAPE(16, 15, 16), Y_SHAPE(25, 10, 16), Y_SHAPE(16, 16, 32), Y_SHAPE(18, 15, 16), Y_SPLIT(18, 16, 16),
     Y_SHAPE(20, 15, 16), Y_SHAPE(20, 16, 16), Y_SPLIT(18, 18, 16), Y_SHAPE(20, 18, 16), Y_SPLIT(24, 16, 16),
     Y_SPLIT(20, 20, 16), Y_SPLIT(24, 18, 16), Y_SPLIT(25, 18, 16), Y_SPLIT(24, 20, 16), Y_SHAPE(27, 18, 16),
