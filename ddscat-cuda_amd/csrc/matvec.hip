@@ -474,7 +474,7 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
 
 void matvec_support(const Context& c, int layout, BatchArgs& k) {
   const MatvecPlan& m = c.mv;
-  const bool reg = !c.fft_generic && !m.plane && m.kind[1] >= 0 && m.kind[2] >= 0 && m.kind[4] >= 0 && m.kind[5] >= 0;
+  const bool reg = !c.fft_generic && !plane_yz_runs(c) && m.kind[1] >= 0 && m.kind[2] >= 0 && m.kind[4] >= 0 && m.kind[5] >= 0;
   k.ysup = layout && reg ? c.ysup : nullptr;
   k.zsh = m.zsh;
 }
@@ -490,7 +490,7 @@ int matvec_launch(Context& c, int cwhat, const float2* x, float2* y, const float
   bt.slab = KxSlab{0, c.nx, c.mv.gx};
   for (int p = 1; p <= 5; ++p) {
     if (ev) hipEventRecord(ev[p - 1], st);
-    if (c.mv.plane && p >= 2 && p <= 4) {
+    if (plane_yz_runs(c) && p >= 2 && p <= 4) {
       if (p != 3) continue;
       if (int rc = plane_yz_launch(c, st, bt)) return rc;
       continue;

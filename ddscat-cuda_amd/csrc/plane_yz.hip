@@ -47,7 +47,7 @@ static size_t lds_bytes(const MatvecPlan& m, const YzShape* z) {
 int plane_yz_setup(Context& c) {
   c.mv.plane = 0;
   const YzShape* z = z_shape(c.mv.gz);
-  if (c.fft_generic || !z || !y_split(c.mv.gy)) return 0;
+  if (!z || !y_split(c.mv.gy)) return 0;
   const size_t lds = lds_bytes(c.mv, z);
   const int planes = c.mv.gx;
   if (lds > YZ_LDS || planes < (lds <= 80 * 1024 ? 0 : lds <= 104 * 1024 ? 32 : 96)) return 0;

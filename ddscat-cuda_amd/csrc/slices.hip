@@ -83,7 +83,7 @@ int slices_matvec(Context& c, int cwhat, const float2* x, float2* y, const float
   bt.k.active = act;
   matvec_support(c, layout, bt.k);
   if (int rc = matvec_end_pass(c, 1, cwhat, x, y, adia, aoff, layout, st, bt)) return rc;
-  if (c.mv.plane) {
+  if (plane_yz_runs(c)) {
     if (int rc = plane_yz_launch(c, st, bt)) return rc;
   } else if (s.nslab == 1) {
     slices_slab(c, 0, bt);

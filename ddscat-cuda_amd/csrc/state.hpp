@@ -174,6 +174,8 @@ void slices_slab(const Context& c, int h0, MvBatch& bt);
 // the plane kernel in place of passes 2 to 4, in place on every plane of bt.a1:
 // whether the prepared grid takes it (c.mv.plane), and its launch
 int plane_yz_setup(Context& c);
+// whether it runs now: the LDS-staged family can be chosen on a prepared target
+inline bool plane_yz_runs(const Context& c) { return c.mv.plane && !c.fft_generic; }
 int plane_yz_launch(Context& c, hipStream_t st, const MvBatch& bt);
 // pass 1 (x -> a1) or 5 (a1 -> y) alone
 int matvec_end_pass(Context& c, int which, int cwhat, const float2* x, float2* y, const float2* adia,

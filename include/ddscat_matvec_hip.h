@@ -361,8 +361,9 @@ DDSCAT_HIP_API int ddscat_hip_get_green(void *out);
 /* Fill up to n int64 fields: nx ny nz nat nat0 green_count matvec_count
  * backend precision gx gy gz rx_fwd cy cz rx_inv green_build_us, then the FFT
  * kernel of passes 1..5 (-1 LDS-staged, k >= 0 register shape k of the axis
- * length), whether the autotuner chose them, and the reliable-residual
- * restarts of the last single-RHS solve. */
+ * length), whether the autotuner chose them, the reliable-residual restarts of
+ * the last single-RHS solve, and whether one kernel runs passes 2 to 4 on whole
+ * kx planes in LDS in place of the kernels given for them. */
 DDSCAT_HIP_API int ddscat_hip_info(long long *out, int n);
 
 /* Run `reps` MATVECs on device pointers with HIP events between the five
