@@ -92,14 +92,17 @@ void release_context(Context& c) {
 // The occupied iy range of each run of 1 << zsh lattice planes iz, the planes
 // that share a half or whole 128-byte line of a1.  Worth a table where it
 // leaves out a thirty-second of the rows (an ellipsoid: a fifth) of an a1 that
-// does not fit the 256 MiB in front of HBM, and where the y passes are those
-// of 512 and 768 points (MATVECs of ellipsoids: 256^3 2,660 -> 2,570 us, SLICES
-// 2,665 -> 2,590, 384^3 9,435 -> 9,120).  The shorter two-level kernels had
-// less to gain: 160^3 720 without and 730 with, 200^3 1,461 and 1,448.
+// does not fit the 256 MiB in front of HBM, and where the kernels of the y
+// passes honour it, those of 512 and 768 points (MATVECs of ellipsoids: 256^3
+// 2,660 -> 2,570 us, SLICES 2,665 -> 2,590, 384^3 9,435 -> 9,120).  The
+// two-level y kernels of the other lengths do not: with a support test on every
+// load and store they lost on ellipsoids of every size tried, 200^3 1,353 ->
+// 1,392 us, 250^3 2,746 -> 3,057, 270^3 3,546 -> 4,068, 300^3 4,847 -> 5,347, 320^3
+// 6,262 -> 6,595, 360^3 8,635 -> 9,949, 375^3 12,624 -> 14,159.
 constexpr size_t SUPPORT_MIN_A1 = (size_t)256 << 20;
 static int upload_support(Context& c, const std::vector<int>& rowptr, int code) {
   c.mv.zsh = c.mv.nzp % 16 == 0 ? 4 : 3;
-  if (c.mv.nzp % 8 || (c.mv.gy != 512 && c.mv.gy != 768) || matvec_a1_count(c) * sizeof(float2) < SUPPORT_MIN_A1) return 0;
+  if (c.mv.nzp % 8 || !reg_row_support(c.mv.gy, 0) || matvec_a1_count(c) * sizeof(float2) < SUPPORT_MIN_A1) return 0;
   const int zt = 1 << c.mv.zsh, runs = c.mv.nzp / zt;
   std::vector<int2> sup((size_t)runs);
   long long rows = 0;

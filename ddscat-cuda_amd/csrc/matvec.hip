@@ -474,8 +474,9 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
 
 void matvec_support(const Context& c, int layout, BatchArgs& k) {
   const MatvecPlan& m = c.mv;
-  const bool reg = !c.fft_generic && !plane_yz_runs(c) && m.kind[1] >= 0 && m.kind[2] >= 0 && m.kind[4] >= 0 && m.kind[5] >= 0;
-  k.ysup = layout && reg ? c.ysup : nullptr;
+  const bool honoured = !c.fft_generic && !plane_yz_runs(c) && m.kind[1] >= 0 && m.kind[5] >= 0 &&
+                        reg_row_support(m.gy, m.kind[2]) && reg_row_support(m.gy, m.kind[4]);
+  k.ysup = layout && honoured ? c.ysup : nullptr;
   k.zsh = m.zsh;
 }
 

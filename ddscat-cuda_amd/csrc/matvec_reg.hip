@@ -232,6 +232,7 @@ static void launch_y_m(Context& c, int dir, const MvBatch& bt, hipStream_t st) {
 struct YShape {
   int L;
   void (*fn)(Context&, int, const MvBatch&, hipStream_t);
+  bool sup = false;  // the kernel honours BatchArgs::ysup
 };
 #define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>}
 #define Y_SPLIT(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C, true>}
@@ -258,8 +259,8 @@ static const YShape kYShapes[] = {
     Y_SHAPE(16, 15, 16), Y_SHAPE(25, 10, 16), Y_SHAPE(16, 16, 32), Y_SHAPE(18, 15, 16), Y_SPLIT(18, 16, 16),
     Y_SHAPE(20, 15, 16), Y_SHAPE(20, 16, 16), Y_SPLIT(18, 18, 16), Y_SHAPE(20, 18, 16), Y_SPLIT(24, 16, 16),
     Y_SPLIT(20, 20, 16), Y_SPLIT(24, 18, 16), Y_SPLIT(25, 18, 16), Y_SPLIT(24, 20, 16), Y_SHAPE(27, 18, 16),
-    Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
-    Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>},
+    Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>, true}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
+    Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>, true},
     // a factor 7
     Y_SHAPE(7, 4, 32), Y_SHAPE(7, 6, 32), Y_SHAPE(8, 7, 32), Y_SHAPE(10, 7, 32), Y_SHAPE(12, 7, 16),
     Y_SHAPE(14, 7, 16), Y_SHAPE(14, 8, 16), Y_SHAPE(14, 9, 16), Y_SHAPE(14, 10, 16), Y_SHAPE(14, 12, 16),
@@ -287,6 +288,11 @@ static const P3Shape* p3_shape(int L, int cand) {
 }
 static const YShape* y_shape(int L, int cand) {
   return nth(kYShapes, (int)(sizeof(kYShapes) / sizeof(kYShapes[0])), cand, [=](const YShape& r) { return r.L == L; });
+}
+
+bool reg_row_support(int L, int cand) {
+  const YShape* y = cand < 0 ? nullptr : y_shape(L, cand);
+  return y && y->sup;
 }
 
 int reg_candidates(int L, int which) {

@@ -164,6 +164,8 @@ size_t matvec_a1_count(const Context& c);
 size_t matvec_a2_count(const Context& c);
 // register-FFT shapes available for pass `which` (1..5) on a padded axis length (0: none)
 int reg_candidates(int L, int which);
+// whether y-pass shape `cand` of a padded length leaves the rows outside the row support alone
+bool reg_row_support(int L, int cand);
 // register-FFT pass `which` (1..5) with shape `cand` of its axis length; 1 = launched
 int reg_pass(Context& c, int which, int cand, int cj, int compact, const float2* x, float2* y, const float2* adia,
              const float2* aoff, hipStream_t st, const MvBatch& bt);

@@ -42,7 +42,7 @@ SOLVER_IDS = {"pbcgs2": 0, "qmrccg": 1, "petrkp": 2, "gpbicg": 3, "pbcgst": 4, "
 INFO_FIELDS = ("nx", "ny", "nz", "nat", "nat0", "green_count", "matvec_count", "backend", "precision",
                "gx", "gy", "gz", "rx_fwd", "cy", "cz", "rx_inv", "green_build_us",
                "kernel_pass1", "kernel_pass2", "kernel_pass3", "kernel_pass4", "kernel_pass5", "autotuned",
-               "restarts", "plane_kernel")
+               "restarts", "plane_kernel", "row_support")
 
 BACKEND_FFT3D, BACKEND_SLICES = 0, 1
 PREC_MIXED, PREC_FP32 = 0, 1

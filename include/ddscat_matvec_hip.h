@@ -362,8 +362,9 @@ DDSCAT_HIP_API int ddscat_hip_get_green(void *out);
  * backend precision gx gy gz rx_fwd cy cz rx_inv green_build_us, then the FFT
  * kernel of passes 1..5 (-1 LDS-staged, k >= 0 register shape k of the axis
  * length), whether the autotuner chose them, the reliable-residual restarts of
- * the last single-RHS solve, and whether one kernel runs passes 2 to 4 on whole
- * kx planes in LDS in place of the kernels given for them. */
+ * the last single-RHS solve, whether one kernel runs passes 2 to 4 on whole
+ * kx planes in LDS in place of the kernels given for them, and whether MATVECs
+ * on compact vectors leave out the lattice rows outside the target (row support). */
 DDSCAT_HIP_API int ddscat_hip_info(long long *out, int n);
 
 /* Run `reps` MATVECs on device pointers with HIP events between the five
