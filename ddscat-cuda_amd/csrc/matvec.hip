@@ -39,6 +39,13 @@ static constexpr int PER_NARROW = 8;  // passes 3, 5 (three components in LDS)
 // rows of 8-16 columns.
 static constexpr int WIDE_THREADS = 1024;
 
+// x / d as a multiplication, exact for x d < 2^32
+struct FastDiv {
+  unsigned m;  // ceil(2^32 / d); 0 for d = 1
+};
+static FastDiv fast_div_by(int d) { return FastDiv{(unsigned)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d)}; }
+__device__ __forceinline__ int fast_div(int x, FastDiv d) { return d.m ? (int)__umulhi((unsigned)x, d.m) : x; }
+
 // ---------------------------------------------------------------- pass 1 --
 // rows q = iy NZ + iz, rx of them per workgroup, so that the transposed store
 // writes runs of consecutive z; rows sit in LDS at stride L + 1
@@ -121,49 +128,66 @@ __global__ __launch_bounds__(NT) void k_pass_y(
 }
 
 // ---------------------------------------------------------------- pass 3 --
-// cz contiguous z columns (slot 2NY + ky) per workgroup, each at stride L + 1 in LDS
+// cz contiguous z columns (slot 2NY + ky) per workgroup, interleaved in LDS at
+// an odd pitch cp: global memory and the Green row are walked with lanes over z,
+// the butterflies with lanes over the columns, and neither conflicts.  cz fills
+// the workgroup also where L is short.  Whole MATVECs against columns one after
+// another in LDS, at most 16 of them: 128 x 128 x 1 92 -> 44 us, 128 x 128 x 10
+// 117 -> 65, 48 x 48 x 280 305 -> 237, 48 x 48 x 1,024 1,053 -> 789.
 template <int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass3_z_green(
     float2* __restrict__ a2, const float2* __restrict__ green, const float2* __restrict__ twg,
-    FftPlan p, int nz, int nzp, int p2, KxSlab sl, int gy, int cz, BatchArgs ba, GreenGeo gg) {
+    FftPlan p, int nz, int nzp, int p2, KxSlab sl, int gy, int cz, FastDiv dz, FastDiv dl, FastDiv dy, BatchArgs ba,
+    GreenGeo gg) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z;
   if (ba.active && !ba.active[rb]) return;
   a2 += rb * ba.a2s;
-  const int L = p.L, LP = cz > 1 ? L + 1 : L;  // L = 2 nz
+  const int L = p.L, cp = cz | 1;  // L = 2 nz
   float2* tw = sm;
   float2* b0 = sm + L;
-  float2* b1 = b0 + LP * cz;
-  float2* b2 = b1 + LP * cz;
+  float2* b1 = b0 + cp * L;
+  float2* b2 = b1 + cp * L;
   const int ncol = 2 * sl.H * gy, q0 = blockIdx.x * cz, nc = min(cz, ncol - q0);
+  const int slot0 = q0 / gy, ky0 = q0 - slot0 * gy;
   const int T = blockDim.x;
   const size_t cstride = (size_t)(2 * sl.H) * p2;
-  const auto column = [&](int r) {
-    const int slot = (q0 + r) / gy;
-    return (size_t)slot * p2 + (size_t)(q0 + r - slot * gy) * nzp;
+  const auto column = [&](int r, int& slot, int& ky) {
+    const int d = fast_div(ky0 + r, dy);
+    slot = slot0 + d;
+    ky = ky0 + r - d * gy;
+  };
+  const auto address = [&](int r) {
+    int slot, ky;
+    column(r, slot, ky);
+    return (size_t)slot * p2 + (size_t)ky * nzp;
   };
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  for (int idx = threadIdx.x; idx < L * cz; idx += T) {
-    const int r = idx / L, e = idx - r * L;
-    float2 v0 = make_float2(0.f, 0.f), v1 = v0, v2 = v0;
-    if (e < nz && r < nc) {
-      const size_t o = column(r) + e;
+  for (int idx = threadIdx.x; idx < nz * cz; idx += T) {
+    const int r = fast_div(idx, dz), e = idx - r * nz;
+    const float2 z = make_float2(0.f, 0.f);
+    float2 v0 = z, v1 = z, v2 = z;
+    if (r < nc) {
+      const size_t o = address(r) + e;
       v0 = a2[o];
       v1 = a2[o + cstride];
       v2 = a2[o + 2 * cstride];
     }
-    const int li = r * LP + e;
+    const int li = e * cp + r, lu = li + nz * cp;
     b0[li] = v0; b1[li] = v1; b2[li] = v2;
+    b0[lu] = z; b1[lu] = z; b2[lu] = z;
   }
   __syncthreads();
-  fft_run<+1, false, PER>(b0, tw, p, cz, 1, LP);
-  fft_run<+1, false, PER>(b1, tw, p, cz, 1, LP);
-  fft_run<+1, false, PER>(b2, tw, p, cz, 1, LP);
+  fft_run<+1, true, PER>(b0, tw, p, cz, cp, 1);
+  fft_run<+1, true, PER>(b1, tw, p, cz, cp, 1);
+  fft_run<+1, true, PER>(b2, tw, p, cz, cp, 1);
   // symmetric 3x3 multiply; trimmed-octant reconstruction for IPBC=0
   // (cu:109-115), whole grid for IPBC=1
   for (int idx = threadIdx.x; idx < L * nc; idx += T) {
-    const int r = idx / L, kz = idx - r * L;
-    const int slot = (q0 + r) / gy, kx = sl.kx(slot), ky = q0 + r - slot * gy;
+    const int r = fast_div(idx, dl), kz = idx - r * L;
+    int slot, ky;
+    column(r, slot, ky);
+    const int kx = sl.kx(slot);
     const int ir = min(kx, gg.mx - kx), jr = min(ky, gg.my - ky), kr = min(kz, gg.mz - kz);
     const float sx = kx <= gg.tx ? 1.f : -1.f, sy = ky <= gg.ty ? 1.f : -1.f;
     const float sz = kz <= gg.tz ? 1.f : -1.f;
@@ -171,20 +195,20 @@ __global__ __launch_bounds__(NT) void k_pass3_z_green(
     const float2 g12 = cscale(G.xy, sx * sy);
     const float2 g13 = cscale(G.xz, sx * sz);
     const float2 g23 = cscale(G.yz, sy * sz);
-    const int li = r * LP + kz;
+    const int li = kz * cp + r;
     const float2 p0 = b0[li], p1 = b1[li], p2 = b2[li];
     b0[li] = cadd(cadd(cmul(G.xx, p0), cmul(g12, p1)), cmul(g13, p2));
     b1[li] = cadd(cadd(cmul(g12, p0), cmul(G.yy, p1)), cmul(g23, p2));
     b2[li] = cadd(cadd(cmul(g13, p0), cmul(g23, p1)), cmul(G.zz, p2));
   }
   __syncthreads();
-  fft_run<-1, false, PER>(b0, tw, p, cz, 1, LP);
-  fft_run<-1, false, PER>(b1, tw, p, cz, 1, LP);
-  fft_run<-1, false, PER>(b2, tw, p, cz, 1, LP);
+  fft_run<-1, true, PER>(b0, tw, p, cz, cp, 1);
+  fft_run<-1, true, PER>(b1, tw, p, cz, cp, 1);
+  fft_run<-1, true, PER>(b2, tw, p, cz, cp, 1);
   for (int idx = threadIdx.x; idx < nz * nc; idx += T) {
-    const int r = idx / nz, e = idx - r * nz;
-    const size_t o = column(r) + e;
-    const int li = r * LP + e;
+    const int r = fast_div(idx, dz), e = idx - r * nz;
+    const size_t o = address(r) + e;
+    const int li = e * cp + r;
     a2[o] = b0[li];
     a2[o + cstride] = b1[li];
     a2[o + 2 * cstride] = b2[li];
@@ -358,7 +382,14 @@ int matvec_plan(Context& c, const char* name) {
   m.rx_inv = std::max(1, narrow / m.gx);
   while (m.rx_inv > 1 && (size_t)((nrows + m.rx_inv - 1) / m.rx_inv) < 1024) m.rx_inv /= 2;
   m.cy = std::min(16, pow2floor(std::max(1, wide / m.gy)));
-  m.cz = std::min(16, pow2floor(std::max(1, narrow / m.gz)));
+  // columns of the LDS-staged Green pass: as many as the workgroup has room for
+  // (8 values a thread) in 1,024 workgroups or more, but at least 4 columns and
+  // an element for every thread
+  const auto green_columns = [&](int elements) {
+    const int ncol = m.gx * m.gy, least = std::max(4, (MV_THREADS + m.gz - 1) / m.gz);
+    return std::max(1, std::min(elements / m.gz, std::max(least, ncol / 1024)));
+  };
+  m.cz = green_columns(narrow);
   m.ty = m.tz = MV_THREADS;
   const size_t lds_max = lds_limit();
   if (m.cy < 8) {
@@ -367,8 +398,8 @@ int matvec_plan(Context& c, const char* name) {
     if (cw > m.cy) { m.cy = cw; m.ty = WIDE_THREADS; }
   }
   if (m.cz < 8) {
-    int cw = std::min(16, pow2floor(std::max(1, PER_NARROW * WIDE_THREADS / m.gz)));
-    while (cw > 1 && (size_t)(m.gz + 3 * cw * (m.gz + 1)) * sizeof(float2) > lds_max) cw /= 2;
+    int cw = green_columns(PER_NARROW * WIDE_THREADS);
+    while (cw > 1 && (size_t)(m.gz + 3 * (cw | 1) * m.gz) * sizeof(float2) > lds_max) --cw;
     if (cw > m.cz) { m.cz = cw; m.tz = WIDE_THREADS; }
   }
   if ((m.ty == WIDE_THREADS || m.tz == WIDE_THREADS) && allow_big_lds(lds_max)) return 206;
@@ -448,13 +479,14 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
     }
     case 3: {
       dim3 grid((2 * bt.slab.H * m.gy + m.cz - 1) / m.cz, 1, nb);
-      const size_t lds = (size_t)(m.gz + 3 * m.cz * (m.gz + (m.cz > 1))) * sizeof(float2);
+      const size_t lds = (size_t)(m.gz + 3 * (m.cz | 1) * m.gz) * sizeof(float2);
+      const FastDiv dz = fast_div_by(c.nz), dl = fast_div_by(m.gz), dy = fast_div_by(m.gy);
       if (m.tz == WIDE_THREADS)
         hipLaunchKernelGGL((k_pass3_z_green<PER_NARROW, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2,
-                           c.green, m.twz, m.pz, c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, bt.k, green_geo(c));
+                           c.green, m.twz, m.pz, c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, dz, dl, dy, bt.k, green_geo(c));
       else
         hipLaunchKernelGGL(k_pass3_z_green<PER_NARROW>, grid, dim3(MV_THREADS), lds, st, a2, c.green, m.twz, m.pz,
-                           c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, bt.k, green_geo(c));
+                           c.nz, m.nzp, m.p2, bt.slab, m.gy, m.cz, dz, dl, dy, bt.k, green_geo(c));
       DDH_LAUNCH_OK("MATVEC pass 3 (z FFT + Green)", 23);
       break;
     }
