@@ -231,8 +231,8 @@ extern "C" DDSCAT_HIP_API int ddscat_hip_info(long long* out, int n) {
   BatchArgs support;
   if (c.ready) matvec_support(c, 1, support);
   const long long v[] = {c.nx, c.ny, c.nz, c.nat, c.nat0, (long long)c.green_count, (long long)c.matvec_count,
-                         c.backend, c.precision, c.mv.gx, c.mv.gy, c.mv.gz, c.mv.rx_fwd, c.mv.cy, c.mv.cz,
-                         c.mv.rx_inv, (long long)(c.green_build_ms * 1000.0), c.mv.kind[1], c.mv.kind[2],
+                         c.backend, c.precision, c.mv.gx, c.mv.gy, c.mv.gz, c.mv.rx, c.mv.cy, c.mv.cz,
+                         c.mv.rx, (long long)(c.green_build_ms * 1000.0), c.mv.kind[1], c.mv.kind[2],
                          c.mv.kind[3], c.mv.kind[4], c.mv.kind[5], c.mv.tuned, c.restarts, plane_yz_runs(c),
                          support.ysup != nullptr};
   const int m = (int)(sizeof(v) / sizeof(v[0]));

@@ -31,13 +31,15 @@
 namespace ddhip {
 
 static constexpr int MV_THREADS = 256;
-static constexpr int PER_WIDE = 16;   // passes 1, 2, 4
-static constexpr int PER_NARROW = 8;  // passes 3, 5 (three components in LDS)
+static constexpr int PER_WIDE = 16;   // passes 2, 4
+static constexpr int PER_NARROW = 8;  // passes 1, 5, and 3 (three components in LDS)
 // Wide tiles: long axes (a 256-thread tile would hold fewer than 8 columns,
 // i.e. rows of < 64 contiguous bytes) run passes 2-4 with 1024-thread
 // workgroups and up to the device's per-workgroup LDS, so each tile reads
-// rows of 8-16 columns.
+// rows of 8-16 columns; passes 1 and 5 with 512 threads and half the LDS, two
+// workgroups to a CU (with 1024 and all of it, 450 x 48 x 48 took 234 us, not 218).
 static constexpr int WIDE_THREADS = 1024;
+static constexpr int ROW_THREADS = 512;
 
 // x / d as a multiplication, exact for x d < 2^32
 struct FastDiv {
@@ -46,45 +48,76 @@ struct FastDiv {
 static FastDiv fast_div_by(int d) { return FastDiv{(unsigned)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d)}; }
 __device__ __forceinline__ int fast_div(int x, FastDiv d) { return d.m ? (int)__umulhi((unsigned)x, d.m) : x; }
 
+// tile of block bx of n: the blocks of one XCD (ids 8 apart) take neighbours,
+// whose pieces of a 128-byte line then meet in that XCD's L2
+__device__ __forceinline__ int xcd_run(int bx, int n) {
+  const int x = bx & 7, q = n >> 3, rem = n & 7;
+  return x * q + min(x, rem) + (bx >> 3);
+}
+
+// The x passes: rows q = iy NZ + iz, rx of them per workgroup, interleaved in
+// LDS at an odd pitch, so that the vectors are walked with lanes over x and the
+// work arrays with lanes over the rows (runs of consecutive z), without
+// conflicts.  MATVECs, rows one after another in LDS and often 1 to 5 of them
+// before: 280 x 48 x 48 193 -> 138 us, 512 x 96 x 96 1,204 -> 984, 400 x 128 x 128
+// 1,607 -> 1,327, 1,024 x 64 x 64 1,407 -> 945, 5 x 128 x 128 with four right-hand
+// sides 214 -> 86.
+struct RowTile {
+  int rx, nr, iy0, z0, nz;  // rows per workgroup, rows of this one, and where it starts
+  FastDiv dz, dr;           // by nz and rx
+  __device__ __forceinline__ void row(int r, int& iy, int& iz) const {
+    const int d = fast_div(z0 + r, dz);
+    iy = iy0 + d;
+    iz = z0 + r - d * nz;
+  }
+};
+__device__ __forceinline__ RowTile row_tile(int rx, int ny, int nz, FastDiv dz, FastDiv dr) {
+  const int q0 = xcd_run((int)blockIdx.x, (int)gridDim.x) * rx, iy0 = q0 / nz;
+  return RowTile{rx, min(rx, ny * nz - q0), iy0, q0 - iy0 * nz, nz, dz, dr};
+}
+
 // ---------------------------------------------------------------- pass 1 --
-// rows q = iy NZ + iz, rx of them per workgroup, so that the transposed store
-// writes runs of consecutive z; rows sit in LDS at stride L + 1
-template <int PER>
-__global__ __launch_bounds__(MV_THREADS) void k_pass1_xfwd(
+template <int PER, int NT = MV_THREADS>
+__global__ __launch_bounds__(NT) void k_pass1_xfwd(
     const float2* __restrict__ x, float2* __restrict__ a1, SiteMap map, const float2* __restrict__ twg, FftPlan p,
-    int nx, int ny, int nz, int nzp, int ks, int rx, int nat, int nat0, int compact, int conj_in, BatchArgs ba) {
+    int nx, int ny, int nz, int nzp, int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int nat, int nat0, int compact,
+    int conj_in, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z;
   if (ba.active && !ba.active[rb]) return;
   x += rb * ba.xs;
   a1 += rb * ba.a1s;
-  const int L = p.L, LP = rx > 1 ? L + 1 : L;
+  const int L = p.L, rp = rx | 1;  // L = 2 nx
   float2* tw = sm;
   float2* buf = sm + L;
   const int c = blockIdx.y;
-  const int q0 = blockIdx.x * rx, nrows = ny * nz;
+  const RowTile t = row_tile(rx, ny, nz, dz, dr);
   const int T = blockDim.x;
-  const int nr = min(rx, nrows - q0);
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
   const float2* xs = x + (size_t)c * (compact ? nat0 : nat);
-  for (int idx = threadIdx.x; idx < rx * L; idx += T) {
-    const int r = idx / L, e = idx - r * L;
+  for (int idx = threadIdx.x; idx < nx * rx; idx += T) {
+    const int r = fast_div(idx, dx), e = idx - r * nx;
     float2 v = make_float2(0.f, 0.f);
-    if (r < nr && e < nx) {
-      const int q = q0 + r, iy = q / nz, g = iy + ny * (q - iy * nz);
+    if (r < t.nr) {
+      int iy, iz;
+      t.row(r, iy, iz);
+      const int g = iy + ny * iz;
       const int o = compact ? compact_index(map, g, e, nx) : g * nx + e;
       if (o >= 0) v = xs[o];
       if (conj_in) v.y = -v.y;
     }
-    buf[r * LP + e] = v;
+    buf[e * rp + r] = v;
+    buf[(e + nx) * rp + r] = make_float2(0.f, 0.f);
   }
   __syncthreads();
-  fft_run<+1, false, PER>(buf, tw, p, rx, 1, LP);
+  fft_run<+1, true, PER>(buf, tw, p, rx, rp, 1);
   float2* out = a1 + (size_t)c * L * ks;
-  for (int idx = threadIdx.x; idx < nr * L; idx += T) {
-    const int k = idx / nr, r = idx - k * nr;
-    const int q = q0 + r, iy = q / nz, iz = q - iy * nz;
-    out[(size_t)k * ks + (size_t)iy * nzp + iz] = buf[r * LP + k];
+  for (int idx = threadIdx.x; idx < rx * L; idx += T) {
+    const int k = fast_div(idx, t.dr), r = idx - k * rx;
+    if (r >= t.nr) continue;
+    int iy, iz;
+    t.row(r, iy, iz);
+    out[(size_t)k * ks + (size_t)iy * nzp + iz] = buf[k * rp + r];
   }
 }
 
@@ -230,12 +263,15 @@ __device__ __forceinline__ void finish_site(float2 x1, float2 x2, float2 x3, flo
   if (cj) { r1.y = -r1.y; r2.y = -r2.y; r3.y = -r3.y; }
 }
 
-template <int PER>
-__global__ __launch_bounds__(MV_THREADS) void k_pass5_xinv_finish(
+// One component after another in LDS, the kept half of each waiting in registers.
+template <int PER, int NT = MV_THREADS>
+__global__ __launch_bounds__(NT, 4) void k_pass5_xinv_finish(
     const float2* __restrict__ a1, const float2* __restrict__ twg, FftPlan p,
     const float2* __restrict__ x, float2* __restrict__ y, const float2* __restrict__ adia,
     const float2* __restrict__ aoff, const int16_t* __restrict__ iocc, SiteMap map, int nx, int ny, int nz, int nzp,
-    int ks, int rx, int nat, int nat0, int compact, int cj, float inv, BatchArgs ba) {
+    int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int nat, int nat0, int compact, int cj, float inv,
+    BatchArgs ba) {
+  constexpr int KEEP = PER / 2;  // kept outputs per thread and component
   extern __shared__ float2 sm[];
   const int rb = blockIdx.y;
   if (ba.active && !ba.active[rb]) return;
@@ -244,45 +280,52 @@ __global__ __launch_bounds__(MV_THREADS) void k_pass5_xinv_finish(
   y += rb * ba.xs;
   adia += rb * ba.os;
   aoff += rb * ba.os;
-  const int L = p.L, LP = rx > 1 ? L + 1 : L;
+  const int L = p.L, rp = rx | 1;
   float2* tw = sm;
-  float2* b0 = sm + L;
-  float2* b1 = b0 + rx * LP;
-  float2* b2 = b1 + rx * LP;
-  const int q0 = blockIdx.x * rx, nrows = ny * nz;
+  float2* buf = sm + L;
+  const RowTile t = row_tile(rx, ny, nz, dz, dr);
   const int T = blockDim.x;
-  const int nr = min(rx, nrows - q0);
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
   const size_t cs = (size_t)L * ks;
-  for (int idx = threadIdx.x; idx < rx * L; idx += T) {
-    const int k = idx / rx, r = idx - k * rx;
-    float2 v0 = make_float2(0.f, 0.f), v1 = v0, v2 = v0;
-    if (r < nr) {
-      const int q = q0 + r, iy = q / nz, iz = q - iy * nz;
-      const float2* src = a1 + (size_t)k * ks + (size_t)iy * nzp + iz;
-      v0 = src[0]; v1 = src[cs]; v2 = src[2 * cs];
+  float2 w[3][KEEP];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (c) __syncthreads();
+    for (int idx = threadIdx.x; idx < rx * L; idx += T) {
+      const int k = fast_div(idx, t.dr), r = idx - k * rx;
+      float2 v = make_float2(0.f, 0.f);
+      if (r < t.nr) {
+        int iy, iz;
+        t.row(r, iy, iz);
+        v = a1[c * cs + (size_t)k * ks + (size_t)iy * nzp + iz];
+      }
+      buf[k * rp + r] = v;
     }
-    const int li = r * LP + k;
-    b0[li] = v0; b1[li] = v1; b2[li] = v2;
+    __syncthreads();
+    fft_run<-1, true, PER>(buf, tw, p, rx, rp, 1);
+#pragma unroll
+    for (int j = 0; j < KEEP; ++j) {
+      const int idx = threadIdx.x + j * T, r = fast_div(idx, dx), ix = idx - r * nx;
+      w[c][j] = r < rx ? buf[ix * rp + r] : make_float2(0.f, 0.f);
+    }
   }
-  __syncthreads();
-  fft_run<-1, false, PER>(b0, tw, p, rx, 1, LP);
-  fft_run<-1, false, PER>(b1, tw, p, rx, 1, LP);
-  fft_run<-1, false, PER>(b2, tw, p, rx, 1, LP);
   const size_t sd = compact ? (size_t)nat0 : (size_t)nat;
-  for (int idx = threadIdx.x; idx < nr * nx; idx += T) {
-    const int r = idx / nx, ix = idx - r * nx;
-    const int q = q0 + r, iy = q / nz, g = iy + ny * (q - iy * nz);
+#pragma unroll
+  for (int j = 0; j < KEEP; ++j) {
+    const int idx = threadIdx.x + j * T, r = fast_div(idx, dx), ix = idx - r * nx;
+    if (r >= t.nr) continue;
+    int iy, iz;
+    t.row(r, iy, iz);
+    const int g = iy + ny * iz;
     const int o = compact ? compact_index(map, g, ix, nx) : g * nx + ix;
     if (o < 0) continue;
     float2 r1, r2, r3;
     if (iocc && iocc[o] == 0) {
       r1 = r2 = r3 = make_float2(0.f, 0.f);
     } else {
-      const int li = r * LP + ix;
-      const size_t j = (size_t)o;
-      finish_site(x[j], x[j + sd], x[j + 2 * sd], adia[j], adia[j + sd], adia[j + 2 * sd], aoff[j], aoff[j + sd],
-                  aoff[j + 2 * sd], b0[li], b1[li], b2[li], inv, cj != 0, r1, r2, r3);
+      const size_t q = (size_t)o;
+      finish_site(x[q], x[q + sd], x[q + 2 * sd], adia[q], adia[q + sd], adia[q + 2 * sd], aoff[q], aoff[q + sd],
+                  aoff[q + 2 * sd], w[0][j], w[1][j], w[2][j], inv, cj != 0, r1, r2, r3);
     }
     y[o] = r1; y[o + sd] = r2; y[o + 2 * sd] = r3;
   }
@@ -344,17 +387,15 @@ static size_t lds_limit() {
 
 // lets the wide-tile kernels take more than 64 KB of dynamic LDS
 static int allow_big_lds(size_t bytes) {
-  const int b = (int)bytes;
-  const hipError_t e[] = {
-      hipFuncSetAttribute((const void*)k_pass_y<+1, PER_WIDE, WIDE_THREADS>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, b),
-      hipFuncSetAttribute((const void*)k_pass_y<-1, PER_WIDE, WIDE_THREADS>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, b),
-      hipFuncSetAttribute((const void*)k_pass3_z_green<PER_NARROW, WIDE_THREADS>,
-                          hipFuncAttributeMaxDynamicSharedMemorySize, b)};
-  for (hipError_t x : e)
-    if (x != hipSuccess) {
-      set_hip_error("MATVEC plan (wide LDS tiles)", x);
+  const void* const wide[] = {(const void*)k_pass1_xfwd<PER_NARROW, ROW_THREADS>,
+                              (const void*)k_pass5_xinv_finish<PER_NARROW, ROW_THREADS>,
+                              (const void*)k_pass_y<+1, PER_WIDE, WIDE_THREADS>,
+                              (const void*)k_pass_y<-1, PER_WIDE, WIDE_THREADS>,
+                              (const void*)k_pass3_z_green<PER_NARROW, WIDE_THREADS>};
+  for (const void* k : wide)
+    if (const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes);
+        e != hipSuccess) {
+      set_hip_error("MATVEC plan (wide LDS tiles)", e);
       return 1;
     }
   return 0;
@@ -376,11 +417,21 @@ int matvec_plan(Context& c, const char* name) {
     return 206;
   }
   const int nrows = c.ny * c.nz;
-  // pass 1 rows per workgroup: fill the LDS tile but keep >= ~4 workgroups per CU
-  m.rx_fwd = std::max(1, wide / m.gx);
-  while (m.rx_fwd > 1 && (size_t)((nrows + m.rx_fwd - 1) / m.rx_fwd) * 3 < 2048) m.rx_fwd /= 2;
-  m.rx_inv = std::max(1, narrow / m.gx);
-  while (m.rx_inv > 1 && (size_t)((nrows + m.rx_inv - 1) / m.rx_inv) < 1024) m.rx_inv /= 2;
+  const size_t lds_max = lds_limit();
+  // rows per workgroup of the LDS-staged x passes: what 256 threads hold at short
+  // axes, at long ones 16 (a 128-byte line of a1 per kx) or what 512 threads
+  // hold in half the LDS; fewer, but for an element a thread, where that leaves
+  // less than 512 workgroups (2,048 of them: 280 x 48 x 48 135 -> 168 us).
+  // Where at most 256 remain they take 512 threads too (16 rows of 1,024 points
+  // and more: 5 to 10 % of a MATVEC; with more workgroups it loses as much).
+  const auto tiles = [&](int rx) { return (nrows + rx - 1) / rx; };
+  int& rx = m.rx;
+  rx = PER_NARROW * MV_THREADS / m.gx;
+  if (rx < 16) rx = std::min(16, PER_NARROW * ROW_THREADS / m.gx);
+  while (rx > 1 && (size_t)m.gx * (1 + (rx | 1)) * sizeof(float2) > lds_max / 2) --rx;
+  while (rx > 1 && tiles(rx) < 512 && rx / 2 * m.gx >= MV_THREADS) rx /= 2;
+  const bool full = rx * m.gx > PER_NARROW * MV_THREADS, few = tiles(rx) <= 256 && rx * m.gx >= 2 * ROW_THREADS;
+  m.tx = full || few ? ROW_THREADS : MV_THREADS;
   m.cy = std::min(16, pow2floor(std::max(1, wide / m.gy)));
   // columns of the LDS-staged Green pass: as many as the workgroup has room for
   // (8 values a thread) in 1,024 workgroups or more, but at least 4 columns and
@@ -391,7 +442,6 @@ int matvec_plan(Context& c, const char* name) {
   };
   m.cz = green_columns(narrow);
   m.ty = m.tz = MV_THREADS;
-  const size_t lds_max = lds_limit();
   if (m.cy < 8) {
     int cw = std::min(16, pow2floor(std::max(1, PER_WIDE * WIDE_THREADS / m.gy)));
     while (cw > 1 && (size_t)(m.gy + cw * m.gy) * sizeof(float2) > lds_max) cw /= 2;
@@ -402,7 +452,7 @@ int matvec_plan(Context& c, const char* name) {
     while (cw > 1 && (size_t)(m.gz + 3 * (cw | 1) * m.gz) * sizeof(float2) > lds_max) --cw;
     if (cw > m.cz) { m.cz = cw; m.tz = WIDE_THREADS; }
   }
-  if ((m.ty == WIDE_THREADS || m.tz == WIDE_THREADS) && allow_big_lds(lds_max)) return 206;
+  if (std::max({m.tx, m.ty, m.tz}) > MV_THREADS && allow_big_lds(lds_max)) return 206;
   if (upload_twiddles(m.gx, &m.twx) || upload_twiddles(m.gy, &m.twy) || upload_twiddles(m.gz, &m.twz)) return 206;
   // z runs start on 128-byte lines, or on half lines where a whole one would
   // pad by more than a twentieth (16 right-hand sides of 48 x 50 x 50: 357 us at
@@ -449,10 +499,12 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
   if (!c.fft_generic && kind >= 0 && reg_pass(c, which, kind, cj, compact, x, y, adia, aoff, st, bt)) return 0;
   switch (which) {
     case 1: {
-      dim3 grid((nrows + m.rx_fwd - 1) / m.rx_fwd, 3, nb);
-      size_t lds = (size_t)(m.gx + m.rx_fwd * (m.gx + (m.rx_fwd > 1))) * sizeof(float2);
-      hipLaunchKernelGGL(k_pass1_xfwd<PER_WIDE>, grid, dim3(MV_THREADS), lds, st, x, a1, sm, m.twx, m.px, c.nx, c.ny,
-                         c.nz, m.nzp, m.p1, m.rx_fwd, c.nat, c.nat0, compact, cj, bt.k);
+      const dim3 grid((nrows + m.rx - 1) / m.rx, 3, nb);
+      const size_t lds = (size_t)m.gx * (1 + (m.rx | 1)) * sizeof(float2);
+      const auto kernel = m.tx == ROW_THREADS ? &k_pass1_xfwd<PER_NARROW, ROW_THREADS> : &k_pass1_xfwd<PER_NARROW>;
+      hipLaunchKernelGGL(kernel, grid, dim3(m.tx), lds, st, x, a1, sm, m.twx, m.px, c.nx, c.ny, c.nz, m.nzp, m.p1,
+                         m.rx, fast_div_by(c.nx), fast_div_by(c.nz), fast_div_by(m.rx), c.nat, c.nat0, compact,
+                         cj, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 1 (x FFT)", 21);
       break;
     }
@@ -491,12 +543,14 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
       break;
     }
     default: {
-      dim3 grid((nrows + m.rx_inv - 1) / m.rx_inv, nb);
-      size_t lds = (size_t)(m.gx + 3 * m.rx_inv * (m.gx + (m.rx_inv > 1))) * sizeof(float2);
+      const dim3 grid((nrows + m.rx - 1) / m.rx, nb);
+      const size_t lds = (size_t)m.gx * (1 + (m.rx | 1)) * sizeof(float2);
       const float inv = 1.f / (float)m.ngrid;
-      hipLaunchKernelGGL(k_pass5_xinv_finish<PER_NARROW>, grid, dim3(MV_THREADS), lds, st, a1, m.twx, m.px, x, y,
-                         adia, aoff, compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz, m.nzp, m.p1, m.rx_inv, c.nat, c.nat0,
-                         compact, cj, inv, bt.k);
+      const auto kernel =
+          m.tx == ROW_THREADS ? &k_pass5_xinv_finish<PER_NARROW, ROW_THREADS> : &k_pass5_xinv_finish<PER_NARROW>;
+      hipLaunchKernelGGL(kernel, grid, dim3(m.tx), lds, st, a1, m.twx, m.px, x, y, adia, aoff,
+                         compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz, m.nzp, m.p1, m.rx, fast_div_by(c.nx),
+                         fast_div_by(c.nz), fast_div_by(m.rx), c.nat, c.nat0, compact, cj, inv, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 5 (x inverse FFT + finish)", 25);
       break;
     }

@@ -18,8 +18,8 @@ struct MatvecPlan {
   FftPlan px{}, py{}, pz{};
   float2 *twx = nullptr, *twy = nullptr, *twz = nullptr;  // device twiddle tables
   // tile parameters
-  int rx_fwd = 1, rx_inv = 1, cy = 1, cz = 1;
-  int ty = 256, tz = 256;  // workgroup size of the LDS-staged y passes and z pass
+  int rx = 1, cy = 1, cz = 1;
+  int tx = 256, ty = 256, tz = 256;  // workgroup sizes of the LDS-staged x, y and z passes
   // z pitch and kx plane strides (elements) of the FFT3D work arrays
   // a1 [3][gx][p1: ny][nzp] and a2 [3][gx][p2: gy][nzp]
   int nzp = 0, p1 = 0, p2 = 0;
