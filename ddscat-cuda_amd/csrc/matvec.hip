@@ -123,12 +123,15 @@ __global__ __launch_bounds__(NT) void k_pass1_xfwd(
 
 // ------------------------------------------------------------- pass 2, 4 --
 // a1 [3][gx][p1: ny][nzp] <-> a2 [3][2H][p2: gy][nzp], FFT along the middle axis of
-// a plane, tiles of cy consecutive z.
+// a plane, cy columns per workgroup: column q = slot ni + iz of ni per plane,
+// NZ rounded up to whole tiles or, where that leaves lanes idle, NZ itself with
+// tiles that cross planes (MATVECs, whole tiles before: 280 x 280 x 1 241 -> 102 us,
+// 512 x 512 x 1 583 -> 203, 512 x 512 x 20 2,080 -> 1,715, 64 x 400 x 4 101 -> 72).
 template <int DIR, int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT) void k_pass_y(
     const float2* __restrict__ in, float2* __restrict__ out, const float2* __restrict__ twg,
     FftPlan p, KxSlab sl, int nin, int nout, int nz, int nzp, int ins,
-    int outs, int cy_log2, BatchArgs ba) {
+    int outs, int cy_log2, int ni, FastDiv dn, BatchArgs ba) {
   extern __shared__ float2 sm[];
   const int rb = blockIdx.z / 3;
   if (ba.active && !ba.active[rb]) return;
@@ -138,25 +141,28 @@ __global__ __launch_bounds__(NT) void k_pass_y(
   const int cy = 1 << cy_log2;
   float2* tw = sm;
   float2* buf = sm + L;
-  const int c = blockIdx.z % 3, slot = blockIdx.y, z0 = blockIdx.x * cy;
+  const int c = blockIdx.z % 3, q0 = blockIdx.x * cy, slot0 = q0 / ni;
   const int T = blockDim.x;
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
-  const size_t pl1 = (size_t)c * sl.gx + sl.kx(slot), pl2 = (size_t)c * (2 * sl.H) + slot;
-  const float2* src = in + (DIR > 0 ? pl1 : pl2) * ins;
+  // this thread's column: T is a multiple of cy
+  const int i = q0 - slot0 * ni + (threadIdx.x & (cy - 1)), d = fast_div(i, dn);
+  const int slot = slot0 + d, iz = i - d * ni;
+  const bool live = iz < nz && slot < 2 * sl.H;
+  const size_t pl1 = (size_t)c * sl.gx + sl.kx(live ? slot : 0), pl2 = (size_t)c * (2 * sl.H) + slot;
+  const float2* src = in + (DIR > 0 ? pl1 : pl2) * ins + iz;
   for (int idx = threadIdx.x; idx < L * cy; idx += T) {
-    const int e = idx >> cy_log2, col = idx & (cy - 1);
-    const int iz = z0 + col;
+    const int e = idx >> cy_log2;
     float2 v = make_float2(0.f, 0.f);
-    if (e < nin && iz < nz) v = src[(size_t)e * nzp + iz];
+    if (e < nin && live) v = src[(size_t)e * nzp];
     buf[idx] = v;
   }
   __syncthreads();
   fft_run<DIR, true, PER>(buf, tw, p, cy, cy, 1);
-  float2* dst = out + (DIR > 0 ? pl2 : pl1) * outs;
+  if (!live) return;
+  float2* dst = out + (DIR > 0 ? pl2 : pl1) * outs + iz;
   for (int idx = threadIdx.x; idx < nout * cy; idx += T) {
-    const int e = idx >> cy_log2, col = idx & (cy - 1);
-    const int iz = z0 + col;
-    if (iz < nz) dst[(size_t)e * nzp + iz] = buf[idx];
+    const int e = idx >> cy_log2;
+    dst[(size_t)e * nzp] = buf[idx];
   }
 }
 
@@ -510,22 +516,22 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
     }
     case 2:
     case 4: {
-      const bool fwd = which == 2;
-      dim3 grid((c.nz + m.cy - 1) / m.cy, 2 * bt.slab.H, 3 * nb);
+      const bool fwd = which == 2, wide = m.ty == WIDE_THREADS;
+      // whole tiles per plane, unless that leaves more than a ninth of them idle
+      const int whole = (c.nz + m.cy - 1) / m.cy * m.cy, ni = 8 * whole > 9 * c.nz ? c.nz : whole;
+      const dim3 grid((unsigned)((2 * bt.slab.H * ni + m.cy - 1) / m.cy), 1, 3 * nb);
       const size_t lds = (size_t)(m.gy + m.cy * m.gy) * sizeof(float2);
-      const int lg = ilog2(m.cy), ins = fwd ? m.p1 : m.p2, outs = fwd ? m.p2 : m.p1;
-      if (fwd && m.ty == WIDE_THREADS)
-        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a1, a2, m.twy,
-                           m.py, bt.slab, c.ny, m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
-      else if (fwd)
-        hipLaunchKernelGGL((k_pass_y<+1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a1, a2, m.twy, m.py, bt.slab, c.ny,
-                           m.gy, c.nz, m.nzp, ins, outs, lg, bt.k);
-      else if (m.ty == WIDE_THREADS)
-        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE, WIDE_THREADS>), grid, dim3(WIDE_THREADS), lds, st, a2, a1, m.twy,
-                           m.py, bt.slab, m.gy, c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
-      else
-        hipLaunchKernelGGL((k_pass_y<-1, PER_WIDE>), grid, dim3(MV_THREADS), lds, st, a2, a1, m.twy, m.py, bt.slab, m.gy,
-                           c.ny, c.nz, m.nzp, ins, outs, lg, bt.k);
+      const int lg = ilog2(m.cy);
+      const FastDiv dn = fast_div_by(ni);
+      if (fwd) {
+        const auto kernel = wide ? &k_pass_y<+1, PER_WIDE, WIDE_THREADS> : &k_pass_y<+1, PER_WIDE>;
+        hipLaunchKernelGGL(kernel, grid, dim3(m.ty), lds, st, a1, a2, m.twy, m.py, bt.slab, c.ny, m.gy, c.nz, m.nzp, m.p1,
+                           m.p2, lg, ni, dn, bt.k);
+      } else {
+        const auto kernel = wide ? &k_pass_y<-1, PER_WIDE, WIDE_THREADS> : &k_pass_y<-1, PER_WIDE>;
+        hipLaunchKernelGGL(kernel, grid, dim3(m.ty), lds, st, a2, a1, m.twy, m.py, bt.slab, m.gy, c.ny, c.nz, m.nzp, m.p2,
+                           m.p1, lg, ni, dn, bt.k);
+      }
       DDH_LAUNCH_OK("MATVEC y FFT", fwd ? 22 : 24);
       break;
     }
