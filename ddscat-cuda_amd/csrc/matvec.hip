@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <array>
 #include <map>
+#include <type_traits>
 
 namespace ddhip {
 
@@ -269,13 +270,16 @@ __device__ __forceinline__ void finish_site(float2 x1, float2 x2, float2 x3, flo
   if (cj) { r1.y = -r1.y; r2.y = -r2.y; r3.y = -r3.y; }
 }
 
-// One component after another in LDS, the kept half of each waiting in registers.
+// One component after another in LDS, the kept half of each waiting in registers;
+// `three`: all of them at once, in launches of up to 256 workgroups that have
+// the room, which then wait for one round of loads and not for three (5 x 24 x 24
+// 25.9 -> 24.5 us, 400 x 10 x 10 67 -> 65).
 template <int PER, int NT = MV_THREADS>
 __global__ __launch_bounds__(NT, 4) void k_pass5_xinv_finish(
     const float2* __restrict__ a1, const float2* __restrict__ twg, FftPlan p,
     const float2* __restrict__ x, float2* __restrict__ y, const float2* __restrict__ adia,
     const float2* __restrict__ aoff, const int16_t* __restrict__ iocc, SiteMap map, int nx, int ny, int nz, int nzp,
-    int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int nat, int nat0, int compact, int cj, float inv,
+    int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int three, int nat, int nat0, int compact, int cj, float inv,
     BatchArgs ba) {
   constexpr int KEEP = PER / 2;  // kept outputs per thread and component
   extern __shared__ float2 sm[];
@@ -293,26 +297,40 @@ __global__ __launch_bounds__(NT, 4) void k_pass5_xinv_finish(
   const int T = blockDim.x;
   for (int i = threadIdx.x; i < L; i += T) tw[i] = twg[i];
   const size_t cs = (size_t)L * ks;
-  float2 w[3][KEEP];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    if (c) __syncthreads();
+  // components c0 .. c0 + NC - 1 of the tile, bs apart in LDS
+  const int bs = three ? rp * L : 0;
+  const auto load = [&](int c0, auto nc) {
+    constexpr int NC = decltype(nc)::value;
     for (int idx = threadIdx.x; idx < rx * L; idx += T) {
       const int k = fast_div(idx, t.dr), r = idx - k * rx;
-      float2 v = make_float2(0.f, 0.f);
+      float2 v[NC];
+#pragma unroll
+      for (int c = 0; c < NC; ++c) v[c] = make_float2(0.f, 0.f);
       if (r < t.nr) {
         int iy, iz;
         t.row(r, iy, iz);
-        v = a1[c * cs + (size_t)k * ks + (size_t)iy * nzp + iz];
+        const float2* src = a1 + c0 * cs + (size_t)k * ks + (size_t)iy * nzp + iz;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) v[c] = src[c * cs];
       }
-      buf[k * rp + r] = v;
+#pragma unroll
+      for (int c = 0; c < NC; ++c) buf[(c0 + c) * bs + k * rp + r] = v[c];
     }
     __syncthreads();
-    fft_run<-1, true, PER>(buf, tw, p, rx, rp, 1);
+  };
+  if (three) load(0, std::integral_constant<int, 3>{});
+  float2 w[3][KEEP];
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    if (!three) {
+      if (c) __syncthreads();
+      load(c, std::integral_constant<int, 1>{});
+    }
+    fft_run<-1, true, PER>(buf + c * bs, tw, p, rx, rp, 1);
 #pragma unroll
     for (int j = 0; j < KEEP; ++j) {
       const int idx = threadIdx.x + j * T, r = fast_div(idx, dx), ix = idx - r * nx;
-      w[c][j] = r < rx ? buf[ix * rp + r] : make_float2(0.f, 0.f);
+      w[c][j] = r < rx ? buf[c * bs + ix * rp + r] : make_float2(0.f, 0.f);
     }
   }
   const size_t sd = compact ? (size_t)nat0 : (size_t)nat;
@@ -428,23 +446,26 @@ int matvec_plan(Context& c, const char* name) {
   // axes, at long ones 16 (a 128-byte line of a1 per kx) or what 512 threads
   // hold in half the LDS; fewer, but for an element a thread, where that leaves
   // less than 512 workgroups (2,048 of them: 280 x 48 x 48 135 -> 168 us).
-  // Where at most 256 remain they take 512 threads too (16 rows of 1,024 points
-  // and more: 5 to 10 % of a MATVEC; with more workgroups it loses as much).
+  // Where at most 256 remain they take 512 threads too (targets of 4 x 4 to 16 x
+  // 16 rows: 5 to 10 % of a MATVEC; with more workgroups it loses as much).
   const auto tiles = [&](int rx) { return (nrows + rx - 1) / rx; };
   int& rx = m.rx;
   rx = PER_NARROW * MV_THREADS / m.gx;
   if (rx < 16) rx = std::min(16, PER_NARROW * ROW_THREADS / m.gx);
   while (rx > 1 && (size_t)m.gx * (1 + (rx | 1)) * sizeof(float2) > lds_max / 2) --rx;
   while (rx > 1 && tiles(rx) < 512 && rx / 2 * m.gx >= MV_THREADS) rx /= 2;
-  const bool full = rx * m.gx > PER_NARROW * MV_THREADS, few = tiles(rx) <= 256 && rx * m.gx >= 2 * ROW_THREADS;
+  const bool full = rx * m.gx > PER_NARROW * MV_THREADS, few = tiles(rx) <= 256 && rx * m.gx >= ROW_THREADS;
   m.tx = full || few ? ROW_THREADS : MV_THREADS;
   m.cy = std::min(16, pow2floor(std::max(1, wide / m.gy)));
   // columns of the LDS-staged Green pass: as many as the workgroup has room for
-  // (8 values a thread) in 1,024 workgroups or more, but at least 4 columns and
-  // an element for every thread
+  // (8 values a thread) in 1,024 workgroups or more, but at least 4 columns, an
+  // element for every thread, and no thread idle in the last round of them (400 x
+  // 10 x 10: 15 columns 75 us, 25 67)
   const auto green_columns = [&](int elements) {
     const int ncol = m.gx * m.gy, least = std::max(4, (MV_THREADS + m.gz - 1) / m.gz);
-    return std::max(1, std::min(elements / m.gz, std::max(least, ncol / 1024)));
+    const int cz = std::max(1, std::min(elements / m.gz, std::max(least, ncol / 1024)));
+    const int rounds = (cz * m.gz + MV_THREADS - 1) / MV_THREADS;
+    return std::max(cz, std::min(elements, rounds * MV_THREADS) / m.gz);
   };
   m.cz = green_columns(narrow);
   m.ty = m.tz = MV_THREADS;
@@ -550,13 +571,15 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
     }
     default: {
       const dim3 grid((nrows + m.rx - 1) / m.rx, nb);
-      const size_t lds = (size_t)m.gx * (1 + (m.rx | 1)) * sizeof(float2);
+      size_t lds = (size_t)m.gx * (1 + 3 * (m.rx | 1)) * sizeof(float2);
+      const int three = lds <= 64 * 1024 && grid.x * nb <= 256;
+      if (!three) lds = (size_t)m.gx * (1 + (m.rx | 1)) * sizeof(float2);
       const float inv = 1.f / (float)m.ngrid;
       const auto kernel =
           m.tx == ROW_THREADS ? &k_pass5_xinv_finish<PER_NARROW, ROW_THREADS> : &k_pass5_xinv_finish<PER_NARROW>;
       hipLaunchKernelGGL(kernel, grid, dim3(m.tx), lds, st, a1, m.twx, m.px, x, y, adia, aoff,
                          compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz, m.nzp, m.p1, m.rx, fast_div_by(c.nx),
-                         fast_div_by(c.nz), fast_div_by(m.rx), c.nat, c.nat0, compact, cj, inv, bt.k);
+                         fast_div_by(c.nz), fast_div_by(m.rx), three, c.nat, c.nat0, compact, cj, inv, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 5 (x inverse FFT + finish)", 25);
       break;
     }
