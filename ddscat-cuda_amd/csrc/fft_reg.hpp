@@ -179,20 +179,12 @@ struct Reg2 {
   static constexpr int G = (R2 + R1 - 1) / R1;
   static constexpr int VN = R2 > G * R1 ? R2 : G * R1;
 };
-// Column tile of block bx (tiles of C complex64 columns, NT tiles) for
-// kernels whose tiles are narrower than a 128-byte line (C < 16).  Blocks go
-// round-robin over the 8 XCDs by linear id, and each XCD has its own L2, so
-// the W = 16/C tiles sharing one line are given to blocks 8 ids apart (same
-// XCD, back to back).  The plain order when NT is not a multiple of 8 times W
-// or C >= 16.
-template <int C>
-__device__ __forceinline__ int xcd_tile(int bx, int NT) {
-  constexpr int W = C >= 16 ? 1 : 16 / C;
-  if (W > 1 && NT % (8 * W) == 0) {
-    const int m = bx >> 3, r = bx & 7;
-    return W * (r + 8 * (m / W)) + m % W;
-  }
-  return bx;
+// Tile of block bx of n.  Blocks go round-robin over the 8 XCDs by linear id, and
+// each XCD has its own L2: the blocks of one XCD (ids 8 apart) take a run of
+// neighbours, so that tiles which share a 128-byte line share it there.
+__device__ __forceinline__ int xcd_run(int bx, int n) {
+  const int x = bx & 7, q = n >> 3, rem = n & 7;
+  return x * q + min(x, rem) + (bx >> 3);
 }
 
 // The padded axes have length L = R1 R2 = 2N with data (forward input) and

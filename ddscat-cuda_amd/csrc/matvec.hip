@@ -20,7 +20,7 @@
 // register shape use the kernels of rows.hpp, matvec_reg.hip and
 // pass3_wave.hpp, which read and write the same arrays.
 #include "state.hpp"
-#include "fft_device.hpp"
+#include "fft_reg.hpp"
 #include "mv_device.hpp"
 #include <vector>
 #include <cmath>
@@ -48,13 +48,6 @@ struct FastDiv {
 };
 static FastDiv fast_div_by(int d) { return FastDiv{(unsigned)((((uint64_t)1 << 32) + d - 1) / (uint64_t)d)}; }
 __device__ __forceinline__ int fast_div(int x, FastDiv d) { return d.m ? (int)__umulhi((unsigned)x, d.m) : x; }
-
-// tile of block bx of n: the blocks of one XCD (ids 8 apart) take neighbours,
-// whose pieces of a 128-byte line then meet in that XCD's L2
-__device__ __forceinline__ int xcd_run(int bx, int n) {
-  const int x = bx & 7, q = n >> 3, rem = n & 7;
-  return x * q + min(x, rem) + (bx >> 3);
-}
 
 // The x passes: rows q = iy NZ + iz, rx of them per workgroup, interleaved in
 // LDS at an odd pitch, so that the vectors are walked with lanes over x and the

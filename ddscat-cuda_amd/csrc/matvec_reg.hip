@@ -20,6 +20,15 @@ struct Cols {
   size_t p1, p2, c1, c2;  // plane and component strides in a1 and a2
   KxSlab sl;
 };
+// Tile of this workgroup.  Where tiles share 128-byte lines (z runs of no whole
+// lines, tiles of less than one) neighbours run on one XCD: MATVECs with the
+// tiles dealt out over the XCDs, and so, 80 x 80 x 20 with 8 right-hand sides 174 ->
+// 137 us, 80 x 80 x 28 243 -> 209, 100^3 181 -> 175, 120^3 302 -> 292; on whole lines
+// 128^3 and 192^3 were up to 1 % slower so.
+template <int C>
+__device__ __forceinline__ int y_tile(const Cols& q) {
+  return C < 16 || q.pitch % 16 ? xcd_run((int)blockIdx.x, (int)gridDim.x) : (int)blockIdx.x;
+}
 // o and i of column q0 + s, q0 the workgroup's first column (divided once, as a scalar)
 __device__ __forceinline__ void column_of(const Cols& q, int q0, int s, int& o, int& i) {
   o = q0 / q.ni;
@@ -43,7 +52,7 @@ __global__ __launch_bounds__(R1 * C) void kr_passy(const float2* __restrict__ in
   in += rb * (DIR > 0 ? ba.a1s : ba.a2s);
   out += rb * (DIR > 0 ? ba.a2s : ba.a1s);
   const int s = threadIdx.x % C, t = threadIdx.x / C;
-  const int q0 = xcd_tile<C>((int)blockIdx.x, (int)gridDim.x) * C, c = blockIdx.z % 3;
+  const int q0 = y_tile<C>(q) * C, c = blockIdx.z % 3;
   for (int i = threadIdx.x; i < L; i += RT) twL[i] = twg[i];
   const bool live = q0 + s < q.total;
   int o, col;
@@ -120,7 +129,7 @@ __global__ __launch_bounds__(M * 16 * C) void kr_passym(const float2* __restrict
   out += rb * (DIR > 0 ? ba.a2s : ba.a1s);
   const int m = threadIdx.x / GT, lt = threadIdx.x % GT;
   const int s = lt % C, t = lt / C, sv = m * C + s;
-  const int q0 = xcd_tile<C>((int)blockIdx.x, (int)gridDim.x) * C, c = blockIdx.z % 3;
+  const int q0 = y_tile<C>(q) * C, c = blockIdx.z % 3;
   for (int i = threadIdx.x; i < L; i += RT) twL[i] = twg[i];
   for (int i = threadIdx.x; i < S; i += RT) twS[i] = twg[M * i];
   const bool live = q0 + s < q.total;
