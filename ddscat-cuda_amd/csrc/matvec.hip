@@ -474,13 +474,16 @@ int matvec_plan(Context& c, const char* name) {
   }
   if (std::max({m.tx, m.ty, m.tz}) > MV_THREADS && allow_big_lds(lds_max)) return 206;
   if (upload_twiddles(m.gx, &m.twx) || upload_twiddles(m.gy, &m.twy) || upload_twiddles(m.gz, &m.twz)) return 206;
-  // z runs start on 128-byte lines, or on half lines where a whole one would
-  // pad by more than a twentieth (16 right-hand sides of 48 x 50 x 50: 357 us at
-  // a pitch of 64, 332 at 56; of 72 x 80 x 120: 1,827 at 128, 1,724 at 120;
-  // NZ = 108, which 112 pads by 4 %: 350 us, 361 unpadded); targets of a few
-  // planes keep a small pitch
-  const int line = (c.nz + 15) & ~15;
-  m.nzp = c.nz <= 32 ? (c.nz + 3) & ~3 : 20 * (line - c.nz) > c.nz ? (c.nz + 7) & ~7 : line;
+  // z runs start on 128-byte lines; on half lines where whole ones would pad by
+  // more than a twentieth (16 right-hand sides of 48 x 50 x 50: 357 us at a pitch of
+  // 64, 332 at 56; of 72 x 80 x 120: 1,827 at 128, 1,724 at 120; NZ = 108, which 112
+  // pads by 4 %: 350 us, 361 unpadded); on quarter lines where half ones would
+  // pad by more than a tenth (8 right-hand sides of 80 x 80 x 36: 314 us at 40, 290
+  // at 36, of 80 x 80 x 50: 482 at 56, 460 at 52; but of 80 x 80 x 75, padded by 7 %: 607
+  // at 80, 639 at 76) and for targets of few planes
+  const auto up = [&](int n) { return (c.nz + n - 1) / n * n; };
+  const auto pads = [&](int n, int part) { return part * (up(n) - c.nz) > c.nz; };
+  m.nzp = c.nz <= 32 ? up(4) : !pads(16, 20) ? up(16) : !pads(8, 10) ? up(8) : up(4);
   // an odd number of 128-byte lines per kx plane: passes 1 and 5 step through
   // the planes, and an even step hits fewer memory channels (pass 4 at 256^3
   // 505 us with the power of two it has unpadded, 456 so; an odd number of
