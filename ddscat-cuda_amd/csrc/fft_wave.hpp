@@ -39,6 +39,12 @@ struct WPlan {
   static constexpr int SLOTS = PAD ? L + L / R0 : L;  // LDS slots of one sequence
   static_assert(T <= 64 && nb(0) >= 1, "a sequence sits in one wave");
 };
+template <class PL>
+FftPlan w_stages() {
+  FftPlan p{PL::L, PL::S, {}};
+  for (int s = 0; s < PL::S; ++s) p.rad[s] = PL::rad(s);
+  return p;
+}
 // LDS slot of point idx: one slot of padding per R0 points, so the stride-R0
 // scatter of stage 0 (odd stride after padding) and the unit-stride gathers
 // both spread over the banks

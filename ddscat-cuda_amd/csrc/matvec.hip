@@ -20,6 +20,7 @@
 // register shape use the kernels of rows.hpp, matvec_reg.hip and
 // pass3_wave.hpp, which read and write the same arrays.
 #include "state.hpp"
+#include "fft_gain.hpp"
 #include "fft_reg.hpp"
 #include "mv_device.hpp"
 #include <vector>
@@ -249,20 +250,6 @@ __global__ __launch_bounds__(NT) void k_pass3_z_green(
 }
 
 // ---------------------------------------------------------------- pass 5 --
-__device__ __forceinline__ void finish_site(float2 x1, float2 x2, float2 x3, float2 d1, float2 d2,
-                                            float2 d3, float2 a23, float2 a31, float2 a12,
-                                            float2 w1, float2 w2, float2 w3, float inv, bool cj,
-                                            float2& r1, float2& r2, float2& r3) {
-  if (cj) { x1.y = -x1.y; x2.y = -x2.y; x3.y = -x3.y; }
-  r1 = csub(cmul(d1, x1), cscale(w1, inv));
-  r2 = csub(cmul(d2, x2), cscale(w2, inv));
-  r3 = csub(cmul(d3, x3), cscale(w3, inv));
-  r1 = cadd(r1, cadd(cmul(a31, x3), cmul(a12, x2)));
-  r2 = cadd(r2, cadd(cmul(a12, x1), cmul(a23, x3)));
-  r3 = cadd(r3, cadd(cmul(a23, x2), cmul(a31, x1)));
-  if (cj) { r1.y = -r1.y; r2.y = -r2.y; r3.y = -r3.y; }
-}
-
 // One component after another in LDS, the kept half of each waiting in registers;
 // `three`: all of them at once, in launches of up to 256 workgroups that have
 // the room, which then wait for one round of loads and not for three (5 x 24 x 24
@@ -272,7 +259,7 @@ __global__ __launch_bounds__(NT, 4) void k_pass5_xinv_finish(
     const float2* __restrict__ a1, const float2* __restrict__ twg, FftPlan p,
     const float2* __restrict__ x, float2* __restrict__ y, const float2* __restrict__ adia,
     const float2* __restrict__ aoff, const int16_t* __restrict__ iocc, SiteMap map, int nx, int ny, int nz, int nzp,
-    int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int three, int nat, int nat0, int compact, int cj, float inv,
+    int ks, int rx, FastDiv dx, FastDiv dz, FastDiv dr, int three, int nat, int nat0, int compact, int cj, float2 inv,
     BatchArgs ba) {
   constexpr int KEEP = PER / 2;  // kept outputs per thread and component
   extern __shared__ float2 sm[];
@@ -340,9 +327,15 @@ __global__ __launch_bounds__(NT, 4) void k_pass5_xinv_finish(
     if (iocc && iocc[o] == 0) {
       r1 = r2 = r3 = make_float2(0.f, 0.f);
     } else {
-      const size_t q = (size_t)o;
-      finish_site(x[q], x[q + sd], x[q + 2 * sd], adia[q], adia[q + sd], adia[q + 2 * sd], aoff[q], aoff[q + sd],
-                  aoff[q + 2 * sd], w[0][j], w[1][j], w[2][j], inv, cj != 0, r1, r2, r3);
+      float2 xv[3], dv[3], av[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        const size_t q = (size_t)o + c * sd;
+        xv[c] = x[q];
+        dv[c] = adia[q];
+        av[c] = aoff[q];
+      }
+      finish_site(xv, dv, av, w[0][j], w[1][j], w[2][j], inv, cj != 0, r1, r2, r3);
     }
     y[o] = r1; y[o + sd] = r2; y[o + 2 * sd] = r3;
   }
@@ -511,6 +504,31 @@ void matvec_release(Context& c) {
   }
 }
 
+// Pass 5's factor for the kernels in use: 1 / G without the gain of the transforms
+// (fft_gain.hpp), in double and then as a float and the rest.
+static void matvec_scale(Context& c, int kind5, const KxSlab& sl) {
+  MatvecPlan& m = c.mv;
+  const FftPlan* staged[6] = {nullptr, &m.px, &m.py, &m.pz, &m.py, &m.px};
+  const int lens[6] = {0, m.gx, m.gy, m.gz, m.gy, m.gx}, plane = plane_yz_runs(c);
+  int key[6] = {plane};
+  for (int p = 1; p <= 5; ++p) key[p] = c.fft_generic ? -1 : p == 5 ? kind5 : m.kind[p];
+  if (key[3] >= 0 && !reg_green_reach(c, sl)) key[3] = -1;
+  if (std::equal(key, key + 6, m.scale_key)) return;
+  const auto gain = [&](int p) { return fft_gain(key[p] >= 0 ? reg_stages(lens[p], p, key[p]) : *staged[p]); };
+  double g = 1.0 + 0.5 * (gain(1) + gain(5));
+  if (plane) {
+    FftPlan y, z;
+    plane_yz_stages(c, y, z);
+    g *= (1.0 + fft_gain(y)) * (1.0 + fft_gain(z));
+  } else {
+    g *= (1.0 + 0.5 * (gain(2) + gain(4))) * (1.0 + gain(3));
+  }
+  const double f = 1.0 / ((double)m.ngrid * g);
+  m.scale.x = (float)f;
+  m.scale.y = (float)(f - (double)m.scale.x);
+  std::copy(key, key + 6, m.scale_key);
+}
+
 // One MATVEC pass with kernel choice `kind` (-1: LDS-staged, >= 0: register shape).
 static int launch_pass(Context& c, int which, int kind, int cj, int compact, const float2* x, float2* y,
                        const float2* adia, const float2* aoff, hipStream_t st, const MvBatch& bt) {
@@ -519,6 +537,7 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
   const unsigned nb = (unsigned)bt.nrhs;
   float2 *a1 = bt.a1, *a2 = bt.a2;
   const SiteMap sm{c.rowptr, c.rowlo, c.qmap, c.rows_contiguous};
+  if (which == 5) matvec_scale(c, kind, bt.slab);
   if (!c.fft_generic && kind >= 0 && reg_pass(c, which, kind, cj, compact, x, y, adia, aoff, st, bt)) return 0;
   switch (which) {
     case 1: {
@@ -570,12 +589,11 @@ static int launch_pass(Context& c, int which, int kind, int cj, int compact, con
       size_t lds = (size_t)m.gx * (1 + 3 * (m.rx | 1)) * sizeof(float2);
       const int three = lds <= 64 * 1024 && grid.x * nb <= 256;
       if (!three) lds = (size_t)m.gx * (1 + (m.rx | 1)) * sizeof(float2);
-      const float inv = 1.f / (float)m.ngrid;
       const auto kernel =
           m.tx == ROW_THREADS ? &k_pass5_xinv_finish<PER_NARROW, ROW_THREADS> : &k_pass5_xinv_finish<PER_NARROW>;
       hipLaunchKernelGGL(kernel, grid, dim3(m.tx), lds, st, a1, m.twx, m.px, x, y, adia, aoff,
                          compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz, m.nzp, m.p1, m.rx, fast_div_by(c.nx),
-                         fast_div_by(c.nz), fast_div_by(m.rx), three, c.nat, c.nat0, compact, cj, inv, bt.k);
+                         fast_div_by(c.nz), fast_div_by(m.rx), three, c.nat, c.nat0, compact, cj, m.scale, bt.k);
       DDH_LAUNCH_OK("MATVEC pass 5 (x inverse FFT + finish)", 25);
       break;
     }

@@ -241,10 +241,11 @@ static void launch_y_m(Context& c, int dir, const MvBatch& bt, hipStream_t st) {
 struct YShape {
   int L;
   void (*fn)(Context&, int, const MvBatch&, hipStream_t);
+  int rad[3];        // its stages in order
   bool sup = false;  // the kernel honours BatchArgs::ysup
 };
-#define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>}
-#define Y_SPLIT(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C, true>}
+#define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>, {R2, R1, 1}}
+#define Y_SPLIT(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C, true>, {R2, R1, 1}}
 // One shape per padded length 2N, N = 2^a 3^b 5^c 7^d from 12 to 256 and a few
 // above (two-level, R1 threads per column, at most 25 values each, C columns
 // per workgroup; 512 and 768 points by decimation, 20 and 30 % faster there).
@@ -268,8 +269,8 @@ static const YShape kYShapes[] = {
     Y_SHAPE(16, 15, 16), Y_SHAPE(25, 10, 16), Y_SHAPE(16, 16, 32), Y_SHAPE(18, 15, 16), Y_SPLIT(18, 16, 16),
     Y_SHAPE(20, 15, 16), Y_SHAPE(20, 16, 16), Y_SPLIT(18, 18, 16), Y_SHAPE(20, 18, 16), Y_SPLIT(24, 16, 16),
     Y_SPLIT(20, 20, 16), Y_SPLIT(24, 18, 16), Y_SPLIT(25, 18, 16), Y_SPLIT(24, 20, 16), Y_SHAPE(27, 18, 16),
-    Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>, true}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
-    Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>, true},
+    Y_SHAPE(25, 20, 16), YShape{512, &launch_y_m<2, 16>, {16, 16, 2}, true}, Y_SHAPE(27, 20, 8), Y_SHAPE(24, 24, 8), Y_SHAPE(25, 24, 8),
+    Y_SHAPE(32, 20, 8), Y_SHAPE(27, 24, 8), Y_SHAPE(30, 24, 8), Y_SHAPE(30, 25, 8), YShape{768, &launch_y_m<3, 16>, {16, 16, 3}, true},
     // a factor 7
     Y_SHAPE(7, 4, 32), Y_SHAPE(7, 6, 32), Y_SHAPE(8, 7, 32), Y_SHAPE(10, 7, 32), Y_SHAPE(12, 7, 16),
     Y_SHAPE(14, 7, 16), Y_SHAPE(14, 8, 16), Y_SHAPE(14, 9, 16), Y_SHAPE(14, 10, 16), Y_SHAPE(14, 12, 16),
@@ -304,12 +305,30 @@ bool reg_row_support(int L, int cand) {
   return y && y->sup;
 }
 
+FftPlan reg_stages(int L, int which, int cand) {
+  if (which == 3) {
+    const P3Shape* r = p3_shape(L, cand);
+    return r ? r->stages() : FftPlan{};
+  }
+  if (which == 1 || which == 5) {
+    const RowShape* r = row_shape(L, which, cand);
+    return r ? FftPlan{L, 2, {r->R2, r->R1}} : FftPlan{};
+  }
+  const YShape* y = y_shape(L, cand);
+  return y ? FftPlan{L, 3, {y->rad[0], y->rad[1], y->rad[2]}} : FftPlan{};
+}
+
 int reg_candidates(int L, int which) {
   int n = 0;
   while (which == 3 ? p3_shape(L, n) != nullptr
                     : (which == 1 || which == 5) ? row_shape(L, which, n) != nullptr : y_shape(L, n) != nullptr)
     ++n;
   return n;
+}
+
+bool reg_green_reach(const Context& c, const KxSlab& sl) {
+  const size_t lim = (size_t)1 << 32, comp = (size_t)(2 * sl.H) * c.mv.p2 * sizeof(float2);
+  return comp < lim && green_points(c.nx, c.ny, c.nz, c.ipbc) * 6 * sizeof(float2) < lim;
 }
 
 // launches register pass `which` (1..5) with shape `cand` of its axis length;
@@ -324,10 +343,7 @@ int reg_pass(Context& c, int which, int cand, int cj, int compact, const float2*
     return r != nullptr;
   }
   if (which == 3) {
-    // the wave kernel addresses a component of a2 and the Green array with
-    // 32-bit byte offsets; larger grids take the LDS-staged kernel
-    const size_t lim = (size_t)1 << 32, comp = (size_t)(2 * bt.slab.H) * m.p2 * sizeof(float2);
-    if (comp >= lim || green_points(c.nx, c.ny, c.nz, c.ipbc) * 6 * sizeof(float2) >= lim) return 0;
+    if (!reg_green_reach(c, bt.slab)) return 0;
     const P3Shape* r = p3_shape(m.gz, cand);
     if (r) r->fn(c, bt, st);
     return r != nullptr;

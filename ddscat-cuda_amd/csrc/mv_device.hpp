@@ -66,6 +66,24 @@ __device__ __forceinline__ Green6 green_at_b(const char* __restrict__ g, unsigne
   return Green6{make_float2(a.x, a.y), make_float2(a.z, a.w), make_float2(b.x, b.y),
                 make_float2(b.z, b.w), make_float2(c.x, c.y), make_float2(c.z, c.w)};
 }
+// d x - (inv.x + inv.y) w: the convolution's scale as a float and the rest
+// (matvec_scale), which enters where a product is rounded anyway
+__device__ __forceinline__ float2 scaled_site(float2 d, float2 x, float2 w, float2 inv) {
+  const float re = fmaf(d.x, x.x, -fmaf(d.y, x.y, w.x * inv.y));
+  const float im = fmaf(d.x, x.y, fmaf(d.y, x.x, -(w.y * inv.y)));
+  return make_float2(fmaf(-w.x, inv.x, re), fmaf(-w.y, inv.x, im));
+}
+// one site of the finish (cu:116-118): r = d x - w / G + offdiag(a) x, conjugated in and out with cj
+__device__ __forceinline__ void finish_site(const float2* x, const float2* d, const float2* a, float2 w1, float2 w2,
+                                            float2 w3, float2 inv, bool cj, float2& r1, float2& r2, float2& r3) {
+  float2 x1 = x[0], x2 = x[1], x3 = x[2];
+  const float2 a23 = a[0], a31 = a[1], a12 = a[2];
+  if (cj) { x1.y = -x1.y; x2.y = -x2.y; x3.y = -x3.y; }
+  r1 = cadd(scaled_site(d[0], x1, w1, inv), cadd(cmul(a31, x3), cmul(a12, x2)));
+  r2 = cadd(scaled_site(d[1], x2, w2, inv), cadd(cmul(a12, x1), cmul(a23, x3)));
+  r3 = cadd(scaled_site(d[2], x3, w3, inv), cadd(cmul(a23, x2), cmul(a31, x1)));
+  if (cj) { r1.y = -r1.y; r2.y = -r2.y; r3.y = -r3.y; }
+}
 // finish of row g (cu:116-118): y = adia x - w/G + offdiag(aoff) x on the
 // unpadded outputs; w0..w2[n2] hold the inverse-transformed components at
 // row index ix(n2) for n2 < H, kept(n2, ix) says whether ix < nx (compact
@@ -79,7 +97,7 @@ __device__ __forceinline__ void p5_finish_at(const float2* w0, const float2* w1,
                                              int g, const float2* __restrict__ x, float2* __restrict__ y,
                                              const float2* __restrict__ adia, const float2* __restrict__ aoff,
                                              const int16_t* __restrict__ iocc, const SiteMap& sm, int nx, int nat,
-                                             int nat0, int compact, int cj, float inv) {
+                                             int nat0, int compact, int cj, float2 inv) {
   size_t o[H];
   bool st[H], zr[H];
   if (!compact) {
@@ -125,16 +143,8 @@ __device__ __forceinline__ void p5_finish_at(const float2* w0, const float2* w1,
 #pragma unroll
     for (int j = 0; j < FG && g0 + j < H; ++j) {
       const int n2 = g0 + j;
-      float2 x1 = xv[j][0], x2 = xv[j][1], x3 = xv[j][2];
-      const float2 a23 = av[j][0], a31 = av[j][1], a12 = av[j][2];
-      if (cj) { x1.y = -x1.y; x2.y = -x2.y; x3.y = -x3.y; }
-      float2 r1 = csub(cmul(dv[j][0], x1), cscale(w0[n2], inv));
-      float2 r2 = csub(cmul(dv[j][1], x2), cscale(w1[n2], inv));
-      float2 r3 = csub(cmul(dv[j][2], x3), cscale(w2[n2], inv));
-      r1 = cadd(r1, cadd(cmul(a31, x3), cmul(a12, x2)));
-      r2 = cadd(r2, cadd(cmul(a12, x1), cmul(a23, x3)));
-      r3 = cadd(r3, cadd(cmul(a23, x2), cmul(a31, x1)));
-      if (cj) { r1.y = -r1.y; r2.y = -r2.y; r3.y = -r3.y; }
+      float2 r1, r2, r3;
+      finish_site(xv[j], dv[j], av[j], w0[n2], w1[n2], w2[n2], inv, cj != 0, r1, r2, r3);
       if (zr[n2]) r1 = r2 = r3 = make_float2(0.f, 0.f);
       if (st[n2]) {
         const size_t e = o[n2];

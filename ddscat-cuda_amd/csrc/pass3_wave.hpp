@@ -212,9 +212,10 @@ static void launch_kw_pass3(Context& c, const MvBatch& bt, hipStream_t st) {
 struct P3Shape {
   int L;
   void (*fn)(Context&, const MvBatch&, hipStream_t);
+  FftPlan (*stages)();
 };
 // P3_PLAN(lanes per column, radices...)
-#define P3_PLAN(...) P3Shape{WPlan<__VA_ARGS__>::L, &launch_kw_pass3<WPlan<__VA_ARGS__>>}
+#define P3_PLAN(...) P3Shape{WPlan<__VA_ARGS__>::L, &launch_kw_pass3<WPlan<__VA_ARGS__>>, &w_stages<WPlan<__VA_ARGS__>>}
 const P3Shape* p3_shapes_short(int& n);   // up to 160 points
 const P3Shape* p3_shapes_medium(int& n);  // 162 to 324
 const P3Shape* p3_shapes_long(int& n);    // 360 to 768

@@ -57,6 +57,12 @@ int plane_yz_setup(Context& c) {
   return 0;
 }
 
+void plane_yz_stages(const Context& c, FftPlan& y, FftPlan& z) {
+  const YzSplit* s = y_split(c.mv.gy);
+  y = FftPlan{c.mv.gy, 2, {s->R2, s->R1}};
+  z = z_shape(c.mv.gz)->stages();
+}
+
 int plane_yz_launch(Context& c, hipStream_t st, const MvBatch& bt) {
   const MatvecPlan& m = c.mv;
   const YzShape* z = z_shape(m.gz);

@@ -210,6 +210,7 @@ int yz_pitch() {
 struct YzShape {
   int L, seq;     // padded z axis, columns per wave
   int (*pitch)();
+  FftPlan (*stages)();
   const void* (*kernel)(bool mirror);
 };
 template <class PL>
@@ -217,7 +218,8 @@ const void* yz_kernel(bool mirror) {
   return mirror ? reinterpret_cast<const void*>(&kw_plane_yz<PL, true>)
                 : reinterpret_cast<const void*>(&kw_plane_yz<PL, false>);
 }
-#define YZ_PLAN(...) YzShape{WPlan<__VA_ARGS__>::L, WPlan<__VA_ARGS__>::SEQ, &yz_pitch<WPlan<__VA_ARGS__>>, &yz_kernel<WPlan<__VA_ARGS__>>}
+#define YZ_PLAN(...) YzShape{WPlan<__VA_ARGS__>::L, WPlan<__VA_ARGS__>::SEQ, &yz_pitch<WPlan<__VA_ARGS__>>, &w_stages<WPlan<__VA_ARGS__>>, \
+  &yz_kernel<WPlan<__VA_ARGS__>>}
 const YzShape* yz_shapes(int& n);
 
 }  // namespace ddhip

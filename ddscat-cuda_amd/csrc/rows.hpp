@@ -138,7 +138,7 @@ __global__ __launch_bounds__(R1 * C) void kx_inv(const float2* __restrict__ a1, 
                                                  const float2* __restrict__ x, float2* __restrict__ y,
                                                  const float2* __restrict__ adia, const float2* __restrict__ aoff,
                                                  const int16_t* __restrict__ iocc, SiteMap sm, int nx, int ny, int nz,
-                                                 int nzp, int ks, int nat, int nat0, int compact, int cj, float inv,
+                                                 int nzp, int ks, int nat, int nat0, int compact, int cj, float2 inv,
                                                  BatchArgs ba) {
   constexpr int L = R1 * R2, RT = R1 * C, P = C + 1, G = Reg2<R1, R2>::G, VN = G * R1, H = (R2 + 1) / 2;
   __shared__ float2 twL[L];
@@ -258,16 +258,17 @@ static void launch_kx_inv(Context& c, const RowArgs& a, const MvBatch& bt, hipSt
   const int nrows = c.ny * m.nzp;
   hipLaunchKernelGGL((kx_inv<R1, R2, C, FG, SPL, EARLY>), dim3((nrows + C - 1) / C, (unsigned)bt.nrhs), dim3(R1 * C),
                      0, st, bt.a1, m.twx, a.x, a.y, a.adia, a.aoff, a.compact ? nullptr : c.iocc, sm, c.nx, c.ny, c.nz,
-                     m.nzp, m.p1, c.nat, c.nat0, a.compact, a.cj, 1.f / (float)m.ngrid, bt.k);
+                     m.nzp, m.p1, c.nat, c.nat0, a.compact, a.cj, m.scale, bt.k);
 }
 struct RowShape {
   int L, pass;  // padded length, pass 1 or 5
   void (*fn)(Context&, const RowArgs&, const MvBatch&, hipStream_t);
+  int R1, R2;
 };
 // the shapes of one length and pass: the first is the default, further ones
 // are autotuner candidates
-#define X_FWD(R1, R2, C) RowShape{(R1) * (R2), 1, &launch_kx_fwd<R1, R2, C>}
-#define X_INV(R1, R2, C, FG, SPL, EARLY) RowShape{(R1) * (R2), 5, &launch_kx_inv<R1, R2, C, FG, SPL, EARLY>}
+#define X_FWD(R1, R2, C) RowShape{(R1) * (R2), 1, &launch_kx_fwd<R1, R2, C>, R1, R2}
+#define X_INV(R1, R2, C, FG, SPL, EARLY) RowShape{(R1) * (R2), 5, &launch_kx_inv<R1, R2, C, FG, SPL, EARLY>, R1, R2}
 const RowShape* row_shapes_short(int& n);  // up to 256 points
 const RowShape* row_shapes_long(int& n);   // 270 to 768
 

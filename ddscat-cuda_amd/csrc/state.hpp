@@ -28,6 +28,9 @@ struct MatvecPlan {
   int kind[6] = {-1, -1, -1, -1, -1, -1};
   int zsh = 0;    // log2 of the z run length of the row support (c.ysup)
   int plane = 0;  // passes 2 to 4 by the plane kernel (plane_yz.hpp)
+  // pass 5's factor of the convolution, a float and the rest, for the kernels of scale_key (matvec_scale)
+  float2 scale{0.f, 0.f};
+  int scale_key[6] = {-2, -2, -2, -2, -2, -2};
   int tuned = 0;
 };
 
@@ -164,6 +167,11 @@ size_t matvec_a1_count(const Context& c);
 size_t matvec_a2_count(const Context& c);
 // register-FFT shapes available for pass `which` (1..5) on a padded axis length (0: none)
 int reg_candidates(int L, int which);
+// stages of shape `cand` of pass `which`
+FftPlan reg_stages(int L, int which, int cand);
+// whether the wave kernel of the Green pass, which addresses a component of a2
+// and the Green array with 32-bit byte offsets, reaches the planes sl
+bool reg_green_reach(const Context& c, const KxSlab& sl);
 // whether y-pass shape `cand` of a padded length leaves the rows outside the row support alone
 bool reg_row_support(int L, int cand);
 // register-FFT pass `which` (1..5) with shape `cand` of its axis length; 1 = launched
@@ -179,6 +187,8 @@ int plane_yz_setup(Context& c);
 // whether it runs now: the LDS-staged family can be chosen on a prepared target
 inline bool plane_yz_runs(const Context& c) { return c.mv.plane && !c.fft_generic; }
 int plane_yz_launch(Context& c, hipStream_t st, const MvBatch& bt);
+// its stages along y and z
+void plane_yz_stages(const Context& c, FftPlan& y, FftPlan& z);
 // pass 1 (x -> a1) or 5 (a1 -> y) alone
 int matvec_end_pass(Context& c, int which, int cwhat, const float2* x, float2* y, const float2* adia,
                     const float2* aoff, int layout, hipStream_t st, const MvBatch& bt);
