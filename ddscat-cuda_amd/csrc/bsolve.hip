@@ -836,7 +836,8 @@ struct Ops {
   }
   int upload(int* dev, const std::vector<int>& h) { return flags(dev, h, nullptr); }
   // start of a chunk of iterations of the RHS in act (a pause cleared the
-  // device flags); the stream is idle, so the pinned requests can be cleared here
+  // device flags); no kernel that writes the pinned requests is in flight (those
+  // of the last chunk ended at its synchronisation), so they can be cleared here
   int chunk_start(const std::vector<int>& act) {
     std::fill(S.hictl + S.B, S.hictl + 2 * (size_t)S.B, 0);
     return flags(S.active, act, S.ctl);

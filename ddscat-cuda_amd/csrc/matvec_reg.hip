@@ -247,8 +247,9 @@ struct YShape {
 #define Y_SHAPE(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C>, {R2, R1, 1}}
 #define Y_SPLIT(R1, R2, C) YShape{(R1) * (R2), &launch_y<R1, R2, C, true>, {R2, R1, 1}}
 // One shape per padded length 2N, N = 2^a 3^b 5^c 7^d from 12 to 256 and a few
-// above (two-level, R1 threads per column, at most 25 values each, C columns
-// per workgroup; 512 and 768 points by decimation, 20 and 30 % faster there).
+// above (two-level, R1 threads per column, up to 25 values each to 500 points and
+// 24 to 35 above, C columns per workgroup; 512 and 768 points by decimation, 20
+// and 30 % faster there).
 // The real and imaginary parts cross in turn (Y_SPLIT), with half the LDS and
 // twice the workgroups on a CU for two further barriers, at the lengths where
 // that gained a percent or more of a MATVEC: 192^3 1,249 -> 1,165 us, 200^3

@@ -1,8 +1,10 @@
 // Green-pass plans for padded z axes of 360 to 768 points (pass3_wave.hpp),
 // the fastest of three to eight measured per length on whole MATVECs of cubes
-// (N, N, N): three stages of 8 to 12 values, one column per wave or two, but
-// for 400 points (20 x 20: 1,538 us at 200^3, three stages 1,570 and more) and
-// 768 (16 16 3: 9,785 at 384^3, 16 8 6 9,796, 8 8 12 9,865, 12 8 8 10,760).  360 points 20 18
+// (N, N, N): three stages, mostly of 8 to 12 values (up to 18 where the length
+// splits no better), one column per wave or two; two stages of 18 to 21 values
+// at 400 points (20 x 20: 1,538 us at 200^3, three stages 1,570 and more), 378 and
+// 420; 768 points 16 16 3 (9,785 at 384^3, 16 8 6 9,796, 8 8 12 9,865, 12 8 8 10,760).
+// 360 points 20 18
 // -> 12 5 6: 180^3 1,187 -> 1,053 us; 384 8 6 8 -> 8 8 6: 192^3 1,332 -> 1,249;
 // 432 8 6 9 -> 12 4 9: 216^3 1,996 -> 1,960.
 #include "pass3_wave.hpp"

@@ -13,9 +13,9 @@
 // this one replaced, which walked z with the plane stride and synchronised
 // 256- to 768-thread workgroups at every exchange (bytes: a2 in and out and the
 // octant once):
-//   128^3, 256 points: 148 -> 125 us (4.1 TB/s)
-//   256^3, 512 points: 1,830 -> 1,078 us (3.75 TB/s)
-//   384^3, 768 points: 7,700 -> 4,150 us (3.3 TB/s)
+//   128^3, 256 points: 148 -> 128 us (4.0 TB/s; 136 to 139 in runs of a few MATVECs)
+//   256^3, 512 points: 1,830 -> 1,110 us (3.6 TB/s; 1,090 to 1,330, with the clock)
+//   384^3, 768 points: 7,700 -> 4,110 us (3.3 TB/s; to 4,480)
 #pragma once
 #include "fft_wave.hpp"
 #include "mv_device.hpp"

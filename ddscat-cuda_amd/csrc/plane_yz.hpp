@@ -13,8 +13,8 @@
 //
 // What bounds it: a plane sits on one CU, where VALU issue of the z columns is
 // two thirds of the time (32^3, one right-hand side: 1.3 + 0.9 us the y levels,
-// 4.5 the columns, 1.5 the inverse levels); a small grid has no more planes
-// than a quarter of the CUs, so the time is one plane's.  Against passes 2, 3
+// 4.5 the columns, 1.5 the inverse levels); a small cube has fewer planes than
+// CUs, so the time is one plane's.  Against passes 2, 3
 // and 4 as kernels of their own, whole MATVECs:
 //   16^3 20.7 -> 16.3 us, 32^3 23.0 -> 20.5, 45^3 41 -> 35;
 //   32 right-hand sides: 32^3 129 -> 110 us, 36^3 259 -> 174, 54^3 878 -> 632.

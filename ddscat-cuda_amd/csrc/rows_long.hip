@@ -1,6 +1,6 @@
 // x-pass shapes for padded x axes of 270 to 768 points (rows.hpp).  The
 // components of pass 5 are loaded and transformed one after another (VN of 18
-// to 32 values), real and imaginary parts crossing LDS in turn, in finish
+// to 35 values), real and imaginary parts crossing LDS in turn, in finish
 // groups of two outputs: 3 to 5 % faster than whole exchanges and groups of
 // four at 270 to 480 points.
 #include "rows.hpp"

@@ -146,7 +146,7 @@ struct KxSlab {
 };
 struct MvBatch {
   int nrhs = 1;
-  KxSlab slab;           // H = 0: every plane
+  KxSlab slab;           // the planes passes 2 to 4 run on
   BatchArgs k;
   float2* a1 = nullptr;  // nullptr: the context's single-RHS buffers
   float2* a2 = nullptr;

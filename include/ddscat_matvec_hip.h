@@ -129,21 +129,25 @@ DDSCAT_HIP_API int ddscat_hip_set_precision(int precision);
 enum { DDSCAT_HIP_RELIABLE_REPLACE = 0, DDSCAT_HIP_RELIABLE_RESTART = 1 };
 DDSCAT_HIP_API int ddscat_hip_set_reliable_mode(int mode);
 
-/* FFT kernel family: 0 = register-resident two-level FFTs where the padded
- * axis length allows (64, 128, 256), LDS-staged Stockham otherwise
- * (default); 1 = LDS-staged Stockham for every axis. */
+/* FFT kernel family: 0 = register-resident FFTs where the padded axis length
+ * has a kernel (24 to 512 points with factors 2, 3, 5, 7, and several up to 768;
+ * on small grids one kernel for passes 2 to 4), LDS-staged Stockham otherwise
+ * (default); 1 = LDS-staged Stockham for every axis.  Takes effect with the
+ * next MATVEC, also of a prepared target. */
 DDSCAT_HIP_API int ddscat_hip_set_fft_kernels(int generic);
 
-/* FFT kernel autotuning at prepare (FFT3D backend): 1 (default) times every
- * candidate kernel of each MATVEC pass (register shapes of the pass's axis
- * length and the LDS-staged kernel) and keeps the fastest, cached per grid
- * for the process; 0 uses each length's default register shape. */
+/* FFT kernel autotuning at prepare (both backends): 1 (default) times the
+ * register shapes of each MATVEC pass whose axis length has several and keeps
+ * the fastest, cached per grid for the process; 0 uses each length's default
+ * shape.  A length without a shape takes the LDS-staged kernel. */
 DDSCAT_HIP_API int ddscat_hip_set_autotune(int on);
 
 /* Override the FFT kernel of MATVEC pass 1..5 of the prepared grid: kind -1
  * = LDS-staged, k >= 0 = register candidate k of the pass's axis length
- * (ddscat_hip_info reports the current choice).  For testing and manual
- * tuning; the next prepare re-tunes.  Codes 10 not prepared, 11 no such kernel. */
+ * (ddscat_hip_info reports the current choice).  On a small grid a call for
+ * any of passes 2 to 4 also returns those from their one kernel to separate
+ * ones, until the next prepare.  For testing and manual tuning; the next
+ * prepare re-tunes.  Codes 10 not prepared (FFT3D), 11 no such kernel. */
 DDSCAT_HIP_API int ddscat_hip_set_pass_kernel(int pass, int kind);
 
 /* y = A x on DEVICE pointers, stream-ordered on `stream` (NULL = library
@@ -369,7 +373,8 @@ DDSCAT_HIP_API int ddscat_hip_info(long long *out, int n);
 
 /* Run `reps` MATVECs on device pointers with HIP events between the five
  * FFT3D passes: ms_out[0..4] mean per-pass milliseconds, ms_out[5] mean
- * MATVEC milliseconds (SLICES backend: only ms_out[5]). */
+ * MATVEC milliseconds (SLICES backend: only ms_out[5]).  Where one kernel runs
+ * passes 2 to 4 (ddscat_hip_info), its time is ms_out[2]. */
 DDSCAT_HIP_API int ddscat_hip_time_matvec(int cwhat, const void *x, void *y, const void *adia,
                                           const void *aoff, int layout, int reps, double *ms_out);
 
